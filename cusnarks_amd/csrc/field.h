@@ -16,6 +16,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "inv30.h"
 
 namespace csk {
 
@@ -265,103 +266,19 @@ template <int PIDX> struct Fp {
     return mul(a, one_n);
   }
 
-  // Inverse in the Montgomery domain: (aR)^-1 R.  Binary extended Euclid on
-  // the integer aR (short latency, branchy: meant for the handful of
-  // single-thread inversions that close an MSM), then a product with R^3.
-  // Returns 0 for a == 0.
+  // Inverse in the Montgomery domain: (aR)^-1 R, 0 for a == 0.  The integer
+  // aR is inverted by division steps (inv30.h), then multiplied by R^3:
+  // (aR)^-1 R^3 R^-1 = a^-1 R.
   __device__ static Fp inv(const Fp &a) {
     if (a.is_zero()) return zero();
-    uint32_t u[8], w[8], x1[8], x2[8];
+    Fp p, r, r3;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-      u[i] = a.v[i];
-      w[i] = C::p[i];
-      x1[i] = 0;
-      x2[i] = 0;
-    }
-    x1[0] = 1;
-    // invariant: x1*a == u, x2*a == w (mod p); stop when u == 1 or w == 1
-    for (;;) {
-      bool u1 = (u[0] == 1), w1 = (w[0] == 1);
-      uint32_t hu = 0, hw = 0;
-      for (int i = 1; i < 8; i++) { hu |= u[i]; hw |= w[i]; }
-      if (u1 && hu == 0) break;
-      if (w1 && hw == 0) {
-        for (int i = 0; i < 8; i++) x1[i] = x2[i];
-        break;
-      }
-      while ((u[0] & 1) == 0) {
-        shr1(u);
-        half_mod(x1);
-      }
-      while ((w[0] & 1) == 0) {
-        shr1(w);
-        half_mod(x2);
-      }
-      if (geq(u, w)) {
-        sub_raw(u, w);
-        sub_mod_raw(x1, x2);
-      } else {
-        sub_raw(w, u);
-        sub_mod_raw(x2, x1);
-      }
-    }
-    Fp r, r3;
-    for (int i = 0; i < 8; i++) {
-      r.v[i] = x1[i];
+      p.v[i] = C::p[i];
       r3.v[i] = C::r3[i];
     }
-    return mul(r, r3);  // (aR)^-1 * R^3 * R^-1 = a^-1 R
-  }
-
- private:
-  __device__ __forceinline__ static void shr1(uint32_t *x) {
-    for (int i = 0; i < 7; i++) x[i] = (x[i] >> 1) | (x[i + 1] << 31);
-    x[7] >>= 1;
-  }
-  // x/2 mod p for x < p
-  __device__ __forceinline__ static void half_mod(uint32_t *x) {
-    if (x[0] & 1) {
-      uint32_t carry = 0;
-      for (int i = 0; i < 8; i++) {
-        uint64_t t = (uint64_t)x[i] + C::p[i] + carry;
-        x[i] = (uint32_t)t;
-        carry = (uint32_t)(t >> 32);
-      }
-      // x + p < 2^255: no ninth bit
-    }
-    shr1(x);
-  }
-  __device__ __forceinline__ static bool geq(const uint32_t *a, const uint32_t *b) {
-    for (int i = 7; i >= 0; i--) {
-      if (a[i] != b[i]) return a[i] > b[i];
-    }
-    return true;
-  }
-  __device__ __forceinline__ static void sub_raw(uint32_t *a, const uint32_t *b) {
-    uint32_t borrow = 0;
-    for (int i = 0; i < 8; i++) {
-      uint64_t t = (uint64_t)a[i] - b[i] - borrow;
-      a[i] = (uint32_t)t;
-      borrow = (uint32_t)(t >> 63);
-    }
-  }
-  // a = a - b mod p (a, b < p)
-  __device__ __forceinline__ static void sub_mod_raw(uint32_t *a, const uint32_t *b) {
-    uint32_t borrow = 0;
-    for (int i = 0; i < 8; i++) {
-      uint64_t t = (uint64_t)a[i] - b[i] - borrow;
-      a[i] = (uint32_t)t;
-      borrow = (uint32_t)(t >> 63);
-    }
-    if (borrow) {
-      uint32_t carry = 0;
-      for (int i = 0; i < 8; i++) {
-        uint64_t t = (uint64_t)a[i] + C::p[i] + carry;
-        a[i] = (uint32_t)t;
-        carry = (uint32_t)(t >> 32);
-      }
-    }
+    i30_inverse(a.v, p.v, C::np, r.v);
+    return mul(r, r3);
   }
 };
 

@@ -895,95 +895,110 @@ void window_sums(const uint32_t *partial, uint32_t nwin, uint32_t S, uint32_t *t
   }
 }
 
-// One wave per member: Horner over its W window sums (c doublings each),
+// One workgroup per member: Horner over its W window sums (c doublings each),
 // written as a canonical affine point to the member's output.  The chain is
-// serial, so the wave evaluates each formula cooperatively: the independent
-// products of a step run on different lanes at once (coop29.h).  G1 keeps the
-// point in every lane's registers as 29-bit limbs and exchanges the products
-// through LDS; G2 keeps every value in 29-bit LDS slots, which holds its
-// register count down.  Infinity is tracked in a flag every lane holds.
+// serial and latency bound, so each product is spread over a row of lanes and
+// the products of a step run on different rows (row29.h): G1 in one wave that
+// holds the point in registers, G2 in four waves that hold every value in LDS
+// (coop29.h).  Infinity is tracked in a flag every lane holds.
+// Measured at 248 doublings and 31 additions (c = 8): G1 333 us, 855 with one
+// lane per product; G2 638 us, 1997 with one lane per product.  One window
+// (table runs: the inversion and the conversions): 50 us, 167 with a binary
+// Euclid.
+template <class F> struct FinalThreads { static constexpr int N = std::is_same<F, Fq>::value ? 64 : 256; };
+
 template <class F>
-__global__ void __launch_bounds__(64) k_final(const MsmSeg *__restrict__ segs, const uint32_t *__restrict__ wsum,
-                                              uint32_t W, uint32_t c) {
+__global__ void __launch_bounds__(FinalThreads<F>::N) k_final(const MsmSeg *__restrict__ segs,
+                                                              const uint32_t *__restrict__ wsum, uint32_t W,
+                                                              uint32_t c) {
   const uint32_t j = blockIdx.x;
   uint32_t *out = segs[j].out;
   if (segs[j].n == 0) {
     if (threadIdx.x == 0) store_affine(out, Affine<F>{F::zero(), F::one()});
     return;
   }
+  constexpr int SW = Slot29<F>::SW;
+  const uint32_t *ws = wsum + (uint64_t)j * W * SW;
   if constexpr (std::is_same<F, Fq>::value) {
-    constexpr int SW = Slot29<F>::SW;
-    __shared__ Fq29 sh[6];
-    const uint32_t *ws = wsum + (uint64_t)j * W * SW;
-    XYZZ29 acc;
-    load29(ws + (uint64_t)(W - 1) * SW, acc);
-    bool inf = is_zero29(acc.ZZ);
+    const RowG1K k;
+    RowG1 acc = row_load_g1(ws + (uint64_t)(W - 1) * SW);
+    bool inf = row_is_zero(acc.ZZ);
+#pragma unroll 1
     for (int w = (int)W - 2; w >= 0; w--) {
+      const RowG1 q = row_load_g1(ws + (uint64_t)w * SW);
       if (!inf)
-        for (uint32_t i = 0; i < c; i++) xdbl29_coop(sh, acc);
-      XYZZ29 q;
-      load29(ws + (uint64_t)w * SW, q);
-      if (is_zero29(q.ZZ)) continue;
+#pragma unroll 1
+        for (uint32_t i = 0; i < c; i++) row_dbl(k, acc);
+      if (row_is_zero(q.ZZ)) continue;
       if (inf) {
         acc = q;
         inf = false;
         continue;
       }
-      xadd29_coop(sh, acc, q, inf);
+      row_add(k, acc, q, inf);
     }
+    const Fq29 X = row_gather(acc.X), Y = row_gather(acc.Y), ZZ = row_gather(acc.ZZ), ZZZ = row_gather(acc.ZZZ);
     if (threadIdx.x == 0) {
       XYZZ<F> a;
-      from29_words(acc.X, a.X.v);
-      from29_words(acc.Y, a.Y.v);
-      from29_words(acc.ZZ, a.ZZ.v);
-      from29_words(acc.ZZZ, a.ZZZ.v);
+      from29_words(X, a.X.v);
+      from29_words(Y, a.Y.v);
+      from29_words(ZZ, a.ZZ.v);
+      from29_words(ZZZ, a.ZZZ.v);
       if (inf) a = XYZZ<F>::inf();
       store_affine(out, xyzz_to_affine(a));
     }
   } else {
     using C = Coop29<F>;
-    constexpr int NC = C::NC, SW = NC * 9;
-    __shared__ uint32_t sh[C::kSlots * 9];
-    __shared__ C29Op prog[C::kOps];
-    C::load(prog);
-    const uint32_t *ws = wsum + (uint64_t)j * W * SW;
-    // acc = window W-1; the zero slot follows the addend
-    for (uint32_t i = threadIdx.x; i < (uint32_t)SW; i += blockDim.x) {
-      sh[i] = ws[(uint64_t)(W - 1) * SW + i];
-      sh[2 * SW + i % 9] = 0;
-    }
+    constexpr int NC = C::NC;
+    __shared__ uint32_t sh[C::kSlots * 16];
+    C prog(sh);
+    // slot word of element word i of a window sum
+    auto slot = [](uint32_t i) { return 16 * (i / 9) + i % 9; };
+    for (uint32_t i = threadIdx.x; i < (uint32_t)SW; i += blockDim.x) sh[slot(i)] = ws[(uint64_t)(W - 1) * SW + i];
     __syncthreads();
-    bool inf = c29_is_zero(sh, C::ZZ);
+    bool inf = prog.is_zero(C::ZZ);
+#pragma unroll 1
     for (int w = (int)W - 2; w >= 0; w--) {
       if (!inf)
-        for (uint32_t i = 0; i < c; i++) C::dbl(sh, prog);
-      for (uint32_t i = threadIdx.x; i < (uint32_t)SW; i += blockDim.x) sh[SW + i] = ws[(uint64_t)w * SW + i];
+#pragma unroll 1
+        for (uint32_t i = 0; i < c; i++) prog.dbl();
+      for (uint32_t i = threadIdx.x; i < (uint32_t)SW; i += blockDim.x)
+        sh[16 * NC + slot(i)] = ws[(uint64_t)w * SW + i];
       __syncthreads();
-      if (c29_is_zero(sh, C::QZZ)) continue;
+      if (prog.is_zero(C::QZZ)) {
+        __syncthreads();  // every wave has read the addend before the next one is loaded
+        continue;
+      }
       if (inf) {
-        for (uint32_t i = threadIdx.x; i < (uint32_t)SW; i += blockDim.x) sh[i] = sh[SW + i];
+        for (uint32_t i = threadIdx.x; i < 16 * NC; i += blockDim.x) sh[i] = sh[16 * NC + i];
         __syncthreads();
         inf = false;
         continue;
       }
-      C::add1(sh, prog);
-      if (c29_is_zero(sh, C::PP)) {
-        if (c29_is_zero(sh, C::RR)) C::dbl(sh, prog);  // acc == q
-        else inf = true;                                // acc == -q
+      prog.add1();
+      if (prog.is_zero(C::PP)) {
+        const bool same = prog.is_zero(C::RR);
+        __syncthreads();  // every wave has read PP and RR
+        if (same) prog.dbl();  // acc == q
+        else inf = true;       // acc == -q
         continue;
       }
-      C::add2(sh, prog);
+      prog.add2();
     }
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 64) {
       uint32_t wds[4 * FieldIO<F>::NW];
+#pragma unroll
       for (int k = 0; k < NC; k++) {
         uint32_t o[8];
-        from29_words(c29_ld(sh, k), o);
+        from29_words(row_gather(sh[16 * k + (threadIdx.x & 15)]), o);
+#pragma unroll
         for (int i = 0; i < 8; i++) wds[8 * k + i] = o[i];
       }
-      XYZZ<F> acc = load_xyzz<F>(wds);
-      if (inf) acc = XYZZ<F>::inf();
-      store_affine(out, xyzz_to_affine(acc));
+      if (threadIdx.x == 0) {
+        XYZZ<F> acc = load_xyzz<F>(wds);
+        if (inf) acc = XYZZ<F>::inf();
+        store_affine(out, xyzz_to_affine(acc));
+      }
     }
   }
 }
@@ -1079,7 +1094,7 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
     window_sums<F>(partial, Wtot, pl.S, b29, wsum, st);  // the bucket slots are free again
     CSK_CHECK_LAUNCH();
   }
-  k_final<F><<<pl.J, 64, 0, st>>>(segs, wsum, pl.W, pl.c);
+  k_final<F><<<pl.J, FinalThreads<F>::N, 0, st>>>(segs, wsum, pl.W, pl.c);
   CSK_CHECK_LAUNCH();
   if (tm) tm->mark(3, st);
   return CSK_OK;
@@ -1325,7 +1340,7 @@ int msm_run_table(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArg
   CSK_CHECK_LAUNCH();
   k_bucket_reduce<F><<<(count * Sm + TB - 1) / TB, TB, 0, st>>>(iota, merged, count, pl.B, Lrm, partial);
   window_sums<F>(partial, count, Sm, merged, wsum, st);  // the merged buckets are free again
-  k_final<F><<<count, 64, 0, st>>>(osegs, wsum, 1, pl.c);
+  k_final<F><<<count, FinalThreads<F>::N, 0, st>>>(osegs, wsum, 1, pl.c);
   CSK_CHECK_LAUNCH();
   return CSK_OK;
 }

@@ -1,0 +1,44 @@
+"""Headers of device code that hold plain integer arithmetic, compiled for the
+host and compared with Python integers."""
+import ctypes
+import os
+import random
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "cusnarks_amd", "csrc")
+Q = 21888242871839275222246405745257275088696311157297823662689037894645226208583
+R = 21888242871839275222246405745257275088548364400416034343698204186575808495617
+W8 = ctypes.c_uint32 * 8
+
+
+def words(v):
+    return W8(*[(v >> (32 * i)) & 0xFFFFFFFF for i in range(8)])
+
+
+def value(w):
+    return sum(int(x) << (32 * i) for i, x in enumerate(w))
+
+
+def compiled(tmp_path, header, body):
+    src = tmp_path / "h.cpp"
+    src.write_text('#define __device__\n#define __constant__\n#define __forceinline__ inline\n#include <stdint.h>\n'
+                   '#include "%s"\nextern "C" %s\n' % (os.path.join(CSRC, header), body))
+    so = str(tmp_path / "h.so")
+    subprocess.run(["g++", "-O2", "-shared", "-fPIC", "-o", so, str(src)], check=True)
+    return ctypes.CDLL(so)
+
+
+@pytest.mark.parametrize("p", [Q, R])
+def test_division_step_inverse(tmp_path, p):
+    L = compiled(tmp_path, "inv30.h", "void inv(const uint32_t *a, const uint32_t *p, uint32_t np, uint32_t *o) "
+                                      "{ csk::i30_inverse(a, p, np, o); }")
+    rng = random.Random(5)
+    np_ = -pow(p, -1, 1 << 32) % (1 << 32)
+    xs = [1, 2, 3, p - 1, p - 2, (p + 1) // 2, p // 2, 1 << 253, p + 5, 2**256 - 1]
+    xs += [rng.randrange(1, p) for _ in range(3000)] + [rng.randrange(1, 1 << rng.randrange(1, 254)) for _ in range(500)]
+    for x in xs:
+        o = W8()
+        L.inv(words(x), words(p), np_, o)
+        assert value(o) < p and value(o) * x % p == 1, hex(x)

@@ -1,0 +1,51 @@
+"""The window combination's exceptional additions: a window sum equal to the
+running sum (a doubling) or to its negative (infinity, with windows still to
+come), windows that sum to infinity, and a chain that starts at infinity."""
+import numpy as np
+import pytest
+
+import oracle as O
+from cusnarks_amd import inputs
+from cusnarks_amd.msm import msm_host
+from oracle import pyoracle as P
+from tests.gpu_util import gen_mul
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(c, g2, base, plus):
+    """Scalars and multiples of the generator: base 2^c under 1, and base
+    under 2^c as the second window's only entry, so the running sum meets the
+    first window's sum base 2^c (plus) or its negative."""
+    k = [1, 1 << c]
+    s = [base << c if plus else -base << c, base]
+    return k, s
+
+
+@pytest.mark.parametrize("g2", [False, True])
+@pytest.mark.parametrize("c", [3, 8])
+@pytest.mark.parametrize("plus", [True, False])
+def test_equal_and_opposite_window_sums(g2, c, plus):
+    k, s = _case(c, g2, 5, plus)
+    # the same one window pair higher, with more windows below it
+    k2 = [x << (2 * c) for x in k] + [1, 3]
+    s2 = s + [7, 11]
+    for ks, ss in ((k, s), (k2, s2)):
+        pts = np.stack([gen_mul(x, g2) for x in ss])
+        want = gen_mul(sum(a * b for a, b in zip(ks, ss)), g2)
+        got = msm_host(inputs.from_ints(ks), pts, g2=g2, window_bits=c)
+        if sum(a * b for a, b in zip(ks, ss)) % P.RR == 0:
+            want = np.array(P.g2_to_words(None) if g2 else P.g1_to_words(None), np.uint32)
+        assert np.array_equal(got, want)
+        exp, _ = O.ec_jacreduce(inputs.from_ints(ks), pts, ec2=g2)
+        assert np.array_equal(got, exp)
+
+
+@pytest.mark.parametrize("g2", [False, True])
+def test_sparse_windows(g2):
+    # one entry each in a few far-apart windows: the windows between are infinity
+    ks = [1 << 250, (1 << 131) + 1, 1 << 64]
+    ss = [3, 1 << 40, P.RR - 9]
+    pts = np.stack([gen_mul(x, g2) for x in ss])
+    got = msm_host(inputs.from_ints(ks), pts, g2=g2, window_bits=7)
+    assert np.array_equal(got, gen_mul(sum(a * b for a, b in zip(ks, ss)) % P.RR, g2))
