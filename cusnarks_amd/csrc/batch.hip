@@ -195,11 +195,12 @@ int plan_batch(csk_msm_batch *b, const uint64_t *n, const uint32_t *window_bits)
   for (auto &g : b->groups) {
     std::vector<uint64_t> gn;
     for (uint32_t i : g.members) gn.push_back(n[i]);
-    g.pl = msm_group_plan(cw[g.members[0]], gn.data(), (uint32_t)gn.size(), g2, 0, 0);
+    g.pl = msm_group_plan(cw[g.members[0]], 1, gn.data(), (uint32_t)gn.size(), g2, 0, 0);
     if (!msm_plan_ok(g.pl)) {
       set_error("msm_batch: unsupported group plan");
       return CSK_ERR_ARG;
     }
+    g.pl = msm_split_plan(g.pl, gn.data(), g2, 0, 0);
   }
   // largest groups first, dealt round-robin over the streams
   std::stable_sort(b->groups.begin(), b->groups.end(),

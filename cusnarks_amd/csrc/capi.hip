@@ -330,7 +330,7 @@ int csk_last_stage_times(csk_ctx *ctx, float *ms, int n) {
 int csk_last_msm_plan(csk_ctx *ctx, uint32_t *out, int n) {
   if (!ctx || !out) return CSK_ERR_ARG;
   const csk::MsmPlan &p = ctx->last_plan;
-  uint64_t v[8] = {p.c, p.W, p.B, p.L, p.Lr, p.S, p.n, p.max_entries};
+  uint64_t v[8] = {p.c, p.W, p.B, p.L, p.Lr, p.S, p.n / (p.E ? p.E : 1), p.max_entries};
   for (int i = 0; i < n && i < 8; i++) out[i] = (uint32_t)v[i];
   return CSK_OK;
 }

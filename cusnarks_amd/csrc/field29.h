@@ -16,7 +16,7 @@
 // G1 loop keeps X < 8q, Y, ZZ, ZZZ < 2q (see madd29).
 //
 // Conversion.  Points enter as the library's 8 x u32 words in Montgomery
-// form for R = 2^256; to29 multiplies by 2^266 mod q (x 2^256 x 2^266 /
+// form for R = 2^256; a product by 2^266 mod q (x 2^256 x 2^266 /
 // 2^261 = x 2^261), stored packed back into 8 words (values are < q).
 // from29 multiplies by 2^256 mod q, which returns to R = 2^256 form.
 #pragma once
@@ -316,11 +316,6 @@ __device__ __forceinline__ void pack29(const Fq29 &a, uint32_t (&w)[8]) {
     }
     w[k] = x;
   }
-}
-
-// R = 2^256 Montgomery words (< q) -> 2^261 form, canonical, packed
-__device__ __forceinline__ void to29_words(const uint32_t (&in)[8], uint32_t (&out)[8]) {
-  pack29(canon29(mul29(unpack29(in), f29_const(Q29::to))), out);
 }
 
 // 2^261 form (value below 8q) -> canonical R = 2^256 words

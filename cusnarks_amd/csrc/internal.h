@@ -59,7 +59,9 @@ struct Carver {
 // [j*K, (j+1)*K); every stage runs once over the whole group.
 struct MsmPlan {
   uint32_t c;            // window bits
-  uint32_t W;            // windows: floor(254 / c) + 1 signed-digit windows cover k < r < 2^254
+  uint32_t E;            // scalars' parts: 2 with the scalars split along the endomorphism (glv.h), else 1
+  uint32_t bits;         // size of a part in bits: 126 or 254
+  uint32_t W;            // windows: floor(bits / c) + 1 signed-digit windows cover a part
   uint32_t B;            // buckets per window, 2^(c-1) (signed digits)
   uint32_t K;            // W * B bucket keys per member
   uint32_t J;            // members
@@ -68,7 +70,7 @@ struct MsmPlan {
   uint32_t L;            // sorted entries per accumulation thread
   uint32_t Lr;           // buckets per reduction thread
   uint32_t S;            // reduction segments per window, B / Lr
-  uint64_t n;            // points over all members
+  uint64_t n;            // points over all members, E for each of the caller's
   uint64_t max_entries;  // n * W (upper bound on nonzero digits)
   uint64_t max_chunks;   // ceil(max_entries / L)
   uint64_t tiles;        // sum over members of ceil(n_j / 4096) (sort tiles per window)

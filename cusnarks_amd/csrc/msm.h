@@ -8,10 +8,10 @@ namespace csk {
 // One multiexp inside a group (device-resident table of J+1 entries; entry J
 // is a sentinel holding the totals).  All members of a group share c.
 struct MsmSeg {
-  const uint32_t *scalars;  // n x 8 u32, normal form
-  const uint32_t *points;   // n affine points, Montgomery form
+  const uint32_t *scalars;  // n / E x 8 u32, normal form
+  const uint32_t *points;   // n / E affine points, Montgomery form
   uint32_t *out;            // one affine point
-  uint64_t n;               // points of this member
+  uint64_t n;               // points of this member (the plan's E for each of the caller's)
   uint64_t pbase;           // points of the members before it
   uint32_t NT;              // sort tiles per window, ceil(n / 4096)
   uint32_t cbase;           // first pass-1 counter of the member
@@ -40,8 +40,13 @@ inline uint64_t msm_sortbuf_bytes(const MsmPlan &pl, bool g2) {
 }
 
 uint32_t msm_choose_c(uint64_t n, bool g2, const csk_ctx *ctx, const csk_msm_cfg *cfg);
-// group plan for members of sizes n[0..J) sharing window width c
-MsmPlan msm_group_plan(uint32_t c, const uint64_t *n, uint32_t J, bool g2, uint32_t chunk, uint32_t reduce_seg);
+// group plan for members of sizes n[0..J) sharing window width c, the scalars
+// taken whole or split (E = 1 or 2)
+MsmPlan msm_group_plan(uint32_t c, uint32_t E, const uint64_t *n, uint32_t J, bool g2, uint32_t chunk,
+                       uint32_t reduce_seg);
+// the plan a group runs by: split scalars, or whole ones where only their
+// entries fit the index range; whole is the plan with E = 1
+MsmPlan msm_split_plan(const MsmPlan &whole, const uint64_t *n, bool g2, uint32_t chunk, uint32_t reduce_seg);
 bool msm_plan_ok(const MsmPlan &pl);
 size_t msm_workspace_bytes(const MsmPlan &pl, bool g2);
 // fill the host copy of a group's descriptor table (J+1 entries)

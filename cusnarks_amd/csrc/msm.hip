@@ -7,7 +7,8 @@
 // so it is bit-identical to the reference's ec_jac2aff_h of its result.
 //
 // Pipeline (all on one stream, no host round trip):
-//   1. k_digits      one thread per point: k mod r, signed c-bit digits for
+//   1. k_digits      one thread per point: k mod r, split in two halves along
+//                    the endomorphism (glv.h), signed c-bit digits of each for
 //                    W windows; (window, |digit|) -> bucket key; histogram.
 //   2. scan          exclusive prefix sum of the histogram -> bucket offsets.
 //   3. k_scatter     counting-sort placement of (point index | sign) by key.
@@ -21,6 +22,7 @@
 #include <vector>
 #include "internal.h"
 #include "field.h"
+#include "glv.h"
 #include "msm.h"
 
 namespace csk {
@@ -38,15 +40,14 @@ uint32_t msm_choose_c(uint64_t n, bool g2, const csk_ctx *ctx, const csk_msm_cfg
   if (cfg && cfg->window_bits) return cfg->window_bits;
   const uint32_t lg = floor_log2(n);
   if (ctx && lg < 64 && ctx->tune[g2][lg].window_bits) return ctx->tune[g2][lg].window_bits;
-  // windows whose top window keeps most of its bits (254 = (W-1) c + t with
-  // t close to c): a narrow top window puts every point in a few buckets
+  // windows whose top window keeps most of its bits (126 = (W-1) c + t with t
+  // close to c): a narrow top window puts every point in a few buckets
   uint32_t c;
-  if (lg <= 9) c = 8;
-  else if (lg <= 13) c = 10;
-  else if (lg <= 17) c = 13;
-  else if (lg <= 19) c = 15;
-  else c = 16;
-  if (g2 && c > 15) c = 15;
+  if (lg <= 11) c = 8;
+  else if (lg <= 14) c = 13;
+  else if (lg <= 22) c = 16;
+  else c = 19;
+  if (g2 && c > 16) c = 16;
   return c;
 }
 
@@ -65,33 +66,36 @@ static uint32_t plan_hi_bits(uint32_t c, uint64_t n_avg) {
 }
 
 // Low bucket bits the second pass sorts the top window by.  That window
-// holds only the scalar's top t = 254 mod c bits (scalars are reduced below
-// r < 2^254, and its digit, at most 2^t <= 2^(c-1), is never negated), so its
-// buckets are below 2^t: its first pass bins by the top hb of those t bits
+// holds only the top t = bits mod c bits of a scalar or of its half (below
+// 2^bits, bits = 254 or 126), and its digit, at most 2^t <= 2^(c-1), has no
+// carry out, so its buckets are below 2^t: its first pass bins by the top hb of those t bits
 // (all HB bins filled, as for the other windows) or, when t <= hb, by all of
 // them, and each of its first-pass bins is then a single bucket.  Binning it
 // like the others instead leaves most of its entries in a few bins, which the
 // second pass takes one workgroup each for (c = 18 at 2^24 points: 22 ms).
-static uint32_t plan_top_bits(uint32_t c, uint32_t hb) {
-  const uint32_t t = 254 % c;
+static uint32_t plan_top_bits(uint32_t bits, uint32_t c, uint32_t hb) {
+  const uint32_t t = bits % c;
   return t > hb ? t - hb : 0;
 }
 
-MsmPlan msm_group_plan(uint32_t c, const uint64_t *n, uint32_t J, bool g2, uint32_t chunk, uint32_t reduce_seg) {
+MsmPlan msm_group_plan(uint32_t c, uint32_t E, const uint64_t *n, uint32_t J, bool g2, uint32_t chunk,
+                       uint32_t reduce_seg) {
   (void)g2;
   MsmPlan pl = {};
   pl.c = c;
-  pl.W = 254 / c + 1;
+  pl.E = E;
+  pl.bits = E == 2 ? kGlvBits : kScalarBits;
+  pl.W = pl.bits / c + 1;
   pl.B = 1u << (c - 1);
   pl.K = pl.W * pl.B;
   pl.J = J;
   for (uint32_t j = 0; j < J; j++) {
-    pl.n += n[j];
-    pl.tiles += (n[j] + kSortTile - 1) / kSortTile;
+    pl.n += E * n[j];
+    pl.tiles += (E * n[j] + kSortTile - 1) / kSortTile;
   }
   pl.max_entries = pl.n * pl.W;
   pl.hb = plan_hi_bits(c, J ? pl.n / J : 0);
-  pl.st = plan_top_bits(c, pl.hb);
+  pl.st = plan_top_bits(pl.bits, c, pl.hb);
   // chunk length: aim for ~2^18 accumulation threads (a few waves per SIMD)
   // so small inputs are not latency bound; at most 256 entries per thread
   uint64_t l = pl.max_entries >> 18;
@@ -109,6 +113,11 @@ MsmPlan msm_group_plan(uint32_t c, const uint64_t *n, uint32_t J, bool g2, uint3
   pl.S = pl.B / pl.Lr;
   pl.max_chunks = (pl.max_entries + pl.L - 1) / pl.L;
   return pl;
+}
+
+MsmPlan msm_split_plan(const MsmPlan &whole, const uint64_t *n, bool g2, uint32_t chunk, uint32_t reduce_seg) {
+  const MsmPlan pl = msm_group_plan(whole.c, 2, n, whole.J, g2, chunk, reduce_seg);
+  return msm_plan_ok(pl) ? pl : whole;
 }
 
 bool msm_plan_ok(const MsmPlan &pl) {
@@ -158,10 +167,10 @@ void msm_fill_segs(const MsmPlan &pl, const uint64_t *n, const uint32_t *const *
     g.scalars = scalars[j];
     g.points = points[j];
     g.out = out[j];
-    g.n = n[j];
-    g.NT = (uint32_t)((n[j] + kSortTile - 1) / kSortTile);
+    g.n = pl.E * n[j];
+    g.NT = (uint32_t)((g.n + kSortTile - 1) / kSortTile);
     g.qbase = (uint32_t)pbase;
-    pbase += n[j];
+    pbase += g.n;
     tiles += g.NT;
   }
 }
@@ -198,11 +207,12 @@ int msm_launch(csk_ctx *ctx, bool g2, const uint32_t *d_scalars, const uint32_t 
   const csk_msm_cfg *tn = lg < 64 ? &ctx->tune[g2][lg] : nullptr;
   const uint32_t chunk = cfg && cfg->chunk ? cfg->chunk : (tn && !(cfg && cfg->window_bits) ? tn->chunk : 0);
   const uint32_t rseg = cfg && cfg->reduce_seg ? cfg->reduce_seg : (tn && !(cfg && cfg->window_bits) ? tn->reduce_seg : 0);
-  MsmPlan pl = msm_group_plan(c, &n, 1, g2, chunk, rseg);
+  MsmPlan pl = msm_group_plan(c, 1, &n, 1, g2, chunk, rseg);
   if (!msm_plan_ok(pl)) {
     set_error("msm: unsupported configuration (window/chunk/segment or size too large)");
     return CSK_ERR_ARG;
   }
+  pl = msm_split_plan(pl, &n, g2, chunk, rseg);
   const size_t seg_bytes = Carver::round(2 * sizeof(MsmSeg));
   int rc = ctx->ws.ensure(seg_bytes + msm_workspace_bytes(pl, g2));
   if (rc) return rc;
@@ -298,10 +308,10 @@ extern "C" int csk_msm_g1_noalloc(csk_ctx *ctx, const uint32_t *d_scalars, const
   const uint32_t chunk = cfg && cfg->chunk ? cfg->chunk : (!fixed_c ? tn->chunk : 0);
   const uint32_t rseg = cfg && cfg->reduce_seg ? cfg->reduce_seg : (!fixed_c ? tn->reduce_seg : 0);
   const size_t seg_bytes = Carver::round(2 * sizeof(MsmSeg));
-  MsmPlan pl = msm_group_plan(c, &n, 1, false, chunk, rseg);
+  MsmPlan pl = msm_group_plan(c, 1, &n, 1, false, chunk, rseg);
   while (!fixed_c && c > 2 && (!msm_plan_ok(pl) || seg_bytes + msm_workspace_bytes(pl, false) > kNoAllocBytes)) {
     c--;
-    pl = msm_group_plan(c, &n, 1, false, chunk, rseg);
+    pl = msm_group_plan(c, 1, &n, 1, false, chunk, rseg);
   }
   if (!msm_plan_ok(pl)) {
     set_error("msm_g1_noalloc: unsupported configuration (window/chunk/segment)");
@@ -313,6 +323,10 @@ extern "C" int csk_msm_g1_noalloc(csk_ctx *ctx, const uint32_t *d_scalars, const
               std::to_string(kNoAllocBytes) + "-byte scratch array");
     return CSK_ERR_ARG;
   }
+  // which widths are taken is settled by the whole scalars' workspace; the
+  // split ones run where theirs fits too
+  const MsmPlan split = msm_split_plan(pl, &n, false, chunk, rseg);
+  if (seg_bytes + msm_workspace_bytes(split, false) <= kNoAllocBytes) pl = split;
   ctx->last_plan = pl;
   MsmSeg segs[2];
   msm_fill_segs(pl, &n, &d_scalars, &d_points, &d_out, segs);
@@ -343,6 +357,8 @@ namespace csk {
 static MsmPlan table_plan(uint32_t c, uint64_t n_pad, uint32_t Wt, uint32_t count) {
   MsmPlan pl = {};
   pl.c = c;
+  pl.E = 1;
+  pl.bits = kScalarBits;
   pl.W = 1;
   pl.B = 1u << (c - 1);
   pl.K = pl.B;
@@ -351,7 +367,7 @@ static MsmPlan table_plan(uint32_t c, uint64_t n_pad, uint32_t Wt, uint32_t coun
   pl.tiles = pl.J * (n_pad / kSortTile);
   pl.max_entries = pl.n;
   pl.hb = plan_hi_bits(c, n_pad);
-  pl.st = plan_top_bits(c, pl.hb);
+  pl.st = plan_top_bits(pl.bits, c, pl.hb);
   uint64_t l = pl.max_entries >> 18;
   if (l < 8) l = 8;
   if (l > 256) l = 256;
@@ -410,7 +426,7 @@ static int table_run(csk_ctx *ctx, uint32_t count, csk_msm_table *const *t, cons
   }
   pl.max_entries = pl.n;
   pl.hb = plan_hi_bits(c, pl.n / pl.J);
-  pl.st = plan_top_bits(c, pl.hb);
+  pl.st = plan_top_bits(pl.bits, c, pl.hb);
   uint64_t l = pl.max_entries >> 18;
   pl.L = (uint32_t)(l < 8 ? 8 : l > 256 ? 256 : l);
   pl.max_chunks = (pl.max_entries + pl.L - 1) / pl.L;

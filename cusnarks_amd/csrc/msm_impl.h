@@ -7,6 +7,7 @@
 #include "curve.h"
 #include "field29.h"
 #include "coop29.h"
+#include "glv.h"
 #include "msm.h"
 
 namespace csk {
@@ -62,42 +63,100 @@ __device__ __forceinline__ uint32_t member_of_tile(const MsmSeg *segs, uint32_t 
   return lo;
 }
 
-// the point in the 2^261 form (field29.h), packed words, component by component
-__device__ __forceinline__ void store_point29(uint32_t *d, const Affine<Fq> &p) {
-  uint32_t o[8];
-  to29_words(p.x.v, o);
-  st8(d, o);
-  to29_words(p.y.v, o);
-  st8(d + 8, o);
+// beta of phi(x, y) = (beta x, y) in the 2^261 form: on G2 the other cube root
+// of unity, so that phi is the multiplication by the same lambda
+template <class F> struct Beta29;
+template <> struct Beta29<Fq> {
+  static constexpr uint32_t v[9] = {171145621u, 361569571u, 412916632u, 318393925u, 408922844u,
+                                    24572269u,  250450874u, 338235712u, 789246u};
+};
+template <> struct Beta29<Fq2> {
+  static constexpr uint32_t v[9] = {416069521u, 391846970u, 193189602u, 244240497u, 310558434u,
+                                    69340804u,  535036287u, 352865610u, 1478937u};
+};
+
+// the point in the 2^261 form (field29.h), packed words, component by
+// component; with E = 2 followed by phi of it
+template <class F, int E> __device__ __forceinline__ void store_point29(uint32_t *d, const uint32_t *comps) {
+  constexpr int NC = FieldIO<F>::NW / 8, PW = 2 * FieldIO<F>::NW;  // components per coordinate, words per point
+#pragma unroll
+  for (int k = 0; k < 2 * NC; k++) {
+    uint32_t in[8], o[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) in[i] = comps[8 * k + i];
+    const Fq29 v = mul29(unpack29(in), f29_const(Q29::to));
+    pack29(canon29(v), o);
+    st8(d + 8 * k, o);
+    if (E == 2) {
+      if (k < NC) pack29(canon29(mul29(v, f29_const(Beta29<F>::v))), o);
+      st8(d + PW + 8 * k, o);
+    }
+  }
 }
-__device__ __forceinline__ void store_point29(uint32_t *d, const Affine<Fq2> &p) {
-  uint32_t o[8];
-  to29_words(p.x.c0.v, o);
-  st8(d, o);
-  to29_words(p.x.c1.v, o);
-  st8(d + 8, o);
-  to29_words(p.y.c0.v, o);
-  st8(d + 16, o);
-  to29_words(p.y.c1.v, o);
-  st8(d + 24, o);
+template <int E> __device__ __forceinline__ void store_point29(uint32_t *d, const Affine<Fq> &p) {
+  uint32_t w[16];
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    w[i] = p.x.v[i];
+    w[8 + i] = p.y.v[i];
+  }
+  store_point29<Fq, E>(d, w);
+}
+template <int E> __device__ __forceinline__ void store_point29(uint32_t *d, const Affine<Fq2> &p) {
+  uint32_t w[32];
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    w[i] = p.x.c0.v[i];
+    w[8 + i] = p.x.c1.v[i];
+    w[16 + i] = p.y.c0.v[i];
+    w[24 + i] = p.y.c1.v[i];
+  }
+  store_point29<Fq2, E>(d, w);
 }
 
 // ------------------------------------------------------------------ digits
-// One workgroup per (member j, tile) of kSortTile points; block b covers the
-// tiles in member order (member j's tiles start at b = tbase_j / W).  Each
-// thread takes every 256th point of the tile and writes its signed digits:
-// member j's digits occupy D[W*pbase_j + w*n_j + i], b | neg << 31 for the
-// nonzero signed digit d of window w (b = |d| - 1 < B), or 0xFFFFFFFF when
-// d == 0 or P_i is at infinity.  The workgroup also counts its digits per
-// (window, hi = b >> s) in LDS and writes the counts as pass 1 of the sort
-// expects them: cnt[cbase_j + (w*HB + hi)*NT_j + tile].  It also writes each
-// point in the 2^261 form for the bucket loop, at concatenated point number
-// pbase_j + i of pts29.
-template <class F>
-__global__ void __launch_bounds__(256) k_digits(const MsmSeg *__restrict__ segs, uint32_t J, uint32_t c,
-                                                uint32_t W, uint32_t s, uint32_t ts, uint32_t HB,
-                                                uint32_t *__restrict__ digits, uint32_t *__restrict__ cnt,
-                                                uint32_t *__restrict__ pts29) {
+// Signed c-bit digits of a number of NW words below 2^bits, lowest first:
+// take() gives the next digit's bucket (|d| - 1, or 2^32 - 1 for d == 0) and
+// whether d is negative.
+template <int NW> struct Digits {
+  uint32_t k[NW + 1];
+  uint32_t c, B, mask, carry = 0;
+  __device__ __forceinline__ Digits(const uint32_t *v, uint32_t c_) : c(c_), B(1u << (c_ - 1)), mask((1u << c_) - 1) {
+#pragma unroll
+    for (int i = 0; i < NW; i++) k[i] = v[i];
+    k[NW] = 0;
+  }
+  __device__ __forceinline__ uint32_t take(bool &neg) {
+    uint32_t raw = (k[0] & mask) + carry;
+#pragma unroll
+    for (int i = 0; i < NW; i++) k[i] = __builtin_amdgcn_alignbit(k[i + 1], k[i], c);
+    neg = raw > B;
+    carry = neg;
+    if (neg) raw = (1u << c) - raw;
+    return raw - 1;
+  }
+};
+
+// One workgroup per (member j, tile) of kSortTile points, E of them for each of
+// the caller's (E = 2: P_i and phi(P_i) with the halves of k_i, glv.h; points
+// 2i and 2i + 1 of the member); block b covers the tiles in member order
+// (member j's tiles start at b = tbase_j / W).  Member j's digits occupy
+// D[W*pbase_j + w*n_j + i], b | neg << 31 for the nonzero signed digit d of
+// window w (b = |d| - 1 < B), or 0xFFFFFFFF when d == 0 or the point is at
+// infinity.  The workgroup also counts its digits per (window, hi = b >> s) in
+// LDS and writes the counts as pass 1 of the sort expects them:
+// cnt[cbase_j + (w*HB + hi)*NT_j + tile].  It also writes each point in the
+// 2^261 form for the bucket loop, at concatenated point number pbase_j + i of
+// pts29.
+//
+// Splitting halves the windows and doubles the points: as many entries, half
+// the buckets to reduce and half the doublings of the window combination, for
+// one product more per point and the second point's 64 B (128 B on G2) here.
+template <class F, int E>
+__global__ void __launch_bounds__(1024) k_digits(const MsmSeg *__restrict__ segs, uint32_t J, uint32_t c,
+                                                 uint32_t W, uint32_t s, uint32_t ts, uint32_t HB,
+                                                 uint32_t *__restrict__ digits, uint32_t *__restrict__ cnt,
+                                                 uint32_t *__restrict__ pts29) {
   extern __shared__ uint32_t hist[];  // W * HB counters
   const uint32_t j = member_of_tile(segs, J, W * blockIdx.x);
   const uint32_t tile = blockIdx.x - segs[j].tbase / W;
@@ -106,39 +165,38 @@ __global__ void __launch_bounds__(256) k_digits(const MsmSeg *__restrict__ segs,
   for (uint32_t i = threadIdx.x; i < W * HB; i += blockDim.x) hist[i] = 0;
   __syncthreads();
   constexpr int PW = 2 * FieldIO<F>::NW;
-  const uint32_t B = 1u << (c - 1);
-  const uint32_t mask = (1u << c) - 1;
   uint32_t *dj = digits + W * pbase;
-  for (uint32_t t = threadIdx.x; t < kSortTile; t += blockDim.x) {
-    const uint64_t i = (uint64_t)tile * kSortTile + t;
-    if (i >= n) break;
-    uint32_t k[9];
+  for (uint32_t t = threadIdx.x; t < kSortTile / E; t += blockDim.x) {
+    const uint64_t i = (uint64_t)tile * (kSortTile / E) + t;
+    if (E * i >= n) break;
+    uint32_t k[8];
     ld8(k, segs[j].scalars + i * 8);
-    k[8] = 0;
     reduce_mod_r(k);
     const Affine<F> p = load_affine<F>(segs[j].points + i * PW);
     const bool zero = affine_is_inf(p);
-    store_point29(pts29 + (pbase + i) * PW, p);
-    uint32_t carry = 0;
-    for (uint32_t w = 0; w < W; w++) {
-      uint32_t off = w * c;
-      uint32_t li = off >> 5, sh = off & 31;
-      uint64_t two = (uint64_t)k[li] | ((uint64_t)(li < 7 ? k[li + 1] : 0u) << 32);
-      uint32_t raw = (uint32_t)(two >> sh) & mask;
-      raw += carry;
-      uint32_t mag, neg;
-      if (raw > B) {
-        mag = (1u << c) - raw;
-        neg = 1;
-        carry = 1;
-      } else {
-        mag = raw;
-        neg = 0;
-        carry = 0;
+    store_point29<E>(pts29 + (pbase + E * i) * PW, p);
+    auto entry = [&](uint32_t w, uint32_t b, bool neg) -> uint32_t {
+      const bool live = b != 0xFFFFFFFFu && !zero;
+      if (live) atomicAdd(&hist[w * HB + (b >> (w == W - 1 ? ts : s))], 1u);
+      return live ? b | ((uint32_t)neg << 31) : 0xFFFFFFFFu;
+    };
+    if constexpr (E == 2) {
+      uint32_t k1[4], k2[4];
+      const uint32_t sg = glv_split(k, k1, k2);
+      Digits<4> d1(k1, c), d2(k2, c);
+      for (uint32_t w = 0; w < W; w++) {
+        bool n1, n2;
+        const uint32_t b1 = d1.take(n1), b2 = d2.take(n2);
+        *reinterpret_cast<uint2 *>(dj + (uint64_t)w * n + 2 * i) =
+            make_uint2(entry(w, b1, n1 != (bool)(sg & 1)), entry(w, b2, n2 != (bool)(sg >> 1)));
       }
-      const bool live = mag != 0 && !zero;
-      dj[(uint64_t)w * n + i] = live ? ((mag - 1) | (neg << 31)) : 0xFFFFFFFFu;
-      if (live) atomicAdd(&hist[w * HB + ((mag - 1) >> (w == W - 1 ? ts : s))], 1u);
+    } else {
+      Digits<8> d(k, c);
+      for (uint32_t w = 0; w < W; w++) {
+        bool neg;
+        const uint32_t b = d.take(neg);
+        dj[(uint64_t)w * n + i] = entry(w, b, neg);
+      }
     }
   }
   __syncthreads();
@@ -1065,8 +1123,14 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
 
   if (tm) tm->mark(0, st);
   if (pl.n > 0) {
-    k_digits<F><<<(uint32_t)pl.tiles, 256, pl.W * HB * 4, st>>>(segs, pl.J, pl.c, pl.W, sb, pl.st, HB, digits, cnt,
-                                                                   pts29);
+    // few tiles leave most of the GPU idle: more threads share a tile's points
+    const uint32_t DT = pl.tiles >= 1024 ? 256 : 1024;
+    if (pl.E == 2)
+      k_digits<F, 2><<<(uint32_t)pl.tiles, DT, pl.W * HB * 4, st>>>(segs, pl.J, pl.c, pl.W, sb, pl.st, HB, digits,
+                                                                    cnt, pts29);
+    else
+      k_digits<F, 1><<<(uint32_t)pl.tiles, DT, pl.W * HB * 4, st>>>(segs, pl.J, pl.c, pl.W, sb, pl.st, HB, digits,
+                                                                    cnt, pts29);
     CSK_CHECK_LAUNCH();
     k_scan_reduce<<<nb, SCAN_THREADS, 0, st>>>(cnt, ncnt, bsum);
     k_scan_blocks<<<1, 1024, 0, st>>>(bsum, nb);
@@ -1131,10 +1195,10 @@ __global__ void __launch_bounds__(256) k_table_build(const uint32_t *__restrict_
   if ((threadIdx.x & 31) == 0 && i < n_pad) live[i >> 5] = (uint32_t)(m >> (threadIdx.x & 32));
   if (inf) return;
   XYZZ<F> acc = XYZZ<F>::from_affine(p);
-  store_point29(table + i * PW, p);
+  store_point29<1>(table + i * PW, p);
   for (uint32_t w = 1; w < Wt; w++) {
     for (uint32_t k = 0; k < c; k++) acc = xyzz_dbl(acc);
-    store_point29(table + ((uint64_t)w * n_pad + i) * PW, xyzz_to_affine(acc));
+    store_point29<1>(table + ((uint64_t)w * n_pad + i) * PW, xyzz_to_affine(acc));
   }
 }
 
@@ -1162,38 +1226,23 @@ __global__ void __launch_bounds__(256) k_digits_tab(TabArgs args, const MsmSeg *
   cnt += g0.cbase;
   for (uint32_t i = threadIdx.x; i < Wt * HB; i += blockDim.x) hist[i] = 0;
   __syncthreads();
-  const uint32_t B = 1u << (c - 1);
-  const uint32_t mask = (1u << c) - 1;
   for (uint32_t t = threadIdx.x; t < kSortTile; t += blockDim.x) {
     const uint64_t i = (uint64_t)tile * kSortTile + t;
     if (i >= n) {
       for (uint32_t w = 0; w < Wt; w++) digits[(uint64_t)w * n_pad + i] = 0xFFFFFFFFu;
       continue;
     }
-    uint32_t k[9];
+    uint32_t k[8];
     ld8(k, scalars + i * 8);
-    k[8] = 0;
     reduce_mod_r(k);
     const bool zero = ((live[i >> 5] >> (i & 31)) & 1u) == 0;
-    uint32_t carry = 0;
+    Digits<8> d(k, c);
     for (uint32_t w = 0; w < Wt; w++) {
-      uint32_t off = w * c;
-      uint32_t li = off >> 5, sh = off & 31;
-      uint64_t two = (uint64_t)k[li] | ((uint64_t)(li < 7 ? k[li + 1] : 0u) << 32);
-      uint32_t raw = ((uint32_t)(two >> sh) & mask) + carry;
-      uint32_t mag, neg;
-      if (raw > B) {
-        mag = (1u << c) - raw;
-        neg = 1;
-        carry = 1;
-      } else {
-        mag = raw;
-        neg = 0;
-        carry = 0;
-      }
-      const bool lv = mag != 0 && !zero;
-      digits[(uint64_t)w * n_pad + i] = lv ? ((mag - 1) | (neg << 31)) : 0xFFFFFFFFu;
-      if (lv) atomicAdd(&hist[w * HB + ((mag - 1) >> (w == Wt - 1 ? ts : s))], 1u);
+      bool neg;
+      const uint32_t b = d.take(neg);
+      const bool lv = b != 0xFFFFFFFFu && !zero;
+      digits[(uint64_t)w * n_pad + i] = lv ? b | ((uint32_t)neg << 31) : 0xFFFFFFFFu;
+      if (lv) atomicAdd(&hist[w * HB + (b >> (w == Wt - 1 ? ts : s))], 1u);
     }
   }
   __syncthreads();

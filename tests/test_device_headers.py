@@ -42,3 +42,26 @@ def test_division_step_inverse(tmp_path, p):
         o = W8()
         L.inv(words(x), words(p), np_, o)
         assert value(o) < p and value(o) * x % p == 1, hex(x)
+
+
+LAMBDA = 4407920970296243842393367215006156084916469457145843978461
+
+
+def test_scalar_split(tmp_path):
+    L = compiled(tmp_path, "glv.h", "uint32_t split(const uint32_t *k, uint32_t *a, uint32_t *b) "
+                                    "{ return csk::glv_split(k, a, b); }")
+    assert pow(LAMBDA, 3, R) == 1 and LAMBDA != 1
+    rng = random.Random(6)
+    ks = [0, 1, 2, R - 1, R - 2, R // 2, R // 2 + 1, R // 3, LAMBDA, LAMBDA - 1, LAMBDA + 1, R - LAMBDA, (1 << 253)]
+    ks += [rng.randrange(R) for _ in range(5000)] + [rng.randrange(1 << rng.randrange(1, 253)) for _ in range(500)]
+    # where c1 or c2 is half way between two whole numbers
+    for n in (9931322734385697763, 147946756881789319000765030803803410728):
+        ks += [x for c in (0, 1, 12345, n - 1) for d in range(-2, 3) for x in [(2 * c + 1) * R // (2 * n) + d] if 0 <= x < R]
+    for k in ks:
+        a, b = W8(), W8()
+        neg = L.split(words(k), a, b)
+        k1 = -value(a) if neg & 1 else value(a)
+        k2 = -value(b) if neg & 2 else value(b)
+        assert (k1 + k2 * LAMBDA - k) % R == 0 and abs(k1) < 1 << 126 and abs(k2) < 1 << 126, hex(k)
+        if k < 1 << 100:
+            assert (k1, k2) == (k, 0)  # small scalars (most wire values) stay small
