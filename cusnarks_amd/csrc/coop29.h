@@ -15,6 +15,7 @@
 // Ranges: X < 8q per component, Y, ZZ, ZZZ < 2q; each operation's bound is
 // noted in its program.
 #pragma once
+#include "curve.h"
 #include "row29.h"
 
 namespace csk {
@@ -274,6 +275,115 @@ template <> struct Coop29<Fq2> {
     const uint32_t k = threadIdx.x & 15;
     const uint32_t x = sh[16 * s[0] + k], y = sh[16 * s[1] + k];
     return row_is_zero(x) && row_is_zero(y);
+  }
+};
+
+// ------------------------------------------------------------ accumulators
+// A running point that a workgroup of RowAcc<F>::N threads holds, over stored
+// 29-bit slots (limbs below 2^29 + 4 allowed): G1 in one wave's registers, G2 in
+// LDS.  Infinity is tracked in a flag every lane holds.
+template <class F> struct RowAcc;
+template <> struct RowAcc<Fq> {
+  static constexpr int N = 64, kLds = 1, SW = 36;
+  RowG1K k;
+  RowG1 p;
+  bool inf;
+  __device__ __forceinline__ RowAcc(uint32_t *, const uint32_t *slot) : p(row_load_g1(slot)) { inf = row_is_zero(p.ZZ); }
+  __device__ __forceinline__ void dbl(uint32_t n) {
+    if (inf) return;
+#pragma unroll 1
+    for (uint32_t i = 0; i < n; i++) row_dbl(k, p);
+  }
+  __device__ __forceinline__ void add(const uint32_t *slot) {
+    const RowG1 q = row_load_g1(slot);
+    if (row_is_zero(q.ZZ)) return;
+    if (inf) {
+      p = q;
+      inf = false;
+    } else {
+      row_add(k, p, q, inf);
+    }
+  }
+  __device__ __forceinline__ void store(uint32_t *slot) const {
+    const uint32_t l = threadIdx.x;
+    if (l < 9) {
+      slot[l] = p.X;
+      slot[9 + l] = p.Y;
+      slot[18 + l] = inf ? 0u : p.ZZ;
+      slot[27 + l] = inf ? 0u : p.ZZZ;
+    }
+  }
+  __device__ __forceinline__ void store_affine_to(uint32_t *out) const {
+    const Fq29 X = row_gather(p.X), Y = row_gather(p.Y), ZZ = row_gather(p.ZZ), ZZZ = row_gather(p.ZZZ);
+    if (threadIdx.x == 0) {
+      XYZZ<Fq> a;
+      from29_words(X, a.X.v);
+      from29_words(Y, a.Y.v);
+      from29_words(ZZ, a.ZZ.v);
+      from29_words(ZZZ, a.ZZZ.v);
+      if (inf) a = XYZZ<Fq>::inf();
+      store_affine(out, xyzz_to_affine(a));
+    }
+  }
+};
+
+template <> struct RowAcc<Fq2> {
+  using C = Coop29<Fq2>;
+  static constexpr int N = 16 * C::kRows, kLds = C::kSlots * 16, SW = 72;
+  C prog;
+  uint32_t *sh;
+  bool inf;
+  // slot word of element word i of a stored slot
+  __device__ __forceinline__ static uint32_t at(uint32_t i) { return 16 * (i / 9) + i % 9; }
+  __device__ __forceinline__ RowAcc(uint32_t *lds, const uint32_t *slot) : prog(lds), sh(lds) {
+    if (threadIdx.x < SW) sh[at(threadIdx.x)] = slot[threadIdx.x];
+    __syncthreads();
+    inf = prog.is_zero(C::ZZ);
+  }
+  __device__ __forceinline__ void dbl(uint32_t n) {
+    if (inf) return;
+#pragma unroll 1
+    for (uint32_t i = 0; i < n; i++) prog.dbl();
+  }
+  __device__ __forceinline__ void add(const uint32_t *slot) {
+    __syncthreads();  // every wave is done with the last addend
+    if (threadIdx.x < SW) sh[16 * C::NC + at(threadIdx.x)] = slot[threadIdx.x];
+    __syncthreads();
+    if (prog.is_zero(C::QZZ)) return;
+    if (inf) {
+      if (threadIdx.x < 16 * C::NC) sh[threadIdx.x] = sh[16 * C::NC + threadIdx.x];
+      __syncthreads();
+      inf = false;
+      return;
+    }
+    prog.add1();
+    if (prog.is_zero(C::PP)) {
+      const bool same = prog.is_zero(C::RR);
+      __syncthreads();  // every wave has read PP and RR
+      if (same) prog.dbl();  // acc == q
+      else inf = true;       // acc == -q
+      return;
+    }
+    prog.add2();
+  }
+  __device__ __forceinline__ void store(uint32_t *slot) const {
+    if (threadIdx.x < SW) slot[threadIdx.x] = inf && threadIdx.x >= SW / 2 ? 0u : sh[at(threadIdx.x)];
+  }
+  __device__ __forceinline__ void store_affine_to(uint32_t *out) const {
+    if (threadIdx.x >= 64) return;
+    uint32_t wds[8 * C::NC];
+#pragma unroll
+    for (int k = 0; k < C::NC; k++) {
+      uint32_t o[8];
+      from29_words(row_gather(sh[16 * k + (threadIdx.x & 15)]), o);
+#pragma unroll
+      for (int i = 0; i < 8; i++) wds[8 * k + i] = o[i];
+    }
+    if (threadIdx.x == 0) {
+      XYZZ<Fq2> acc = load_xyzz<Fq2>(wds);
+      if (inf) acc = XYZZ<Fq2>::inf();
+      store_affine(out, xyzz_to_affine(acc));
+    }
   }
 };
 

@@ -147,6 +147,33 @@ __device__ __forceinline__ void mul29x2(const Fq29 &a, const Fq29 &b, const Fq29
   cd.l[8] = (uint32_t)acd;
 }
 
+// One product whose a*b and reduction products run on two chains, merged once
+// per column: for code with a single product to form at a time.
+__device__ __forceinline__ Fq29 mul29_2c(const Fq29 &a, const Fq29 &b) {
+  uint32_t m[9];
+  Fq29 r;
+  uint64_t acc = 0;
+#pragma unroll
+  for (int k = 0; k < 17; k++) {
+    uint64_t u = 0;
+#pragma unroll
+    for (int j = (k > 8 ? k - 8 : 0); j <= (k < 8 ? k : 8); j++) {
+      mad29(u, a.l[j], b.l[k - j]);
+      if (j < k && j < 9) mad29(acc, m[j], Q29::p[k - j]);
+    }
+    acc += u;
+    if (k < 9) {
+      m[k] = ((uint32_t)acc * Q29::np) & Q29::M;
+      mad29(acc, m[k], Q29::p[0]);
+    } else {
+      r.l[k - 9] = (uint32_t)acc & Q29::M;
+    }
+    acc >>= 29;
+  }
+  r.l[8] = (uint32_t)acc;
+  return r;
+}
+
 // a^2 and c^2 (normalised a, c), interleaved as mul29x2: each cross product
 // a_i a_j (i < j) once, on the doubled limb 2 a_i (< 2^30), 126 multiply-adds
 // per square instead of 162.

@@ -75,10 +75,10 @@ struct TabArgs {
 // of run p, n = the table's n_pad, points = that window's slice), copied into
 // the workspace; max_nt: the largest n_pad / 4096 among the runs.
 int msm_run_table_g1(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArgs &args, uint32_t count,
-                     uint32_t max_nt, uint32_t Lrm, uint32_t Sm, hipStream_t st);
+                     uint32_t max_nt, uint32_t Lrm, hipStream_t st);
 int msm_run_table_g2(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArgs &args, uint32_t count,
-                     uint32_t max_nt, uint32_t Lrm, uint32_t Sm, hipStream_t st);
-size_t msm_table_ws_bytes(const MsmPlan &pl, bool g2, uint32_t Sm, uint32_t count);
+                     uint32_t max_nt, uint32_t Lrm, hipStream_t st);
+size_t msm_table_ws_bytes(const MsmPlan &pl, bool g2, uint32_t count);
 
 // looks up this device's copy of the no-allocation scratch array (the device current)
 int msm_noalloc_setup(int device);

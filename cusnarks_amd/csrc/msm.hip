@@ -16,8 +16,10 @@
 //                    array into XYZZ bucket sums with mixed additions; runs
 //                    that start in an earlier chunk are handed over as carries.
 //   5. k_fixup       the owner of each bucket split over chunks adds the carries.
-//   6. k_bucket_reduce  per (window, segment): sum_b (b+1) B_b by running sums.
-//   7. k_window_reduce  per window: sum of the segment results.
+//   6. k_bucket_reduce  per (window, segment): sum B_b and sum (b+1) B_b by
+//                    running sums.
+//   7. k_tree, k_window_horner  per window: the segments joined pairwise, then
+//                    their weights' powers of two.
 //   8. k_final       Horner over the windows (c doublings each) -> affine.
 #include <vector>
 #include "internal.h"
@@ -105,7 +107,7 @@ MsmPlan msm_group_plan(uint32_t c, uint32_t E, const uint64_t *n, uint32_t J, bo
   // buckets per reduction thread: aim for ~2^15 reduction threads
   const uint64_t Ktot = (uint64_t)J * pl.K;
   uint32_t lr = 16;
-  if (reduce_seg) lr = reduce_seg;
+  if (reduce_seg) lr = reduce_seg < 2 ? 2 : reduce_seg;  // a segment keeps two sums in its slots
   else
     while (lr > 2 && Ktot / lr < (1u << 15)) lr >>= 1;
   if (lr > pl.B) lr = pl.B;
@@ -147,7 +149,6 @@ size_t msm_workspace_bytes(const MsmPlan &pl, bool g2) {
   b += Carver::round(nb * 4);                   // scan block sums
   b += Carver::round((Ktot + 1) * 4);           // bucket offsets
   b += Carver::round(pl.max_chunks * 4);        // carry keys
-  b += Carver::round(Wtot * pl.S * (g2 ? 288 : 144)); // partials (29-bit slots)
   b += Carver::round(Wtot * (g2 ? 288 : 144));  // window sums (29-bit slots)
   return b + 4096;
 }
@@ -264,6 +265,14 @@ int msm_noalloc_setup(int device) {
   return CSK_OK;
 }
 
+// The bytes that decide which widths the array takes: the workspace of the
+// whole-scalar plan and a slot per reduction segment.  The pipeline that runs
+// needs no more, so a width is accepted or refused by n and cfg alone.
+static size_t noalloc_bytes(const MsmPlan &pl, uint32_t rseg) {
+  const uint32_t seg = rseg && rseg < pl.Lr ? rseg : pl.Lr;
+  return msm_workspace_bytes(pl, false) + Carver::round((uint64_t)pl.J * pl.W * (pl.B / seg) * 144);
+}
+
 // out = (0, 1*R), the affine point at infinity of the empty sum
 __global__ void k_put_inf_g1(uint32_t *out) {
   uint32_t i = threadIdx.x;
@@ -309,7 +318,7 @@ extern "C" int csk_msm_g1_noalloc(csk_ctx *ctx, const uint32_t *d_scalars, const
   const uint32_t rseg = cfg && cfg->reduce_seg ? cfg->reduce_seg : (!fixed_c ? tn->reduce_seg : 0);
   const size_t seg_bytes = Carver::round(2 * sizeof(MsmSeg));
   MsmPlan pl = msm_group_plan(c, 1, &n, 1, false, chunk, rseg);
-  while (!fixed_c && c > 2 && (!msm_plan_ok(pl) || seg_bytes + msm_workspace_bytes(pl, false) > kNoAllocBytes)) {
+  while (!fixed_c && c > 2 && (!msm_plan_ok(pl) || seg_bytes + noalloc_bytes(pl, rseg) > kNoAllocBytes)) {
     c--;
     pl = msm_group_plan(c, 1, &n, 1, false, chunk, rseg);
   }
@@ -317,9 +326,9 @@ extern "C" int csk_msm_g1_noalloc(csk_ctx *ctx, const uint32_t *d_scalars, const
     set_error("msm_g1_noalloc: unsupported configuration (window/chunk/segment)");
     return CSK_ERR_ARG;
   }
-  if (seg_bytes + msm_workspace_bytes(pl, false) > kNoAllocBytes) {
+  if (seg_bytes + noalloc_bytes(pl, rseg) > kNoAllocBytes) {
     set_error("msm_g1_noalloc: the workspace for window width " + std::to_string(pl.c) + " needs " +
-              std::to_string(seg_bytes + msm_workspace_bytes(pl, false)) + " bytes, more than the " +
+              std::to_string(seg_bytes + noalloc_bytes(pl, rseg)) + " bytes, more than the " +
               std::to_string(kNoAllocBytes) + "-byte scratch array");
     return CSK_ERR_ARG;
   }
@@ -346,7 +355,7 @@ struct csk_msm_table {
   uint32_t c = 0, Wt = 0;
   uint32_t *table = nullptr;  // Wt * n_pad points in the 2^261 form
   uint32_t *live = nullptr;   // one bit per point: not at infinity
-  uint32_t Lrm = 0, Sm = 0;
+  uint32_t Lrm = 0;
   uint64_t table_bytes = 0;
 };
 
@@ -447,7 +456,7 @@ static int table_run(csk_ctx *ctx, uint32_t count, csk_msm_table *const *t, cons
   }
   std::vector<MsmSeg> segs(pl.J + 1);
   msm_fill_segs(pl, ns.data(), sc.data(), pts.data(), outs.data(), segs.data());
-  int rc = ctx->ws.ensure(msm_table_ws_bytes(pl, t0->ec2 != 0, t0->Sm, count));
+  int rc = ctx->ws.ensure(msm_table_ws_bytes(pl, t0->ec2 != 0, count));
   if (rc) return rc;
   TabArgs args = {};
   for (uint32_t p = 0; p < count; p++) {
@@ -456,8 +465,8 @@ static int table_run(csk_ctx *ctx, uint32_t count, csk_msm_table *const *t, cons
     args.live[p] = t[p]->live;
     args.n[p] = t[p]->n;
   }
-  return t0->ec2 ? msm_run_table_g2(ctx->ws.ptr, pl, segs.data(), args, count, max_nt, t0->Lrm, t0->Sm, st)
-                 : msm_run_table_g1(ctx->ws.ptr, pl, segs.data(), args, count, max_nt, t0->Lrm, t0->Sm, st);
+  return t0->ec2 ? msm_run_table_g2(ctx->ws.ptr, pl, segs.data(), args, count, max_nt, t0->Lrm, st)
+                 : msm_run_table_g1(ctx->ws.ptr, pl, segs.data(), args, count, max_nt, t0->Lrm, st);
 }
 
 }  // namespace csk
@@ -505,7 +514,6 @@ extern "C" int csk_msm_table_create(csk_ctx *ctx, int ec2, const uint32_t *d_poi
   while (lr > 2 && pl.B / lr < (1u << 15)) lr >>= 1;
   if (lr > pl.B) lr = pl.B;
   t->Lrm = lr;
-  t->Sm = pl.B / lr;
   const uint64_t PW = ec2 ? 32 : 16;
   t->table_bytes = table_point_bytes(t->ec2, n_pad, Wt);
   hipError_t e = hipMalloc(&t->table, (size_t)Wt * n_pad * PW * 4);
@@ -579,7 +587,7 @@ extern "C" int csk_msm_table_run_multi(csk_ctx *ctx, uint32_t count, csk_msm_tab
 extern "C" int csk_msm_table_info(const csk_msm_table *t, uint64_t *out, int n) {
   if (!t || !out || n < 1) return CSK_ERR_ARG;
   const MsmPlan pl = table_plan(t->c, t->n_pad, t->Wt, 1);
-  const uint64_t v[5] = {t->n, t->c, t->Wt, t->table_bytes, msm_table_ws_bytes(pl, t->ec2 != 0, t->Sm, 1)};
+  const uint64_t v[5] = {t->n, t->c, t->Wt, t->table_bytes, msm_table_ws_bytes(pl, t->ec2 != 0, 1)};
   for (int i = 0; i < n && i < 5; i++) out[i] = v[i];
   return CSK_OK;
 }

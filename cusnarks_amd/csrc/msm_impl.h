@@ -8,6 +8,7 @@
 #include "field29.h"
 #include "coop29.h"
 #include "glv.h"
+#include "quad29.h"
 #include "msm.h"
 
 namespace csk {
@@ -816,10 +817,12 @@ __device__ __forceinline__ void load29(const uint32_t *s, XYZZ2_29 &a) {
 template <class F> struct Acc29;
 template <> struct Acc29<Fq> {
   using T = XYZZ29;
+  using Q = Fq29;  // one lane's part in a quad
   __device__ __forceinline__ static T inf() { return inf29(); }
 };
 template <> struct Acc29<Fq2> {
   using T = XYZZ2_29;
+  using Q = Fq2_29;
   __device__ __forceinline__ static T inf() { return inf2_29(); }
 };
 
@@ -830,29 +833,38 @@ template <> struct Acc29<Fq2> {
 // step 8^r the slot at chain index i (i % 8^(r+1) == 0) adds the slots at
 // i + k*8^r, k = 1..7, that lie in the chain.  The slots read are never
 // written in the same round.  Slots are 29-bit (SW words).
+// A quad of lanes per slot (quad29.h): a round is a chain of up to seven
+// additions, and few slots of a round head one.
 template <class F>
 __global__ void __launch_bounds__(256) k_carry_round(const uint32_t *__restrict__ off, uint32_t K, uint32_t L,
                                                      uint32_t *__restrict__ carry,
                                                      const uint32_t *__restrict__ carry_key, uint32_t step) {
   constexpr int SW = Slot29<F>::SW;
-  using A = typename Acc29<F>::T;
-  const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
+  using T = typename Acc29<F>::Q;
+  const uint64_t u = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 2;
   const uint32_t E = off[K];
-  if ((uint64_t)u * L >= E) return;
-  const uint32_t key = carry_key[u];
-  if (key == 0xFFFFFFFFu) return;
-  const uint32_t t0 = off[key] / L, t1 = (off[key + 1] - 1) / L;
-  const uint32_t i = u - (t0 + 1), len = t1 - t0;
-  if (((uint64_t)i & (8ull * step - 1)) != 0 || (uint64_t)i + step >= len) return;
-  A a;
-  load29(carry + (uint64_t)u * SW, a);
-#pragma unroll 1
-  for (uint64_t k = 1; k < 8 && i + k * step < len; k++) {
-    A b;
-    load29(carry + (u + k * step) * SW, b);
-    xadd29(a, b);
+  uint32_t i = 0, len = 0;
+  if (u * L < E) {
+    const uint32_t key = carry_key[u];
+    if (key != 0xFFFFFFFFu) {
+      const uint32_t t0 = off[key] / L, t1 = (off[key + 1] - 1) / L;
+      i = (uint32_t)u - (t0 + 1);
+      len = t1 - t0;
+    }
   }
-  store29(carry + (uint64_t)u * SW, a);
+  const bool head = ((uint64_t)i & (8ull * step - 1)) == 0 && (uint64_t)i + step < len;
+  if (!__any(head)) return;
+  T a = {};
+  if (head) quad_load(carry + u * SW, a);
+#pragma unroll 1
+  for (uint64_t k = 1; k < 8; k++) {
+    const bool more = head && i + k * step < len;
+    if (!__any(more)) break;
+    T b = {};  // infinity where the chain has ended
+    if (more) quad_load(carry + (u + k * step) * SW, b);
+    quad_add(a, b);
+  }
+  if (head) quad_store(carry + u * SW, a);
 }
 
 // One thread per bucket: add the (reduced) chain head at slot t0+1.
@@ -875,82 +887,152 @@ __global__ void __launch_bounds__(256) k_fixup(const uint32_t *__restrict__ off,
   store29(buckets + (uint64_t)key * SW, acc);
 }
 
-// per (window, segment): sum_{b in seg} (b+1) * bucket_b
+// ------------------------------------------------------------ window sums
+// sum_b (b + 1) bucket_b of every window, in place in the bucket slots.
+//
+// A node stands for a run of buckets of one window and holds K points at the
+// start of the run's slots: R, the sum of its buckets, A, and C_0 .. C_(K-3),
+// where its weighted sum is A + Lr (C_0 + 2 C_1 + 4 C_2 + ...).  The first
+// nodes are segments of Lr buckets (k_bucket_reduce: running sums; A weights
+// bucket i of the segment i + 1).  Two neighbouring nodes of equal length make
+// one of twice the length (k_tree): R, A and every C_j add, and the upper
+// node's R becomes the new C, whose weight is the lower one's length.  So a
+// window of B buckets takes 2 B additions, about 2 Lr + log2(B / Lr) of them in
+// a row, and no doublings before the last step (k_window_horner), log2(B)
+// doublings and additions of C's on rows of lanes.  The additions run on quads
+// of lanes (quad29.h), as the chain is what costs.
+// Measured, 2^20 points (c = 16, 8 x 32768 buckets): 101 + 67 + 38 us; segments
+// each multiplied by their offset and summed by lanes, 256 + 118 us.
+
+// a quad per (window, segment)
 template <class F>
-__global__ void __launch_bounds__(256) k_bucket_reduce(const uint32_t *__restrict__ off,
-                                                       const uint32_t *__restrict__ buckets, uint32_t W,
-                                                       uint32_t B, uint32_t Lr,
-                                                       uint32_t *__restrict__ partial) {
+__global__ void __launch_bounds__(256) k_bucket_reduce(const uint32_t *__restrict__ off, uint32_t *buckets,
+                                                       uint32_t nseg, uint32_t Lr) {
+  constexpr int SW = Slot29<F>::SW;
+  using T = typename Acc29<F>::Q;
+  const uint32_t seg = (uint32_t)(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 2);
+  const bool live = seg < nseg;
+  const uint64_t lo = (uint64_t)seg * Lr;  // windows follow each other: key = w * B + s * Lr
+  T run = {}, acc = {};
+#pragma unroll 1
+  for (int b = (int)Lr - 1; b >= 0; b--) {
+    T bk = {};
+    const uint64_t key = lo + (uint32_t)b;
+    if (live && off[key + 1] != off[key]) quad_load(buckets + key * SW, bk);
+    quad_add(run, bk);
+    quad_add(acc, run);
+  }
+  if (live) {
+    quad_store(buckets + lo * SW, run);
+    quad_store(buckets + (lo + 1) * SW, acc);
+  }
+}
+
+// the same with a lane per segment
+template <class F>
+__global__ void __launch_bounds__(256) k_bucket_reduce_lanes(const uint32_t *__restrict__ off, uint32_t *buckets,
+                                                             uint32_t nseg, uint32_t Lr) {
   constexpr int SW = Slot29<F>::SW;
   using A = typename Acc29<F>::T;
-  uint32_t S = B / Lr;
-  uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
-  if (tid >= W * S) return;
-  uint32_t w = tid / S, s = tid % S;
-  uint32_t lo = s * Lr;
+  const uint32_t seg = blockIdx.x * blockDim.x + threadIdx.x;
+  if (seg >= nseg) return;
+  const uint64_t lo = (uint64_t)seg * Lr;
   A run = Acc29<F>::inf(), acc = Acc29<F>::inf();
 #pragma unroll 1
-  for (int b = (int)(lo + Lr) - 1; b >= (int)lo; b--) {
-    uint32_t key = w * B + (uint32_t)b;
+  for (int b = (int)Lr - 1; b >= 0; b--) {
+    const uint64_t key = lo + (uint32_t)b;
     if (off[key + 1] != off[key]) {
       A bk;
-      load29(buckets + (uint64_t)key * SW, bk);
+      load29(buckets + key * SW, bk);
       xadd29(run, bk);
     }
     xadd29(acc, run);
   }
-  xadd29(acc, xmul_small29(run, lo, Acc29<F>::inf()));
-  store29(partial + (uint64_t)tid * SW, acc);
+  store29(buckets + lo * SW, run);
+  store29(buckets + (lo + 1) * SW, acc);
 }
 
-// one block per window (256 threads G1, 128 G2): sum of its S segment
-// results, written as a 29-bit slot
+// Threads of the largest k_tree workgroup (the G2 addition takes more than the
+// 128 registers a wave of a 1024-thread workgroup has), and its LDS.
+template <class F> struct TreeDim { static constexpr uint32_t kThreads = std::is_same<F, Fq>::value ? 1024 : 512; };
+static constexpr uint32_t kTreeLds = 65536;
+
+// One workgroup joins n (a power of two) nodes of `span` slots and K points
+// each into one of n * span slots.  It has a quad for each of the (n / 2) K
+// additions and n / 2 copies of its first level; later levels have fewer.
 template <class F>
-__global__ void __launch_bounds__(256) k_window_reduce(const uint32_t *__restrict__ partial, uint32_t S,
-                                                       uint32_t *__restrict__ wsum) {
+__global__ void __launch_bounds__(TreeDim<F>::kThreads) k_tree(uint32_t *slots, uint32_t span, uint32_t K,
+                                                               uint32_t n) {
   constexpr int SW = Slot29<F>::SW;
-  using A = typename Acc29<F>::T;
-  __shared__ uint32_t sh[256 * 36];  // blockDim * SW words
-  uint32_t w = blockIdx.x;
-  A acc = Acc29<F>::inf();
-#pragma unroll 1
-  for (uint32_t s = threadIdx.x; s < S; s += blockDim.x) {
-    A b;
-    load29(partial + ((uint64_t)w * S + s) * SW, b);
-    xadd29(acc, b);
+  using T = typename Acc29<F>::Q;
+  extern __shared__ uint32_t sh[];  // n * K slots: point k of node i at k * n + i
+  uint32_t *base = slots + (uint64_t)blockIdx.x * n * span * SW;
+  for (uint32_t w = threadIdx.x; w < n * K * SW; w += blockDim.x) {
+    const uint32_t i = w / (K * SW), r = w - i * (K * SW), k = r / SW;
+    sh[(k * n + i) * SW + (r - k * SW)] = base[(uint64_t)i * span * SW + r];
   }
-  store29(sh + threadIdx.x * SW, acc);
   __syncthreads();
-  for (uint32_t st = blockDim.x / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) {
-      A a, b;
-      load29(sh + threadIdx.x * SW, a);
-      load29(sh + (threadIdx.x + st) * SW, b);
-      xadd29(a, b);
-      store29(sh + threadIdx.x * SW, a);
+  const uint32_t quad = threadIdx.x >> 2;
+  for (uint32_t m = n; m > 1; m >>= 1, K++) {
+    const uint32_t h = m >> 1;
+    // point k of the new node i; the quads after the additions' copy the upper R
+    const uint32_t k = quad / h, i = quad - k * h;
+    T a = {}, b = {};
+    const bool add = k < K, copy = k == K;
+    if (add) {
+      quad_load(sh + (k * m + 2 * i) * SW, a);
+      quad_load(sh + (k * m + 2 * i + 1) * SW, b);
+    } else if (copy) {
+      quad_load(sh + (2 * i + 1) * SW, a);
     }
+    if (__any(add)) quad_add(a, b);
+    __syncthreads();
+    if (add || copy) quad_store(sh + (k * h + i) * SW, a);
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    for (int k = 0; k < SW; k++) wsum[(uint64_t)w * SW + k] = sh[k];
-  }
+  for (uint32_t w = threadIdx.x; w < K * SW; w += blockDim.x) base[w] = sh[w];
 }
 
-// Window sums from nwin * S segment results (window-major).  One block per
-// window leaves each thread S / blockDim serial additions; above one result
-// per thread the sum runs in two launches: groups of blockDim results into
-// tmp (nwin * S / blockDim slots, which may alias the bucket slots the
-// segment results were made from), then one block per window over those.
+// A + Lr (C_0 + 2 C_1 + ...) of each window's last node (one workgroup per
+// window), a 29-bit slot of limbs below 2^29 + 4
 template <class F>
-void window_sums(const uint32_t *partial, uint32_t nwin, uint32_t S, uint32_t *tmp, uint32_t *wsum,
-                 hipStream_t st) {
-  const uint32_t TB = FieldIO<F>::NW == 16 ? 128 : 256;
-  if (S > TB) {
-    k_window_reduce<F><<<nwin * (S / TB), TB, 0, st>>>(partial, TB, tmp);
-    k_window_reduce<F><<<nwin, TB, 0, st>>>(tmp, S / TB, wsum);
-  } else {
-    k_window_reduce<F><<<nwin, TB, 0, st>>>(partial, S, wsum);
+__global__ void __launch_bounds__(RowAcc<F>::N) k_window_horner(const uint32_t *__restrict__ slots, uint32_t B,
+                                                                uint32_t K, uint32_t lgLr,
+                                                                uint32_t *__restrict__ wsum) {
+  __shared__ uint32_t lds[RowAcc<F>::kLds];
+  constexpr int SW = Slot29<F>::SW;
+  const uint32_t *node = slots + (uint64_t)blockIdx.x * B * SW;
+  RowAcc<F> acc(lds, node + (uint64_t)(K - 1) * SW);
+#pragma unroll 1
+  for (int k = (int)K - 2; k >= 1; k--) {
+    acc.dbl(k == 1 ? lgLr : 1);
+    acc.add(node + (uint64_t)k * SW);
   }
+  acc.store(wsum + (uint64_t)blockIdx.x * SW);
+}
+
+template <class F>
+void window_sums(const uint32_t *off, uint32_t *buckets, uint32_t nwin, uint32_t B, uint32_t Lr, uint32_t *wsum,
+                 hipStream_t st) {
+  const uint32_t nseg = nwin * (B / Lr);
+  // From 2^20 buckets (a wave of segments per SIMD) the additions fill the GPU
+  // with a lane each, which is the fewest instructions; below, quads shorten
+  // the chain (7 x 2^18 buckets: 396 us against 583).
+  if ((uint64_t)nwin * B >= 1u << 20)
+    k_bucket_reduce_lanes<F><<<(nseg + 255) / 256, 256, 0, st>>>(off, buckets, nseg, Lr);
+  else
+    k_bucket_reduce<F><<<(nseg + 63) / 64, 256, 0, st>>>(off, buckets, nseg, Lr);
+  uint32_t N = B / Lr, span = Lr, K = 2;
+  while (N > 1) {
+    uint32_t n = 2;
+    while (n < N && 4 * n * (K + 1) <= TreeDim<F>::kThreads && 2 * n * K * Slot29<F>::SW * 4 <= kTreeLds) n *= 2;
+    const uint32_t th = (2 * n * (K + 1) + 63) / 64 * 64;  // a quad per addition and copy of the first level
+    k_tree<F><<<nwin * (N / n), th, n * K * Slot29<F>::SW * 4, st>>>(buckets, span, K, n);
+    for (uint32_t m = n; m > 1; m >>= 1) K++;
+    span *= n;
+    N /= n;
+  }
+  k_window_horner<F><<<nwin, RowAcc<F>::N, 0, st>>>(buckets, B, K, 31 - __builtin_clz(Lr), wsum);
 }
 
 // One workgroup per member: Horner over its W window sums (c doublings each),
@@ -963,102 +1045,25 @@ void window_sums(const uint32_t *partial, uint32_t nwin, uint32_t S, uint32_t *t
 // lane per product; G2 638 us, 1997 with one lane per product.  One window
 // (table runs: the inversion and the conversions): 50 us, 167 with a binary
 // Euclid.
-template <class F> struct FinalThreads { static constexpr int N = std::is_same<F, Fq>::value ? 64 : 256; };
-
 template <class F>
-__global__ void __launch_bounds__(FinalThreads<F>::N) k_final(const MsmSeg *__restrict__ segs,
-                                                              const uint32_t *__restrict__ wsum, uint32_t W,
-                                                              uint32_t c) {
+__global__ void __launch_bounds__(RowAcc<F>::N) k_final(const MsmSeg *__restrict__ segs,
+                                                        const uint32_t *__restrict__ wsum, uint32_t W, uint32_t c) {
   const uint32_t j = blockIdx.x;
   uint32_t *out = segs[j].out;
   if (segs[j].n == 0) {
     if (threadIdx.x == 0) store_affine(out, Affine<F>{F::zero(), F::one()});
     return;
   }
+  __shared__ uint32_t lds[RowAcc<F>::kLds];
   constexpr int SW = Slot29<F>::SW;
   const uint32_t *ws = wsum + (uint64_t)j * W * SW;
-  if constexpr (std::is_same<F, Fq>::value) {
-    const RowG1K k;
-    RowG1 acc = row_load_g1(ws + (uint64_t)(W - 1) * SW);
-    bool inf = row_is_zero(acc.ZZ);
+  RowAcc<F> acc(lds, ws + (uint64_t)(W - 1) * SW);
 #pragma unroll 1
-    for (int w = (int)W - 2; w >= 0; w--) {
-      const RowG1 q = row_load_g1(ws + (uint64_t)w * SW);
-      if (!inf)
-#pragma unroll 1
-        for (uint32_t i = 0; i < c; i++) row_dbl(k, acc);
-      if (row_is_zero(q.ZZ)) continue;
-      if (inf) {
-        acc = q;
-        inf = false;
-        continue;
-      }
-      row_add(k, acc, q, inf);
-    }
-    const Fq29 X = row_gather(acc.X), Y = row_gather(acc.Y), ZZ = row_gather(acc.ZZ), ZZZ = row_gather(acc.ZZZ);
-    if (threadIdx.x == 0) {
-      XYZZ<F> a;
-      from29_words(X, a.X.v);
-      from29_words(Y, a.Y.v);
-      from29_words(ZZ, a.ZZ.v);
-      from29_words(ZZZ, a.ZZZ.v);
-      if (inf) a = XYZZ<F>::inf();
-      store_affine(out, xyzz_to_affine(a));
-    }
-  } else {
-    using C = Coop29<F>;
-    constexpr int NC = C::NC;
-    __shared__ uint32_t sh[C::kSlots * 16];
-    C prog(sh);
-    // slot word of element word i of a window sum
-    auto slot = [](uint32_t i) { return 16 * (i / 9) + i % 9; };
-    for (uint32_t i = threadIdx.x; i < (uint32_t)SW; i += blockDim.x) sh[slot(i)] = ws[(uint64_t)(W - 1) * SW + i];
-    __syncthreads();
-    bool inf = prog.is_zero(C::ZZ);
-#pragma unroll 1
-    for (int w = (int)W - 2; w >= 0; w--) {
-      if (!inf)
-#pragma unroll 1
-        for (uint32_t i = 0; i < c; i++) prog.dbl();
-      for (uint32_t i = threadIdx.x; i < (uint32_t)SW; i += blockDim.x)
-        sh[16 * NC + slot(i)] = ws[(uint64_t)w * SW + i];
-      __syncthreads();
-      if (prog.is_zero(C::QZZ)) {
-        __syncthreads();  // every wave has read the addend before the next one is loaded
-        continue;
-      }
-      if (inf) {
-        for (uint32_t i = threadIdx.x; i < 16 * NC; i += blockDim.x) sh[i] = sh[16 * NC + i];
-        __syncthreads();
-        inf = false;
-        continue;
-      }
-      prog.add1();
-      if (prog.is_zero(C::PP)) {
-        const bool same = prog.is_zero(C::RR);
-        __syncthreads();  // every wave has read PP and RR
-        if (same) prog.dbl();  // acc == q
-        else inf = true;       // acc == -q
-        continue;
-      }
-      prog.add2();
-    }
-    if (threadIdx.x < 64) {
-      uint32_t wds[4 * FieldIO<F>::NW];
-#pragma unroll
-      for (int k = 0; k < NC; k++) {
-        uint32_t o[8];
-        from29_words(row_gather(sh[16 * k + (threadIdx.x & 15)]), o);
-#pragma unroll
-        for (int i = 0; i < 8; i++) wds[8 * k + i] = o[i];
-      }
-      if (threadIdx.x == 0) {
-        XYZZ<F> acc = load_xyzz<F>(wds);
-        if (inf) acc = XYZZ<F>::inf();
-        store_affine(out, xyzz_to_affine(acc));
-      }
-    }
+  for (int w = (int)W - 2; w >= 0; w--) {
+    acc.dbl(c);
+    acc.add(ws + (uint64_t)w * SW);
   }
+  acc.store_affine_to(out);
 }
 
 // The sort's placement passes over the counted and scanned digits: pass 1
@@ -1114,7 +1119,6 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
   uint32_t *bsum = cv.take<uint32_t>(nb);
   uint32_t *offsets = cv.take<uint32_t>((size_t)Ktot + 1);
   uint32_t *carry_key = cv.take<uint32_t>(pl.max_chunks);
-  uint32_t *partial = cv.take<uint32_t>((size_t)Wtot * pl.S * SW);
   uint32_t *wsum = cv.take<uint32_t>((size_t)Wtot * SW);
   // the pass-1 arrays are free once the sort is done: bucket and carry slots
   Carver c29(after);
@@ -1148,17 +1152,15 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
     if (tm) tm->mark(2, st);
     // chains can be at most max_chunks long
     for (uint64_t step = 1; step < pl.max_chunks; step *= 8)
-      k_carry_round<F><<<ga, TB, 0, st>>>(offsets, Ktot, pl.L, cr29, carry_key, (uint32_t)step);
+      k_carry_round<F><<<(uint32_t)((pl.max_chunks + 63) / 64), 256, 0, st>>>(offsets, Ktot, pl.L, cr29, carry_key,
+                                                                               (uint32_t)step);
     CSK_CHECK_LAUNCH();
     k_fixup<F><<<(Ktot + TB - 1) / TB, TB, 0, st>>>(offsets, Ktot, pl.L, b29, cr29);
     CSK_CHECK_LAUNCH();
-    uint32_t nseg = Wtot * pl.S;
-    k_bucket_reduce<F><<<(nseg + TB - 1) / TB, TB, 0, st>>>(offsets, b29, Wtot, pl.B, pl.Lr, partial);
-    CSK_CHECK_LAUNCH();
-    window_sums<F>(partial, Wtot, pl.S, b29, wsum, st);  // the bucket slots are free again
+    window_sums<F>(offsets, b29, Wtot, pl.B, pl.Lr, wsum, st);
     CSK_CHECK_LAUNCH();
   }
-  k_final<F><<<pl.J, FinalThreads<F>::N, 0, st>>>(segs, wsum, pl.W, pl.c);
+  k_final<F><<<pl.J, RowAcc<F>::N, 0, st>>>(segs, wsum, pl.W, pl.c);
   CSK_CHECK_LAUNCH();
   if (tm) tm->mark(3, st);
   return CSK_OK;
@@ -1298,7 +1300,7 @@ __global__ void k_put_outs(TabArgs args, uint32_t count, MsmSeg *osegs) {
 
 // Workspace of a table run over count scalar vectors, carved in this order
 // by msm_run_table.
-inline size_t msm_table_workspace_bytes(const MsmPlan &pl, bool g2, uint32_t Sm, uint32_t count) {
+inline size_t msm_table_workspace_bytes(const MsmPlan &pl, bool g2, uint32_t count) {
   const uint32_t hi_bits = pl.hb;
   const uint64_t ncnt = (uint64_t)pl.W * (1u << hi_bits) * pl.tiles;
   const uint64_t nb = (ncnt + SCAN_TILE - 1) / SCAN_TILE;
@@ -1316,7 +1318,6 @@ inline size_t msm_table_workspace_bytes(const MsmPlan &pl, bool g2, uint32_t Sm,
   b += Carver::round(pl.max_chunks * 4);
   b += Carver::round((uint64_t)count * pl.B * sb);        // merged buckets
   b += Carver::round(((uint64_t)count * pl.B + 1) * 4);   // iota offsets
-  b += Carver::round((uint64_t)count * Sm * sb);          // partials of the merged windows
   b += Carver::round((uint64_t)count * sb);               // their sums
   b += Carver::round((uint64_t)(count + 1) * sizeof(MsmSeg));  // output descriptors
   b += Carver::round(((uint64_t)pl.J + 1) * sizeof(MsmSeg));   // member descriptors
@@ -1327,10 +1328,10 @@ inline size_t msm_table_workspace_bytes(const MsmPlan &pl, bool g2, uint32_t Sm,
 // table -> args.o[p]): pl is the group plan of the count * Wt one-window
 // members m = p * Wt + w (J = count * Wt, W = 1), hsegs their host
 // descriptors (member m reads its table's slice of window w through its points
-// pointer), Lrm / Sm the reduction split of a merged window.
+// pointer), Lrm the buckets a reduction quad sums of a merged window.
 template <class F>
 int msm_run_table(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArgs &args, uint32_t count,
-                  uint32_t max_nt, uint32_t Lrm, uint32_t Sm, hipStream_t st) {
+                  uint32_t max_nt, uint32_t Lrm, hipStream_t st) {
   const bool g2 = FieldIO<F>::NW == 16;
   constexpr int SW = Slot29<F>::SW;
   Carver cv(ws);
@@ -1339,7 +1340,7 @@ int msm_run_table(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArg
   const uint32_t nblk = (uint32_t)(pl.W * pl.tiles);
   const uint32_t ncnt = nblk * HB;
   const uint32_t nb = (ncnt + SCAN_TILE - 1) / SCAN_TILE;
-  const uint32_t Ktot = pl.J * pl.K, Wtot = pl.J * pl.W;
+  const uint32_t Ktot = pl.J * pl.K;
   uint32_t *digits = cv.take<uint32_t>(pl.max_entries);
   uint32_t *sorted = cv.take<uint32_t>(pl.max_entries + 4);
   const uint64_t sortb = Carver::round(pl.max_entries * 4) + pl.max_entries * 2;
@@ -1357,7 +1358,6 @@ int msm_run_table(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArg
   uint32_t *carry_key = cv.take<uint32_t>(pl.max_chunks);
   uint32_t *merged = cv.take<uint32_t>((size_t)count * pl.B * SW);
   uint32_t *iota = cv.take<uint32_t>((size_t)count * pl.B + 1);
-  uint32_t *partial = cv.take<uint32_t>((size_t)count * Sm * SW);
   uint32_t *wsum = cv.take<uint32_t>((size_t)count * SW);
   MsmSeg *osegs = cv.take<MsmSeg>(count + 1);
   MsmSeg *segs = cv.take<MsmSeg>(pl.J + 1);
@@ -1381,15 +1381,15 @@ int msm_run_table(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArg
                                              carry_key);
   CSK_CHECK_LAUNCH();
   for (uint64_t step = 1; step < pl.max_chunks; step *= 8)
-    k_carry_round<F><<<ga, TB, 0, st>>>(offsets, Ktot, pl.L, cr29, carry_key, (uint32_t)step);
+    k_carry_round<F><<<(uint32_t)((pl.max_chunks + 63) / 64), 256, 0, st>>>(offsets, Ktot, pl.L, cr29, carry_key,
+                                                                             (uint32_t)step);
   CSK_CHECK_LAUNCH();
   k_fixup<F><<<(Ktot + TB - 1) / TB, TB, 0, st>>>(offsets, Ktot, pl.L, b29, cr29);
   k_merge_members<F><<<dim3((pl.B + TB - 1) / TB, count), TB, 0, st>>>(offsets, b29, Wt, pl.B, merged);
   k_iota<<<(uint32_t)(((uint64_t)count * pl.B + 1 + 255) / 256), 256, 0, st>>>(iota, count * pl.B + 1);
   CSK_CHECK_LAUNCH();
-  k_bucket_reduce<F><<<(count * Sm + TB - 1) / TB, TB, 0, st>>>(iota, merged, count, pl.B, Lrm, partial);
-  window_sums<F>(partial, count, Sm, merged, wsum, st);  // the merged buckets are free again
-  k_final<F><<<count, FinalThreads<F>::N, 0, st>>>(osegs, wsum, 1, pl.c);
+  window_sums<F>(iota, merged, count, pl.B, Lrm, wsum, st);
+  k_final<F><<<count, RowAcc<F>::N, 0, st>>>(osegs, wsum, 1, pl.c);
   CSK_CHECK_LAUNCH();
   return CSK_OK;
 }

@@ -49,3 +49,19 @@ def test_sparse_windows(g2):
     pts = np.stack([gen_mul(x, g2) for x in ss])
     got = msm_host(inputs.from_ints(ks), pts, g2=g2, window_bits=7)
     assert np.array_equal(got, gen_mul(sum(a * b for a, b in zip(ks, ss)) % P.RR, g2))
+
+
+@pytest.mark.parametrize("g2", [False, True])
+@pytest.mark.parametrize("c", [2, 3, 6, 10, 13, 17])
+@pytest.mark.parametrize("reduce_seg", [0, 1, 2, 32])
+def test_reduction_shapes(g2, c, reduce_seg):
+    # one to three joining passes, windows down to two buckets, segments that
+    # are most of a window; equal points put equal sums in neighbouring nodes
+    n = 90
+    ks = inputs.field_elements(40, n)
+    ks[:30] = ks[0]
+    exps = [1 + (i % 7) for i in range(n)]
+    base = {e: gen_mul(e, g2) for e in set(exps)}
+    pts = np.stack([base[e] for e in exps])
+    want = gen_mul(sum(k * e for k, e in zip(inputs.to_ints(ks), exps)) % P.RR, g2)
+    assert np.array_equal(msm_host(ks, pts, g2=g2, window_bits=c, reduce_seg=min(reduce_seg, 1 << (c - 1))), want)
