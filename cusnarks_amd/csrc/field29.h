@@ -147,6 +147,46 @@ __device__ __forceinline__ void mul29x2(const Fq29 &a, const Fq29 &b, const Fq29
   cd.l[8] = (uint32_t)acd;
 }
 
+// mul29x2 plus an unreduced number in each result: ab = redc(a b) + s, cd =
+// redc(c d) + t.  s and t may have limbs up to 2^32; they join the columns
+// above the reduced ones (a multiply-add by 1 each), so a sum or difference
+// that follows a product costs no carry pass of its own.  The top limbs may
+// be taken modulo 2^32 (a difference whose top limb borrows).
+__device__ __forceinline__ void mul29x2_add(const Fq29 &a, const Fq29 &b, const Fq29 &s, const Fq29 &c,
+                                            const Fq29 &d, const Fq29 &t, Fq29 &ab, Fq29 &cd) {
+  uint32_t m[9], n[9], one = 1;
+  asm("" : "+s"(one));  // opaque, so the additions stay single multiply-adds
+  uint64_t acc = 0, acd = 0;
+#pragma unroll
+  for (int k = 0; k < 17; k++) {
+#pragma unroll
+    for (int j = (k > 8 ? k - 8 : 0); j <= (k < 8 ? k : 8); j++) {
+      mad29(acc, a.l[j], b.l[k - j]);
+      mad29(acd, c.l[j], d.l[k - j]);
+    }
+#pragma unroll
+    for (int j = (k > 8 ? k - 8 : 0); j < (k < 9 ? k : 9); j++) {
+      mad29(acc, m[j], Q29::p[k - j]);
+      mad29(acd, n[j], Q29::p[k - j]);
+    }
+    if (k < 9) {
+      m[k] = ((uint32_t)acc * Q29::np) & Q29::M;
+      n[k] = ((uint32_t)acd * Q29::np) & Q29::M;
+      mad29(acc, m[k], Q29::p[0]);
+      mad29(acd, n[k], Q29::p[0]);
+    } else {
+      mad29(acc, s.l[k - 9], one);
+      mad29(acd, t.l[k - 9], one);
+      ab.l[k - 9] = (uint32_t)acc & Q29::M;
+      cd.l[k - 9] = (uint32_t)acd & Q29::M;
+    }
+    acc >>= 29;
+    acd >>= 29;
+  }
+  ab.l[8] = (uint32_t)acc + s.l[8];
+  cd.l[8] = (uint32_t)acd + t.l[8];
+}
+
 // One product whose a*b and reduction products run on two chains, merged once
 // per column: for code with a single product to form at a time.
 __device__ __forceinline__ Fq29 mul29_2c(const Fq29 &a, const Fq29 &b) {
@@ -265,6 +305,52 @@ template <int K> __device__ __forceinline__ Fq29 sub29(const Fq29 &a, const Fq29
   return r;
 }
 
+// a + K*q - b without the carry pass: limbs below 1.5 * 2^30 for normalised a
+// and b.  As an operand of a product its top limb must not borrow: b below
+// (K - 0.001) q.
+template <int K> __device__ __forceinline__ Fq29 sub29_loose(const Fq29 &a, const Fq29 &b) {
+  Fq29 r;
+#pragma unroll
+  for (int i = 0; i < 9; i++) r.l[i] = a.l[i] + (QMul<K>::d[i] - b.l[i]);
+  return r;
+}
+template <int K> __device__ __forceinline__ Fq29 neg29_loose(const Fq29 &b) {
+  Fq29 r;
+#pragma unroll
+  for (int i = 0; i < 9; i++) r.l[i] = QMul<K>::d[i] - b.l[i];
+  return r;
+}
+// carries of limbs below 2^32
+__device__ __forceinline__ Fq29 norm29(const Fq29 &a) {
+  Fq29 r;
+  uint32_t c = 0;
+#pragma unroll
+  for (int i = 0; i < 9; i++) {
+    const uint32_t t = a.l[i] + c;
+    r.l[i] = i < 8 ? (t & Q29::M) : t;
+    c = t >> 29;
+  }
+  return r;
+}
+// a + K q - b - 2c for b + 2c below K q, normalised: K q with its low limbs
+// raised by 3 * 2^29, so one pass serves both differences
+template <int K> struct QMul3;
+template <> struct QMul3<6> {
+  static constexpr uint32_t d[9] = {1928196010u, 1712997445u, 1789907927u, 1895747810u, 1629690061u,
+                                    1898153089u, 1676232579u, 1982391605u, 19028435u};
+};
+template <int K> __device__ __forceinline__ Fq29 sub3_29(const Fq29 &a, const Fq29 &b, const Fq29 &c) {
+  Fq29 r;
+  uint32_t cy = 0;
+#pragma unroll
+  for (int i = 0; i < 9; i++) {
+    const uint32_t t = a.l[i] + (QMul3<K>::d[i] - b.l[i]) - 2 * c.l[i] + cy;
+    r.l[i] = i < 8 ? (t & Q29::M) : t;
+    cy = t >> 29;
+  }
+  return r;
+}
+
 // a + k*b, normalised (k = 1 or 2)
 template <int k> __device__ __forceinline__ Fq29 add29(const Fq29 &a, const Fq29 &b) {
   Fq29 r;
@@ -291,6 +377,29 @@ __device__ __forceinline__ bool is_zero29(const Fq29 &a) {
     e |= a.l[i] ^ Q29::p[i];
   }
   return z == 0 || e == 0;
+}
+
+// the same, by the low limb alone unless that agrees (rarely): for the tests of
+// the bucket loops, which all but never hold.  UPTO: the value is below
+// (UPTO + 1) q.
+template <int UPTO> __device__ __forceinline__ bool is_multiple29(const Fq29 &a) {
+  bool may = false;
+#pragma unroll
+  for (int k = 0; k <= UPTO; k++) may |= a.l[0] == ((k * Q29::p[0]) & Q29::M);
+  if (!may) return false;
+  bool is = false;
+#pragma unroll
+  for (int k = 0; k <= UPTO; k++) {
+    uint32_t e = 0, c = 0;
+#pragma unroll
+    for (int i = 0; i < 9; i++) {
+      const uint32_t t = k * Q29::p[i] + c;
+      e |= a.l[i] ^ (i < 8 ? (t & Q29::M) : t);
+      c = t >> 29;
+    }
+    is |= e == 0;
+  }
+  return is;
 }
 
 // a - m when a >= m (normalised a, m a normalised constant)
@@ -354,7 +463,7 @@ struct XYZZ29 {
   Fq29 X, Y, ZZ, ZZZ;
 };
 
-// 2*q for affine q (x < q, y <= q), mdbl-2008-s-1 with ranges as madd29's
+// 2*q for affine q (x < q, y < 2q), mdbl-2008-s-1 with ranges as madd29's
 // output: X3 < 6q, Y3, ZZ, ZZZ < 2q.
 __device__ __forceinline__ XYZZ29 dbl29_affine(const Fq29 &x, const Fq29 &y) {
   const Fq29 U = add29<1>(y, y);
@@ -367,8 +476,11 @@ __device__ __forceinline__ XYZZ29 dbl29_affine(const Fq29 &x, const Fq29 &y) {
   return {X3, Y3, V, W};
 }
 
-// acc += q for affine q (x < q, y <= q), madd-2008-s.  acc ranges on entry
-// and exit: X < 8q, Y, ZZ, ZZZ < 2q (bias multiples chosen from them).
+// acc += q for affine q (x < q; y < 2q with limbs below 2^30), madd-2008-s.  acc
+// ranges on entry and exit: X < 8q, Y, ZZ, ZZZ < 2q, normalised (bias multiples
+// chosen from them).  A product of values whose product is below c q^2 is below
+// (c / 170 + 1) q: RR, PPP and Qv are below 1.1q, so X3 is below 7.1q and the
+// loose differences below do not borrow from their top limbs.
 // The caller tracks infinity in ainf (true exactly when acc is infinity,
 // which then also has ZZ == 0): a run starts at infinity and returns there
 // only by cancellation.  Updated in place, one coordinate at a time, so the
@@ -376,20 +488,19 @@ __device__ __forceinline__ XYZZ29 dbl29_affine(const Fq29 &x, const Fq29 &y) {
 __device__ __forceinline__ void madd29(XYZZ29 &acc, bool &ainf, const Fq29 &x, const Fq29 &y) {
   if (ainf) {
     acc.X = x;
-    acc.Y = y;
+    acc.Y = norm29(y);
     acc.ZZ = f29_const(Q29::one);
     acc.ZZZ = f29_const(Q29::one);
     ainf = false;
     return;
   }
-  Fq29 U2, S2, PP, RR, PPP, Qv, ZZ3, ZZZ3;
-  mul29x2(x, acc.ZZ, y, acc.ZZZ, U2, S2);
-  const Fq29 P = sub29<8>(U2, acc.X);  // < 10q
-  const Fq29 R = sub29<2>(S2, acc.Y);  // < 4q
+  Fq29 P, R, PP, RR, PPP, Qv, ZZ3, ZZZ3;
+  // P = x ZZ - X < 10q, R = y ZZZ - Y < 4q
+  mul29x2_add(x, acc.ZZ, neg29_loose<8>(acc.X), y, acc.ZZZ, neg29_loose<2>(acc.Y), P, R);
   sqr29x2(P, R, PP, RR);
-  if (is_zero29(PP)) {
-    if (is_zero29(RR)) {
-      const XYZZ29 d = dbl29_affine(x, y);
+  if (is_multiple29<1>(PP)) {
+    if (is_multiple29<1>(RR)) {
+      const XYZZ29 d = dbl29_affine(x, norm29(y));
       acc.X = d.X;
       acc.Y = d.Y;
       acc.ZZ = d.ZZ;
@@ -405,9 +516,10 @@ __device__ __forceinline__ void madd29(XYZZ29 &acc, bool &ainf, const Fq29 &x, c
   mul29x2(acc.ZZ, PP, acc.ZZZ, PPP, ZZ3, ZZZ3);
   acc.ZZ = ZZ3;
   acc.ZZZ = ZZZ3;
-  const Fq29 X3 = sub29<6>(RR, add29<2>(PPP, Qv));  // PPP + 2Qv < 6q; X3 < 8q
-  // Y3 = R (Qv - X3) - Y PPP, one reduction of R T + Y (2q - PPP) < 44 q^2
-  acc.Y = dot29(R, sub29<8>(Qv, X3), acc.Y, sub29<2>(Fq29{}, PPP));
+  const Fq29 X3 = sub3_29<6>(RR, PPP, Qv);
+  // Y3 = R (Qv - X3) - Y PPP, one reduction of R T + Y (2q - PPP) < 44 q^2;
+  // columns below (13.5 + 9 + 4.5) 2^59
+  acc.Y = dot29(R, sub29_loose<8>(Qv, X3), acc.Y, neg29_loose<2>(PPP));
   acc.X = X3;
 }
 
