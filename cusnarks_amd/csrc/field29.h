@@ -288,6 +288,37 @@ __device__ __forceinline__ Fq29 dot29(const Fq29 &a, const Fq29 &b, const Fq29 &
   return r;
 }
 
+// redc(a0 b0 + a1 b1 + a2 b2 + a3 b3) on two chains
+__device__ __forceinline__ Fq29 dot4_29(const Fq29 &a0, const Fq29 &b0, const Fq29 &a1, const Fq29 &b1,
+                                        const Fq29 &a2, const Fq29 &b2, const Fq29 &a3, const Fq29 &b3) {
+  uint32_t m[9];
+  Fq29 r;
+  uint64_t acc = 0;
+#pragma unroll
+  for (int k = 0; k < 17; k++) {
+    uint64_t u = 0;
+#pragma unroll
+    for (int j = (k > 8 ? k - 8 : 0); j <= (k < 8 ? k : 8); j++) {
+      mad29(u, a0.l[j], b0.l[k - j]);
+      mad29(acc, a2.l[j], b2.l[k - j]);
+      mad29(u, a1.l[j], b1.l[k - j]);
+      mad29(acc, a3.l[j], b3.l[k - j]);
+    }
+#pragma unroll
+    for (int j = (k > 8 ? k - 8 : 0); j < (k < 9 ? k : 9); j++) mad29(acc, m[j], Q29::p[k - j]);
+    acc += u;
+    if (k < 9) {
+      m[k] = ((uint32_t)acc * Q29::np) & Q29::M;
+      mad29(acc, m[k], Q29::p[0]);
+    } else {
+      r.l[k - 9] = (uint32_t)acc & Q29::M;
+    }
+    acc >>= 29;
+  }
+  r.l[8] = (uint32_t)acc;
+  return r;
+}
+
 // a + K*q - b, normalised.  b's value at most K*q, its low limbs normalised.
 template <int K> __device__ __forceinline__ Fq29 sub29(const Fq29 &a, const Fq29 &b) {
   Fq29 r;

@@ -819,15 +819,17 @@ __device__ __forceinline__ void load29(const uint32_t *s, XYZZ2_29 &a) {
   load4x29(s, a.X.c0, a.X.c1, a.Y.c0, a.Y.c1);
   load4x29(s + 36, a.ZZ.c0, a.ZZ.c1, a.ZZZ.c0, a.ZZZ.c1);
 }
+// 256-thread workgroups of `count` groups of lanes
+template <class F> static uint32_t grp_blocks(uint64_t count) {
+  return (uint32_t)((count * Grp<F>::N + 255) / 256);
+}
 template <class F> struct Acc29;
 template <> struct Acc29<Fq> {
   using T = XYZZ29;
-  using Q = Fq29;  // one lane's part in a quad
   __device__ __forceinline__ static T inf() { return inf29(); }
 };
 template <> struct Acc29<Fq2> {
   using T = XYZZ2_29;
-  using Q = Fq2_29;
   __device__ __forceinline__ static T inf() { return inf2_29(); }
 };
 
@@ -838,15 +840,15 @@ template <> struct Acc29<Fq2> {
 // step 8^r the slot at chain index i (i % 8^(r+1) == 0) adds the slots at
 // i + k*8^r, k = 1..7, that lie in the chain.  The slots read are never
 // written in the same round.  Slots are 29-bit (SW words).
-// A quad of lanes per slot (quad29.h): a round is a chain of up to seven
+// A group of lanes per slot (quad29.h): a round is a chain of up to seven
 // additions, and few slots of a round head one.
 template <class F>
 __global__ void __launch_bounds__(256) k_carry_round(const uint32_t *__restrict__ off, uint32_t K, uint32_t L,
                                                      uint32_t *__restrict__ carry,
                                                      const uint32_t *__restrict__ carry_key, uint32_t step) {
   constexpr int SW = Slot29<F>::SW;
-  using T = typename Acc29<F>::Q;
-  const uint64_t u = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 2;
+  constexpr uint32_t GN = Grp<F>::N;
+  const uint64_t u = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / GN;
   const uint32_t E = off[K];
   uint32_t i = 0, len = 0;
   if (u * L < E) {
@@ -859,17 +861,17 @@ __global__ void __launch_bounds__(256) k_carry_round(const uint32_t *__restrict_
   }
   const bool head = ((uint64_t)i & (8ull * step - 1)) == 0 && (uint64_t)i + step < len;
   if (!__any(head)) return;
-  T a = {};
-  if (head) quad_load(carry + u * SW, a);
+  Fq29 a = {};
+  if (head) grp_load<F>(carry + u * SW, a);
 #pragma unroll 1
   for (uint64_t k = 1; k < 8; k++) {
     const bool more = head && i + k * step < len;
     if (!__any(more)) break;
-    T b = {};  // infinity where the chain has ended
-    if (more) quad_load(carry + (u + k * step) * SW, b);
-    quad_add(a, b);
+    Fq29 b = {};  // infinity where the chain has ended
+    if (more) grp_load<F>(carry + (u + k * step) * SW, b);
+    grp_add<F>(a, b);
   }
-  if (head) quad_store(carry + u * SW, a);
+  if (head) grp_store<F>(carry + u * SW, a);
 }
 
 // One thread per bucket: add the (reduced) chain head at slot t0+1.
@@ -904,32 +906,32 @@ __global__ void __launch_bounds__(256) k_fixup(const uint32_t *__restrict__ off,
 // node's R becomes the new C, whose weight is the lower one's length.  So a
 // window of B buckets takes 2 B additions, about 2 Lr + log2(B / Lr) of them in
 // a row, and no doublings before the last step (k_window_horner), log2(B)
-// doublings and additions of C's on rows of lanes.  The additions run on quads
+// doublings and additions of C's on rows of lanes.  The additions run on groups
 // of lanes (quad29.h), as the chain is what costs.
 // Measured, 2^20 points (c = 16, 8 x 32768 buckets): 101 + 67 + 38 us; segments
 // each multiplied by their offset and summed by lanes, 256 + 118 us.
 
-// a quad per (window, segment)
+// a group per (window, segment)
 template <class F>
 __global__ void __launch_bounds__(256) k_bucket_reduce(const uint32_t *__restrict__ off, uint32_t *buckets,
                                                        uint32_t nseg, uint32_t Lr) {
   constexpr int SW = Slot29<F>::SW;
-  using T = typename Acc29<F>::Q;
-  const uint32_t seg = (uint32_t)(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 2);
+  constexpr uint32_t GN = Grp<F>::N;
+  const uint32_t seg = (uint32_t)(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / GN);
   const bool live = seg < nseg;
   const uint64_t lo = (uint64_t)seg * Lr;  // windows follow each other: key = w * B + s * Lr
-  T run = {}, acc = {};
+  Fq29 run = {}, acc = {};
 #pragma unroll 1
   for (int b = (int)Lr - 1; b >= 0; b--) {
-    T bk = {};
+    Fq29 bk = {};
     const uint64_t key = lo + (uint32_t)b;
-    if (live && off[key + 1] != off[key]) quad_load(buckets + key * SW, bk);
-    quad_add(run, bk);
-    quad_add(acc, run);
+    if (live && off[key + 1] != off[key]) grp_load<F>(buckets + key * SW, bk);
+    grp_add<F>(run, bk);
+    grp_add<F>(acc, run);
   }
   if (live) {
-    quad_store(buckets + lo * SW, run);
-    quad_store(buckets + (lo + 1) * SW, acc);
+    grp_store<F>(buckets + lo * SW, run);
+    grp_store<F>(buckets + (lo + 1) * SW, acc);
   }
 }
 
@@ -958,18 +960,18 @@ __global__ void __launch_bounds__(256) k_bucket_reduce_lanes(const uint32_t *__r
 }
 
 // Threads of the largest k_tree workgroup (the G2 addition takes more than the
-// 128 registers a wave of a 1024-thread workgroup has), and its LDS.
-template <class F> struct TreeDim { static constexpr uint32_t kThreads = std::is_same<F, Fq>::value ? 1024 : 512; };
+// 128 registers a lane of a 1024-thread workgroup has), and its LDS.
+template <class F> static constexpr uint32_t kTreeThreads = std::is_same<F, Fq>::value ? 1024 : 512;
 static constexpr uint32_t kTreeLds = 65536;
 
 // One workgroup joins n (a power of two) nodes of `span` slots and K points
-// each into one of n * span slots.  It has a quad for each of the (n / 2) K
+// each into one of n * span slots.  It has a group for each of the (n / 2) K
 // additions and n / 2 copies of its first level; later levels have fewer.
 template <class F>
-__global__ void __launch_bounds__(TreeDim<F>::kThreads) k_tree(uint32_t *slots, uint32_t span, uint32_t K,
+__global__ void __launch_bounds__(kTreeThreads<F>) k_tree(uint32_t *slots, uint32_t span, uint32_t K,
                                                                uint32_t n) {
   constexpr int SW = Slot29<F>::SW;
-  using T = typename Acc29<F>::Q;
+  constexpr uint32_t GN = Grp<F>::N;
   extern __shared__ uint32_t sh[];  // n * K slots: point k of node i at k * n + i
   uint32_t *base = slots + (uint64_t)blockIdx.x * n * span * SW;
   for (uint32_t w = threadIdx.x; w < n * K * SW; w += blockDim.x) {
@@ -977,22 +979,22 @@ __global__ void __launch_bounds__(TreeDim<F>::kThreads) k_tree(uint32_t *slots, 
     sh[(k * n + i) * SW + (r - k * SW)] = base[(uint64_t)i * span * SW + r];
   }
   __syncthreads();
-  const uint32_t quad = threadIdx.x >> 2;
+  const uint32_t grp = threadIdx.x / GN;
   for (uint32_t m = n; m > 1; m >>= 1, K++) {
     const uint32_t h = m >> 1;
     // point k of the new node i; the quads after the additions' copy the upper R
-    const uint32_t k = quad / h, i = quad - k * h;
-    T a = {}, b = {};
+    const uint32_t k = grp / h, i = grp - k * h;
+    Fq29 a = {}, b = {};
     const bool add = k < K, copy = k == K;
     if (add) {
-      quad_load(sh + (k * m + 2 * i) * SW, a);
-      quad_load(sh + (k * m + 2 * i + 1) * SW, b);
+      grp_load<F>(sh + (k * m + 2 * i) * SW, a);
+      grp_load<F>(sh + (k * m + 2 * i + 1) * SW, b);
     } else if (copy) {
-      quad_load(sh + (2 * i + 1) * SW, a);
+      grp_load<F>(sh + (2 * i + 1) * SW, a);
     }
-    if (__any(add)) quad_add(a, b);
+    if (__any(add)) grp_add<F>(a, b);
     __syncthreads();
-    if (add || copy) quad_store(sh + (k * h + i) * SW, a);
+    if (add || copy) grp_store<F>(sh + (k * h + i) * SW, a);
     __syncthreads();
   }
   for (uint32_t w = threadIdx.x; w < K * SW; w += blockDim.x) base[w] = sh[w];
@@ -1026,12 +1028,13 @@ void window_sums(const uint32_t *off, uint32_t *buckets, uint32_t nwin, uint32_t
   if ((uint64_t)nwin * B >= 1u << 20)
     k_bucket_reduce_lanes<F><<<(nseg + 255) / 256, 256, 0, st>>>(off, buckets, nseg, Lr);
   else
-    k_bucket_reduce<F><<<(nseg + 63) / 64, 256, 0, st>>>(off, buckets, nseg, Lr);
+    k_bucket_reduce<F><<<grp_blocks<F>(nseg), 256, 0, st>>>(off, buckets, nseg, Lr);
   uint32_t N = B / Lr, span = Lr, K = 2;
   while (N > 1) {
     uint32_t n = 2;
-    while (n < N && 4 * n * (K + 1) <= TreeDim<F>::kThreads && 2 * n * K * Slot29<F>::SW * 4 <= kTreeLds) n *= 2;
-    const uint32_t th = (2 * n * (K + 1) + 63) / 64 * 64;  // a quad per addition and copy of the first level
+    constexpr uint32_t GN = Grp<F>::N;
+    while (n < N && n * (K + 1) * GN <= kTreeThreads<F> && 2 * n * K * Slot29<F>::SW * 4 <= kTreeLds) n *= 2;
+    const uint32_t th = (n / 2 * (K + 1) * GN + 63) / 64 * 64;  // a group per addition and copy of the first level
     k_tree<F><<<nwin * (N / n), th, n * K * Slot29<F>::SW * 4, st>>>(buckets, span, K, n);
     for (uint32_t m = n; m > 1; m >>= 1) K++;
     span *= n;
@@ -1157,7 +1160,7 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
     if (tm) tm->mark(2, st);
     // chains can be at most max_chunks long
     for (uint64_t step = 1; step < pl.max_chunks; step *= 8)
-      k_carry_round<F><<<(uint32_t)((pl.max_chunks + 63) / 64), 256, 0, st>>>(offsets, Ktot, pl.L, cr29, carry_key,
+      k_carry_round<F><<<grp_blocks<F>(pl.max_chunks), 256, 0, st>>>(offsets, Ktot, pl.L, cr29, carry_key,
                                                                                (uint32_t)step);
     CSK_CHECK_LAUNCH();
     k_fixup<F><<<(Ktot + TB - 1) / TB, TB, 0, st>>>(offsets, Ktot, pl.L, b29, cr29);
@@ -1386,7 +1389,7 @@ int msm_run_table(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArg
                                              carry_key);
   CSK_CHECK_LAUNCH();
   for (uint64_t step = 1; step < pl.max_chunks; step *= 8)
-    k_carry_round<F><<<(uint32_t)((pl.max_chunks + 63) / 64), 256, 0, st>>>(offsets, Ktot, pl.L, cr29, carry_key,
+    k_carry_round<F><<<grp_blocks<F>(pl.max_chunks), 256, 0, st>>>(offsets, Ktot, pl.L, cr29, carry_key,
                                                                              (uint32_t)step);
   CSK_CHECK_LAUNCH();
   k_fixup<F><<<(Ktot + TB - 1) / TB, TB, 0, st>>>(offsets, Ktot, pl.L, b29, cr29);
