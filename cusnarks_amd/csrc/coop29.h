@@ -279,16 +279,23 @@ template <> struct Coop29<Fq2> {
 };
 
 // ------------------------------------------------------------ accumulators
-// A running point that a workgroup of RowAcc<F>::N threads holds, over stored
-// 29-bit slots (limbs below 2^29 + 4 allowed): G1 in one wave's registers, G2 in
-// LDS.  Infinity is tracked in a flag every lane holds.
+// A running point over stored 29-bit slots (limbs below 2^29 + 4 allowed): G1 in
+// the registers of one wave, G2 in LDS, held by a workgroup of four.  Infinity
+// is tracked in a flag every lane holds.
 template <class F> struct RowAcc;
 template <> struct RowAcc<Fq> {
-  static constexpr int N = 64, kLds = 1, SW = 36;
+  static constexpr int SW = 36;
   RowG1K k;
   RowG1 p;
   bool inf;
-  __device__ __forceinline__ RowAcc(uint32_t *, const uint32_t *slot) : p(row_load_g1(slot)) { inf = row_is_zero(p.ZZ); }
+  __device__ __forceinline__ void clear() {
+    p = {0, 0, 0, 0};
+    inf = true;
+  }
+  __device__ __forceinline__ void set(const uint32_t *slot) {
+    p = row_load_g1(slot);
+    inf = row_is_zero(p.ZZ);
+  }
   __device__ __forceinline__ void dbl(uint32_t n) {
     if (inf) return;
 #pragma unroll 1
@@ -305,7 +312,7 @@ template <> struct RowAcc<Fq> {
     }
   }
   __device__ __forceinline__ void store(uint32_t *slot) const {
-    const uint32_t l = threadIdx.x;
+    const uint32_t l = threadIdx.x & 63;
     if (l < 9) {
       slot[l] = p.X;
       slot[9 + l] = p.Y;
@@ -313,17 +320,19 @@ template <> struct RowAcc<Fq> {
       slot[27 + l] = inf ? 0u : p.ZZZ;
     }
   }
+  // canonical affine words, by one wave
   __device__ __forceinline__ void store_affine_to(uint32_t *out) const {
-    const Fq29 X = row_gather(p.X), Y = row_gather(p.Y), ZZ = row_gather(p.ZZ), ZZZ = row_gather(p.ZZZ);
-    if (threadIdx.x == 0) {
-      XYZZ<Fq> a;
-      from29_words(X, a.X.v);
-      from29_words(Y, a.Y.v);
-      from29_words(ZZ, a.ZZ.v);
-      from29_words(ZZZ, a.ZZZ.v);
-      if (inf) a = XYZZ<Fq>::inf();
-      store_affine(out, xyzz_to_affine(a));
+    const uint32_t l = threadIdx.x & 63;
+    uint32_t w[8];
+    if (inf) {
+      for (int i = 0; i < 8; i++) w[i] = l ? FieldConst<0>::one[i] : 0u;
+    } else {
+      const uint32_t t = row_inverse(k, row_mul(k, p.ZZ, p.ZZZ));
+      const uint32_t i = row_mul(k, t, k.odd ? p.ZZ : p.ZZZ);  // 1/ZZ | 1/ZZZ
+      const uint32_t v = row_mul(k, i, k.odd ? p.Y : p.X);
+      row_words(row_mul(k, v, kRowFrom[l & 15]), w);
     }
+    if (l == 0 || l == 16) st8(out + l / 2, w);
   }
 };
 
@@ -369,21 +378,34 @@ template <> struct RowAcc<Fq2> {
   __device__ __forceinline__ void store(uint32_t *slot) const {
     if (threadIdx.x < SW) slot[threadIdx.x] = inf && threadIdx.x >= SW / 2 ? 0u : sh[at(threadIdx.x)];
   }
+  // canonical affine words, by the first wave
   __device__ __forceinline__ void store_affine_to(uint32_t *out) const {
     if (threadIdx.x >= 64) return;
-    uint32_t wds[8 * C::NC];
-#pragma unroll
-    for (int k = 0; k < C::NC; k++) {
-      uint32_t o[8];
-      from29_words(row_gather(sh[16 * k + (threadIdx.x & 15)]), o);
-#pragma unroll
-      for (int i = 0; i < 8; i++) wds[8 * k + i] = o[i];
+    const uint32_t l = threadIdx.x, ln = l & 15;
+    uint32_t w[8];
+    if (inf) {
+      for (int i = 0; i < 8; i++) w[i] = l == 32 ? FieldConst<0>::one[i] : 0u;  // (0, 0, 1, 0)
+    } else {
+      const RowK &k = prog.rk;
+      const bool odd = (l >> 4) & 1, hi = (l >> 5) & 1;
+      auto v = [&](int i) { return sh[16 * i + ln]; };
+      auto neg = [&](uint32_t x) { return row_norm(kRowD[1][ln] - x); };  // 2q - x
+      // rows 2h, 2h + 1: the components of a_h b_h
+      auto mul2 = [&](uint32_t a00, uint32_t a01, uint32_t b00, uint32_t b01, uint32_t a10, uint32_t a11,
+                      uint32_t b10, uint32_t b11) {
+        const uint32_t a0 = hi ? a10 : a00, a1 = hi ? a11 : a01, b0 = hi ? b10 : b00, b1 = hi ? b11 : b01;
+        return row_dot(k, a0, odd ? b1 : b0, a1, odd ? b0 : neg(b1));
+      };
+      const uint32_t zz0 = v(H_ZZ0), zz1 = v(H_ZZ1), z30 = v(H_ZZZ0), z31 = v(H_ZZZ1);
+      uint32_t t0, t1, u0, u1, a0, a1, b0, b1;
+      row_spread2(mul2(zz0, zz1, z30, z31, zz0, zz1, z30, z31), t0, t1);  // ZZ ZZZ
+      const uint32_t n = row_inverse(k, row_dot(k, t0, t0, t1, t1));       // its inverse: (t0 - t1 u) / (t0^2 + t1^2)
+      row_spread2(row_mul(k, odd ? neg(t1) : t0, n), u0, u1);
+      row_spread4(mul2(u0, u1, z30, z31, u0, u1, zz0, zz1), a0, a1, b0, b1);  // 1/ZZ, 1/ZZZ
+      const uint32_t r = mul2(v(H_X0), v(H_X1), a0, a1, v(H_Y0), v(H_Y1), b0, b1);
+      row_words(row_mul(k, r, kRowFrom[ln]), w);
     }
-    if (threadIdx.x == 0) {
-      XYZZ<Fq2> acc = load_xyzz<Fq2>(wds);
-      if (inf) acc = XYZZ<Fq2>::inf();
-      store_affine(out, xyzz_to_affine(acc));
-    }
+    if (ln == 0) st8(out + l / 2, w);
   }
 };
 

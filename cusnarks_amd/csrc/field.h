@@ -277,7 +277,7 @@ template <int PIDX> struct Fp {
       p.v[i] = C::p[i];
       r3.v[i] = C::r3[i];
     }
-    i30_inverse(a.v, p.v, C::np, r.v);
+    i30_inverse<false>(a.v, p.v, C::np, r.v);
     return mul(r, r3);
   }
 };

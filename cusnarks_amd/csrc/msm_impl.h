@@ -1000,22 +1000,73 @@ __global__ void __launch_bounds__(kTreeThreads<F>) k_tree(uint32_t *slots, uint3
   for (uint32_t w = threadIdx.x; w < K * SW; w += blockDim.x) base[w] = sh[w];
 }
 
+// sum_i 2^(step i) v_i over n stored slots, v_i at base + i * stride words, by a
+// workgroup of kChainThreads; the result is in sum (G1: of the first wave).
+// G1: each of the four waves takes a run of the values, then the runs join
+// pairwise: as many doublings in a row, fewer additions.  lds: kChainLds words.
+static constexpr uint32_t kChainThreads = 256;
+template <class F> static constexpr uint32_t kChainLds = std::is_same<F, Fq>::value ? 4 * 36 : 1;
+__device__ __forceinline__ void horner(RowAcc<Fq> &sum, uint32_t *lds, const uint32_t *base, uint32_t stride,
+                                       uint32_t n, uint32_t step) {
+  // runs of a, b, a and the rest, the last the longest: the waves wait for each
+  // other before a join, and with equal even runs no wait adds a doubling
+  const uint32_t a = n / 4, b = (n - 2 * a) / 2, wave = threadIdx.x / 64;
+  const uint32_t start[5] = {0, a, a + b, 2 * a + b, n};
+  const uint32_t lo = wave == 0 ? start[0] : wave == 1 ? start[1] : wave == 2 ? start[2] : start[3];
+  const uint32_t hi = wave == 0 ? start[1] : wave == 1 ? start[2] : wave == 2 ? start[3] : start[4];
+  sum.clear();
+#pragma unroll 1
+  for (uint32_t i = hi; i-- > lo;) {
+    sum.dbl(step);
+    sum.add(base + (uint64_t)i * stride);
+  }
+#pragma unroll 1
+  for (uint32_t d = 1; d < 4; d *= 2) {
+    sum.store(lds + wave * 36);
+    __syncthreads();
+    if (wave % (2 * d) == 0) {
+      sum.set(lds + (wave + d) * 36);
+      sum.dbl(step * (d == 1 ? a : a + b));
+      sum.add(lds + wave * 36);
+    }
+    __syncthreads();
+  }
+}
+__device__ __forceinline__ void horner(RowAcc<Fq2> &sum, uint32_t *, const uint32_t *base, uint32_t stride,
+                                       uint32_t n, uint32_t step) {
+#pragma unroll 1
+  for (uint32_t i = n - 1; i-- > 0;) {  // sum starts as the last value
+    sum.dbl(step);
+    sum.add(base + (uint64_t)i * stride);
+  }
+}
+
 // A + Lr (C_0 + 2 C_1 + ...) of each window's last node (one workgroup per
 // window), a 29-bit slot of limbs below 2^29 + 4
 template <class F>
-__global__ void __launch_bounds__(RowAcc<F>::N) k_window_horner(const uint32_t *__restrict__ slots, uint32_t B,
-                                                                uint32_t K, uint32_t lgLr,
-                                                                uint32_t *__restrict__ wsum) {
-  __shared__ uint32_t lds[RowAcc<F>::kLds];
+__global__ void __launch_bounds__(kChainThreads) k_window_horner(const uint32_t *__restrict__ slots, uint32_t B,
+                                                                 uint32_t K, uint32_t lgLr,
+                                                                 uint32_t *__restrict__ wsum) {
   constexpr int SW = Slot29<F>::SW;
   const uint32_t *node = slots + (uint64_t)blockIdx.x * B * SW;
-  RowAcc<F> acc(lds, node + (uint64_t)(K - 1) * SW);
-#pragma unroll 1
-  for (int k = (int)K - 2; k >= 1; k--) {
-    acc.dbl(k == 1 ? lgLr : 1);
-    acc.add(node + (uint64_t)k * SW);
+  if constexpr (std::is_same<F, Fq>::value) {
+    __shared__ uint32_t lds[kChainLds<F>];
+    RowAcc<F> acc;
+    horner(acc, lds, node + 2 * SW, SW, K - 2, 1);
+    if (threadIdx.x >= 64) return;
+    acc.dbl(lgLr);
+    acc.add(node + SW);
+    acc.store(wsum + (uint64_t)blockIdx.x * SW);
+  } else {
+    __shared__ uint32_t lds[RowAcc<F>::kLds];
+    RowAcc<F> acc(lds, node + (uint64_t)(K - 1) * SW);
+    if (K > 2) {
+      horner(acc, lds, node + 2 * SW, SW, K - 2, 1);
+      acc.dbl(lgLr);
+      acc.add(node + SW);
+    }
+    acc.store(wsum + (uint64_t)blockIdx.x * SW);
   }
-  acc.store(wsum + (uint64_t)blockIdx.x * SW);
 }
 
 template <class F>
@@ -1040,38 +1091,40 @@ void window_sums(const uint32_t *off, uint32_t *buckets, uint32_t nwin, uint32_t
     span *= n;
     N /= n;
   }
-  k_window_horner<F><<<nwin, RowAcc<F>::N, 0, st>>>(buckets, B, K, 31 - __builtin_clz(Lr), wsum);
+  k_window_horner<F><<<nwin, kChainThreads, 0, st>>>(buckets, B, K, 31 - __builtin_clz(Lr), wsum);
 }
 
 // One workgroup per member: Horner over its W window sums (c doublings each),
 // written as a canonical affine point to the member's output.  The chain is
 // serial and latency bound, so each product is spread over a row of lanes and
-// the products of a step run on different rows (row29.h): G1 in one wave that
-// holds the point in registers, G2 in four waves that hold every value in LDS
-// (coop29.h).  Infinity is tracked in a flag every lane holds.
-// Measured at 248 doublings and 31 additions (c = 8): G1 333 us, 855 with one
-// lane per product; G2 638 us, 1997 with one lane per product.  One window
-// (table runs: the inversion and the conversions): 50 us, 167 with a binary
-// Euclid.
+// the products of a step run on different rows (row29.h): G1 in waves that
+// hold a point in registers each and take a part of the windows, G2 in four
+// waves that hold every value in LDS (coop29.h).  Infinity is tracked in a flag every lane holds.
+// Measured: 120 doublings 174 us on G1, 273 on G2 (whole scalars' 248 doublings
+// with one lane per product: 855 and 1997 us).  One window (table runs: the
+// inversion and the conversions): 33 us, 167 with a binary Euclid on one lane.
 template <class F>
-__global__ void __launch_bounds__(RowAcc<F>::N) k_final(const MsmSeg *__restrict__ segs,
-                                                        const uint32_t *__restrict__ wsum, uint32_t W, uint32_t c) {
+__global__ void __launch_bounds__(kChainThreads) k_final(const MsmSeg *__restrict__ segs,
+                                                         const uint32_t *__restrict__ wsum, uint32_t W, uint32_t c) {
   const uint32_t j = blockIdx.x;
   uint32_t *out = segs[j].out;
   if (segs[j].n == 0) {
     if (threadIdx.x == 0) store_affine(out, Affine<F>{F::zero(), F::one()});
     return;
   }
-  __shared__ uint32_t lds[RowAcc<F>::kLds];
   constexpr int SW = Slot29<F>::SW;
   const uint32_t *ws = wsum + (uint64_t)j * W * SW;
-  RowAcc<F> acc(lds, ws + (uint64_t)(W - 1) * SW);
-#pragma unroll 1
-  for (int w = (int)W - 2; w >= 0; w--) {
-    acc.dbl(c);
-    acc.add(ws + (uint64_t)w * SW);
+  if constexpr (std::is_same<F, Fq>::value) {
+    __shared__ uint32_t lds[kChainLds<F>];
+    RowAcc<F> acc;
+    horner(acc, lds, ws, SW, W, c);
+    if (threadIdx.x < 64) acc.store_affine_to(out);
+  } else {
+    __shared__ uint32_t lds[RowAcc<F>::kLds];
+    RowAcc<F> acc(lds, ws + (uint64_t)(W - 1) * SW);
+    horner(acc, lds, ws, SW, W, c);
+    acc.store_affine_to(out);
   }
-  acc.store_affine_to(out);
 }
 
 // The sort's placement passes over the counted and scanned digits: pass 1
@@ -1168,7 +1221,7 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
     window_sums<F>(offsets, b29, Wtot, pl.B, pl.Lr, wsum, st);
     CSK_CHECK_LAUNCH();
   }
-  k_final<F><<<pl.J, RowAcc<F>::N, 0, st>>>(segs, wsum, pl.W, pl.c);
+  k_final<F><<<pl.J, kChainThreads, 0, st>>>(segs, wsum, pl.W, pl.c);
   CSK_CHECK_LAUNCH();
   if (tm) tm->mark(3, st);
   return CSK_OK;
@@ -1397,7 +1450,7 @@ int msm_run_table(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArg
   k_iota<<<(uint32_t)(((uint64_t)count * pl.B + 1 + 255) / 256), 256, 0, st>>>(iota, count * pl.B + 1);
   CSK_CHECK_LAUNCH();
   window_sums<F>(iota, merged, count, pl.B, Lrm, wsum, st);
-  k_final<F><<<count, RowAcc<F>::N, 0, st>>>(osegs, wsum, 1, pl.c);
+  k_final<F><<<count, kChainThreads, 0, st>>>(osegs, wsum, 1, pl.c);
   CSK_CHECK_LAUNCH();
   return CSK_OK;
 }

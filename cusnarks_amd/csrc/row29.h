@@ -22,6 +22,7 @@
 // of values whose sum s is below 169 q^2 give a value below 2q.  Column sums
 // stay below 2^64 (4 * 9 * (2^29 + 4)^2 + 9 * 2^29 (2^29 + 2)).
 #pragma once
+#include "field.h"
 #include "field29.h"
 
 namespace csk {
@@ -46,6 +47,13 @@ __constant__ uint32_t kRowD[6][16] = {
      25371249u},
     {1424090310u, 1244383009u, 1551524116u, 1548966950u, 1463451310u, 1552975748u, 1183108232u, 1335459334u,
      31714062u}};
+
+// 2^783 mod q (2^261 cubed: from the inverse of a 2^261-form number to the
+// 2^261 form of the inverse) and 2^256 mod q (to the 2^256 form)
+__constant__ uint32_t kRowR3[16] = {237179570u, 381705378u, 197673865u, 484389131u, 296595421u,
+                                    53368462u,  493544588u, 282381599u, 2540242u};
+__constant__ uint32_t kRowFrom[16] = {93261213u,  451550318u, 297979764u, 299258347u, 342016167u,
+                                      297253948u, 482187706u, 406012155u, 920183u};
 
 // lane moves within the row; lanes without a source take 0
 template <int N> __device__ __forceinline__ uint32_t row_bcast(uint32_t x) {
@@ -158,11 +166,31 @@ __device__ __forceinline__ bool row_is_zero(uint32_t x) {
   return (z & 0xFFFF) == 0xFFFF || (q & 0xFFFF) == 0xFFFF;
 }
 
-// row 0's (every row's) element gathered into each lane, exact limbs
+// each row's element gathered into its lanes, exact limbs
 __device__ __forceinline__ Fq29 row_gather(uint32_t x) {
   x = row_exact(x);
   return {{row_bcast<0>(x), row_bcast<1>(x), row_bcast<2>(x), row_bcast<3>(x), row_bcast<4>(x), row_bcast<5>(x),
            row_bcast<6>(x), row_bcast<7>(x), row_bcast<8>(x)}};
+}
+
+// an element held by every lane to the rows
+__device__ __forceinline__ uint32_t row_scatter(const Fq29 &a) {
+  const uint32_t k = threadIdx.x & 15;
+  uint32_t r = 0;
+#pragma unroll
+  for (int i = 0; i < 9; i++) r = k == (uint32_t)i ? a.l[i] : r;
+  return r;
+}
+// canonical words of each row's element (below 2q)
+__device__ __forceinline__ void row_words(uint32_t x, uint32_t (&w)[8]) { pack29(canon29(row_gather(x)), w); }
+// the inverse of an element every row holds (2^261 form, below 2q, not 0)
+__device__ __forceinline__ uint32_t row_inverse(const RowK &k, uint32_t x) {
+  uint32_t w[8], p[8], o[8];
+  row_words(x, w);
+#pragma unroll
+  for (int i = 0; i < 8; i++) p[i] = FieldConst<0>::p[i];
+  i30_inverse<true>(w, p, FieldConst<0>::np, o);
+  return row_mul(k, row_scatter(unpack29(o)), kRowR3[threadIdx.x & 15]);
 }
 
 // rows 0, 2 hold one value and rows 1, 3 another: both in every row
