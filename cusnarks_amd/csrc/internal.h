@@ -71,6 +71,7 @@ struct MsmPlan {
   uint32_t Lr;           // buckets per reduction thread
   uint32_t S;            // reduction segments per window, B / Lr
   uint64_t n;            // points over all members, E for each of the caller's
+  uint64_t most;         // points of the largest member
   uint64_t max_entries;  // n * W (upper bound on nonzero digits)
   uint64_t max_chunks;   // ceil(max_entries / L)
   uint64_t tiles;        // sum over members of ceil(n_j / 4096) (sort tiles per window)

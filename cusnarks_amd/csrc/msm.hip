@@ -93,6 +93,7 @@ MsmPlan msm_group_plan(uint32_t c, uint32_t E, const uint64_t *n, uint32_t J, bo
   pl.J = J;
   for (uint32_t j = 0; j < J; j++) {
     pl.n += E * n[j];
+    if (E * n[j] > pl.most) pl.most = E * n[j];
     pl.tiles += (E * n[j] + kSortTile - 1) / kSortTile;
   }
   pl.max_entries = pl.n * pl.W;
@@ -373,6 +374,7 @@ static MsmPlan table_plan(uint32_t c, uint64_t n_pad, uint32_t Wt, uint32_t coun
   pl.K = pl.B;
   pl.J = Wt * count;
   pl.n = n_pad * pl.J;
+  pl.most = n_pad;
   pl.tiles = pl.J * (n_pad / kSortTile);
   pl.max_entries = pl.n;
   pl.hb = plan_hi_bits(c, n_pad);
@@ -430,6 +432,7 @@ static int table_run(csk_ctx *ctx, uint32_t count, csk_msm_table *const *t, cons
     }
     const uint32_t nt = (uint32_t)(t[p]->n_pad / kSortTile);
     pl.n += (uint64_t)Wt * t[p]->n_pad;
+    if (t[p]->n_pad > pl.most) pl.most = t[p]->n_pad;
     pl.tiles += (uint64_t)Wt * nt;
     if (nt > max_nt) max_nt = nt;
   }

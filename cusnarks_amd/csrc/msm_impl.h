@@ -2,6 +2,7 @@
 // pipeline overview).  Included by msm_g1.hip and msm_g2.hip so that the two
 // curves compile as separate translation units.
 #pragma once
+#include <algorithm>
 #include <type_traits>
 #include "internal.h"
 #include "curve.h"
@@ -282,14 +283,61 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_final(const uint32_t *in,
   }
 }
 
-// exclusive scan of arr[0..len) in LDS by one workgroup of SORT_THREADS;
-// tmp holds SORT_THREADS / 64 words (one per wave); returns the total (all threads)
+// The whole scan by one workgroup, in place, for K <= SCAN_SMALL: three launches
+// cost more than one workgroup's walk (12800 counters: 14 us against 9).
+static constexpr uint32_t SCAN_SMALL = 16384;
+__global__ void __launch_bounds__(1024) k_scan_small(uint32_t *arr, uint32_t K) {
+  __shared__ uint32_t wsum[16];
+  const uint32_t per = (K + 1023) / 1024, lo = threadIdx.x * per;
+  uint32_t v[SCAN_SMALL / 1024], s = 0;
+#pragma unroll
+  for (uint32_t j = 0; j < SCAN_SMALL / 1024; j++) {
+    v[j] = j < per && lo + j < K ? arr[lo + j] : 0u;
+    s += v[j];
+  }
+  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  uint32_t x = s;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(x, o, 64);
+    if (lane >= (uint32_t)o) x += y;
+  }
+  if (lane == 63) wsum[wv] = x;
+  __syncthreads();
+  uint32_t run = x - s, total = 0;
+  for (uint32_t k = 0; k < 16; k++) {
+    run += k < wv ? wsum[k] : 0u;
+    total += wsum[k];
+  }
+#pragma unroll
+  for (uint32_t j = 0; j < SCAN_SMALL / 1024; j++) {
+    if (j < per && lo + j < K) arr[lo + j] = run;
+    run += v[j];
+  }
+  if (threadIdx.x == 0) arr[K] = total;
+}
+
+// exclusive prefix sums of cnt[0..K) in place, cnt[K] = total; bsum: a word per
+// SCAN_TILE counters
+static inline void scan_counts(uint32_t *cnt, uint32_t K, uint32_t *bsum, hipStream_t st) {
+  if (K <= SCAN_SMALL) {
+    k_scan_small<<<1, 1024, 0, st>>>(cnt, K);
+    return;
+  }
+  const uint32_t nb = (K + SCAN_TILE - 1) / SCAN_TILE;
+  k_scan_reduce<<<nb, SCAN_THREADS, 0, st>>>(cnt, K, bsum);
+  k_scan_blocks<<<1, 1024, 0, st>>>(bsum, nb);
+  k_scan_final<<<nb, SCAN_THREADS, 0, st>>>(cnt, K, bsum, cnt);
+}
+
 static constexpr int SORT_THREADS = 256;
 static constexpr int SORT_TILE = 4096;  // digits of one window per pass-1 workgroup
 static constexpr int SORT_IPT = SORT_TILE / SORT_THREADS;
 
+// exclusive scan of arr[0..len) in LDS by one workgroup of THREADS; tmp holds
+// THREADS / 64 words (one per wave); returns the total (all threads)
+template <int THREADS>
 __device__ uint32_t block_exclusive_scan(uint32_t *arr, uint32_t len, uint32_t *tmp) {
-  const uint32_t per = (len + SORT_THREADS - 1) / SORT_THREADS;
+  const uint32_t per = (len + THREADS - 1) / THREADS;
   const uint32_t lo = threadIdx.x * per;
   uint32_t s = 0;
   for (uint32_t j = 0; j < per; j++)
@@ -304,7 +352,7 @@ __device__ uint32_t block_exclusive_scan(uint32_t *arr, uint32_t len, uint32_t *
   if (lane == 63) tmp[wv] = x;
   __syncthreads();
   uint32_t run = x - s, total = 0;
-  for (uint32_t k = 0; k < SORT_THREADS / 64; k++) {
+  for (uint32_t k = 0; k < THREADS / 64; k++) {
     const uint32_t t = tmp[k];
     run += k < wv ? t : 0;
     total += t;
@@ -404,7 +452,7 @@ __global__ void __launch_bounds__(SORT_THREADS) k_sort_scatter1(const uint32_t *
   __syncthreads();
   for (uint32_t i = threadIdx.x; i < HB; i += SORT_THREADS) base[i] = h[i];
   __syncthreads();
-  const uint32_t total = block_exclusive_scan(base, HB, scan_tmp);
+  const uint32_t total = block_exclusive_scan<SORT_THREADS>(base, HB, scan_tmp);
   // h (the counts are in base now) takes each bin's output start minus its
   // tile-local start; offsets are < 2^31, the u32 difference wraps back on +p
   for (uint32_t i = threadIdx.x; i < HB; i += SORT_THREADS) h[i] = goff[t.cb + i * t.NT] - base[i];
@@ -442,16 +490,36 @@ __global__ void __launch_bounds__(SORT_THREADS) k_sort_scatter1(const uint32_t *
 // gw*B + hi*2^ts + lo; its last segment also points the buckets it cannot
 // reach (from HB*2^ts on) at its end, and with ts = 0 pass 1 has placed its
 // entries already, so only the offsets are written.
-template <int TILE>
-__global__ void __launch_bounds__(SORT_THREADS) k_sort_pass2(const uint32_t *__restrict__ tix,
+// counter[key] += 1 for the live lanes, the count before this lane's: the lanes
+// that agree with the first one add once together.  For segments far above the
+// average, which hold a bucket of very many entries (the ones among wire
+// values): 64 additions to one counter take 64 turns.
+__device__ __forceinline__ uint32_t count_hot(uint32_t *counter, uint32_t key, bool live) {
+  const uint64_t act = __ballot(live);
+  if (act == 0) return 0;
+  const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)key, __builtin_ctzll(act));
+  const uint64_t same = __ballot(live && key == first);
+  const uint32_t lane = threadIdx.x & 63, lead = __builtin_ctzll(same);
+  uint32_t r = 0;
+  if (live && (key != first || lane == lead)) r = atomicAdd(&counter[key], key == first ? __popcll(same) : 1u);
+  const uint32_t base = (uint32_t)__builtin_amdgcn_readlane((int)r, lead);
+  return key == first ? base + __popcll(same & ((1ull << lane) - 1)) : r;
+}
+
+// Segments above `split` entries are left to a launch of their own (LONG), whose
+// workgroups have more threads: few segments are long (most of a window's
+// entries in one bin: wire values), so one workgroup's time is what they cost
+// (300007 scalars, half of them 0 or 1: 249 us without the split, 13 + 70 with).
+template <int TILE, int THREADS, bool LONG>
+__global__ void __launch_bounds__(THREADS) k_sort_pass2(const uint32_t *__restrict__ tix,
                                                              const uint16_t *__restrict__ tlo,
                                                              const uint32_t *__restrict__ goff,
                                                              const MsmSeg *__restrict__ segs, uint32_t HB,
                                                              uint32_t s, uint32_t ts, uint32_t W, uint32_t Wwin,
-                                                             uint32_t Ktot, uint32_t *__restrict__ offsets,
+                                                             uint32_t Ktot, uint32_t split, uint32_t *__restrict__ offsets,
                                                              uint32_t *__restrict__ sorted) {
   extern __shared__ uint32_t dyn[];  // 3 * 2^s words: counts, cursors, tile bases
-  __shared__ uint32_t scan_tmp[SORT_THREADS];
+  __shared__ uint32_t scan_tmp[THREADS / 64];
   __shared__ uint32_t stage[TILE];
   __shared__ uint16_t sbin[TILE];
   const uint32_t seg = blockIdx.x, per = W * HB, mj = seg / per, rem = seg - mj * per;
@@ -461,54 +529,60 @@ __global__ void __launch_bounds__(SORT_THREADS) k_sort_pass2(const uint32_t *__r
   const uint32_t L2 = 1u << s, key0 = gw * B + hi * L2;
   uint32_t *cntv = dyn, *cur = dyn + L2, *tb = dyn + 2 * L2;
   const uint32_t start = goff[cb + rem * NT], end = goff[cb + (rem + 1) * NT];
-  if (seg == gridDim.x - 1 && threadIdx.x == 0) offsets[Ktot] = end;
-  if (hi == HB - 1)
-    for (uint32_t k = key0 + L2 + threadIdx.x; k < (gw + 1) * B; k += SORT_THREADS) offsets[k] = end;
+  if (LONG && end - start <= split) return;
+  if (!LONG && seg == gridDim.x - 1 && threadIdx.x == 0) offsets[Ktot] = end;
+  if (!LONG && hi == HB - 1)
+    for (uint32_t k = key0 + L2 + threadIdx.x; k < (gw + 1) * B; k += THREADS) offsets[k] = end;
   if (s == 0) {
     if (threadIdx.x == 0) offsets[key0] = start;
     return;
   }
-  for (uint32_t i = threadIdx.x; i < L2; i += SORT_THREADS) cntv[i] = 0;
+  if (!LONG && end - start > split) return;
+  for (uint32_t i = threadIdx.x; i < L2; i += THREADS) cntv[i] = 0;
   __syncthreads();
   // eight unconditional (clamped) loads in flight per thread, then their counts
-  for (uint32_t e0 = start; e0 < end; e0 += 8 * SORT_THREADS) {
+  for (uint32_t e0 = start; e0 < end; e0 += 8 * THREADS) {
     uint32_t l[8];
     for (int k = 0; k < 8; k++) {
-      const uint32_t e = e0 + k * SORT_THREADS + threadIdx.x;
+      const uint32_t e = e0 + k * THREADS + threadIdx.x;
       l[k] = tlo[e < end ? e : end - 1];
     }
-    for (int k = 0; k < 8; k++)
-      if (e0 + k * SORT_THREADS + threadIdx.x < end) atomicAdd(&cntv[l[k]], 1u);
+    for (int k = 0; k < 8; k++) {
+      const bool live = e0 + k * THREADS + threadIdx.x < end;
+      if (LONG) count_hot(cntv, l[k], live);
+      else if (live) atomicAdd(&cntv[l[k]], 1u);
+    }
   }
   __syncthreads();
-  block_exclusive_scan(cntv, L2, scan_tmp);
-  for (uint32_t i = threadIdx.x; i < L2; i += SORT_THREADS) {
+  block_exclusive_scan<THREADS>(cntv, L2, scan_tmp);
+  for (uint32_t i = threadIdx.x; i < L2; i += THREADS) {
     offsets[key0 + i] = start + cntv[i];
     cur[i] = start + cntv[i];
   }
   __syncthreads();
   for (uint32_t t0 = start; t0 < end; t0 += TILE) {
     const uint32_t tn = min((uint32_t)TILE, end - t0);
-    for (uint32_t i = threadIdx.x; i < L2; i += SORT_THREADS) tb[i] = 0;
+    for (uint32_t i = threadIdx.x; i < L2; i += THREADS) tb[i] = 0;
     __syncthreads();
-    constexpr int IPT = TILE / SORT_THREADS;
+    constexpr int IPT = TILE / THREADS;
     uint32_t v[IPT], vl[IPT], rk[IPT];
     for (int j = 0; j < IPT; j++) {  // unconditional loads (clamped; tn >= 1)
-      const uint32_t q = j * SORT_THREADS + threadIdx.x, qc = q < tn ? q : tn - 1;
+      const uint32_t q = j * THREADS + threadIdx.x, qc = q < tn ? q : tn - 1;
       v[j] = tix[t0 + qc];
       vl[j] = tlo[t0 + qc];
     }
     for (int j = 0; j < IPT; j++) {
-      const uint32_t q = j * SORT_THREADS + threadIdx.x;
-      rk[j] = q < tn ? atomicAdd(&tb[vl[j]], 1u) : 0u;
+      const uint32_t q = j * THREADS + threadIdx.x;
+      if (LONG) rk[j] = count_hot(tb, vl[j], q < tn);
+      else rk[j] = q < tn ? atomicAdd(&tb[vl[j]], 1u) : 0u;
     }
     __syncthreads();
     // tile-local counts -> tile-local bases; keep the counts for the cursor update
-    for (uint32_t i = threadIdx.x; i < L2; i += SORT_THREADS) cntv[i] = tb[i];
+    for (uint32_t i = threadIdx.x; i < L2; i += THREADS) cntv[i] = tb[i];
     __syncthreads();
-    block_exclusive_scan(tb, L2, scan_tmp);
+    block_exclusive_scan<THREADS>(tb, L2, scan_tmp);
     for (int j = 0; j < IPT; j++) {
-      uint32_t q = j * SORT_THREADS + threadIdx.x;
+      uint32_t q = j * THREADS + threadIdx.x;
       if (q < tn) {
         uint32_t lo = vl[j];
         uint32_t pos = tb[lo] + rk[j];
@@ -517,12 +591,12 @@ __global__ void __launch_bounds__(SORT_THREADS) k_sort_pass2(const uint32_t *__r
       }
     }
     __syncthreads();
-    for (uint32_t p = threadIdx.x; p < tn; p += SORT_THREADS) {
+    for (uint32_t p = threadIdx.x; p < tn; p += THREADS) {
       uint32_t lo = sbin[p];
       sorted[cur[lo] + (p - tb[lo])] = stage[p];
     }
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < L2; i += SORT_THREADS) cur[i] += cntv[i];
+    for (uint32_t i = threadIdx.x; i < L2; i += THREADS) cur[i] += cntv[i];
     __syncthreads();
   }
 }
@@ -874,6 +948,62 @@ __global__ void __launch_bounds__(256) k_carry_round(const uint32_t *__restrict_
   if (head) grp_store<F>(carry + u * SW, a);
 }
 
+// The slots kCarryTail apart that the rounds of step 1 .. kCarryTail / 8 leave in a
+// longer chain, summed by the wave that finds the chain's head: its groups take
+// every NG-th slot each, then join.  Chains this long are few (a bucket of more
+// than kCarryTail L entries), so one launch that looks for them costs less than a
+// launch per round.
+static constexpr uint32_t kCarryTail = 64;
+template <class F>
+__global__ void __launch_bounds__(256) k_carry_tail(const uint32_t *__restrict__ off, uint32_t K, uint32_t L,
+                                                    uint32_t *carry, const uint32_t *__restrict__ carry_key) {
+  constexpr uint32_t SW = Slot29<F>::SW, GN = Grp<F>::N, NG = 64 / GN;
+  const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
+  uint32_t len = 0;
+  if ((uint64_t)u * L < off[K]) {
+    const uint32_t key = carry_key[u];
+    if (key != 0xFFFFFFFFu) {
+      const uint32_t t0 = off[key] / L, t1 = (off[key + 1] - 1) / L;
+      if (u == t0 + 1) len = t1 - t0;
+    }
+  }
+  uint64_t heads = __ballot(len > kCarryTail);
+  const uint32_t lane = threadIdx.x & 63, grp = lane / GN;
+  for (; heads; heads &= heads - 1) {
+    const uint32_t h = __builtin_ctzll(heads);
+    const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)len, h);
+    uint32_t *base = carry + (uint64_t)(u - lane + h) * SW;
+    const uint32_t count = (n + kCarryTail - 1) / kCarryTail;
+    Fq29 a = {};
+    if (grp < count) grp_load<F>(base + (uint64_t)grp * kCarryTail * SW, a);
+#pragma unroll 1
+    for (uint32_t k0 = NG; k0 < count; k0 += NG) {
+      Fq29 b = {};
+      if (k0 + grp < count) grp_load<F>(base + (uint64_t)(k0 + grp) * kCarryTail * SW, b);
+      grp_add<F>(a, b);
+    }
+#pragma unroll 1
+    for (uint32_t d = NG / 2; d > 0; d /= 2) {
+      Fq29 b;
+#pragma unroll
+      for (int i = 0; i < 9; i++) b.l[i] = __shfl_down(a.l[i], d * GN, 64);
+      if (grp >= d) b = Fq29{};
+      grp_add<F>(a, b);
+    }
+    if (grp == 0) grp_store<F>(base, a);
+  }
+}
+
+// every chain's sum into its head slot
+template <class F>
+static void carry_chains(const uint32_t *off, uint32_t K, const MsmPlan &pl, uint32_t *carry,
+                         const uint32_t *carry_key, hipStream_t st) {
+  for (uint64_t step = 1; step < kCarryTail && step < pl.max_chunks; step *= 8)
+    k_carry_round<F><<<grp_blocks<F>(pl.max_chunks), 256, 0, st>>>(off, K, pl.L, carry, carry_key, (uint32_t)step);
+  if (pl.max_chunks > kCarryTail)
+    k_carry_tail<F><<<(uint32_t)((pl.max_chunks + 255) / 256), 256, 0, st>>>(off, K, pl.L, carry, carry_key);
+}
+
 // One thread per bucket: add the (reduced) chain head at slot t0+1.
 template <class F>
 __global__ void __launch_bounds__(256) k_fixup(const uint32_t *__restrict__ off, uint32_t K, uint32_t L,
@@ -1144,12 +1274,20 @@ static inline void sort_place(const MsmPlan &pl, uint32_t Wwin, const uint32_t *
                                                            tlo, sorted);
   // the 8192-entry tile keeps 49 KB of staging in LDS beside 3 * 2^sb counter
   // words: used up to sb = 10 (61 KB); wider windows take the 4096 tile
+  const uint32_t lds = 3 * (1u << sb) * 4;
+  // a segment holds at most a member's points; the long ones have eight times
+  // the average, and more than four tiles
+  const uint64_t longest = std::max<uint64_t>(4 * SORT_TILE, 8 * (pl.most >> pl.hb));
+  const uint32_t split = pl.most > longest ? (uint32_t)longest : 0xFFFFFFFFu;
   if (pl.max_entries < (1ull << 27) || sb > 10)
-    k_sort_pass2<SORT_TILE><<<Wtot * HB, SORT_THREADS, 3 * (1u << sb) * 4, st>>>(
-        tix, tlo, cnt, segs, HB, sb, pl.st, pl.W, Wwin, Ktot, offsets, sorted);
+    k_sort_pass2<SORT_TILE, SORT_THREADS, false><<<Wtot * HB, SORT_THREADS, lds, st>>>(
+        tix, tlo, cnt, segs, HB, sb, pl.st, pl.W, Wwin, Ktot, split, offsets, sorted);
   else
-    k_sort_pass2<2 * SORT_TILE><<<Wtot * HB, SORT_THREADS, 3 * (1u << sb) * 4, st>>>(
-        tix, tlo, cnt, segs, HB, sb, pl.st, pl.W, Wwin, Ktot, offsets, sorted);
+    k_sort_pass2<2 * SORT_TILE, SORT_THREADS, false><<<Wtot * HB, SORT_THREADS, lds, st>>>(
+        tix, tlo, cnt, segs, HB, sb, pl.st, pl.W, Wwin, Ktot, split, offsets, sorted);
+  if (split != 0xFFFFFFFFu)
+    k_sort_pass2<SORT_TILE, 1024, true><<<Wtot * HB, 1024, lds, st>>>(tix, tlo, cnt, segs, HB, sb, pl.st, pl.W, Wwin,
+                                                                      Ktot, split, offsets, sorted);
 }
 
 // Enqueue the whole pipeline for one group on stream st.  segs is the
@@ -1197,9 +1335,7 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
       k_digits<F, 1><<<(uint32_t)pl.tiles, DT, pl.W * HB * 4, st>>>(segs, pl.J, pl.c, pl.W, sb, pl.st, HB, digits,
                                                                     cnt, pts29);
     CSK_CHECK_LAUNCH();
-    k_scan_reduce<<<nb, SCAN_THREADS, 0, st>>>(cnt, ncnt, bsum);
-    k_scan_blocks<<<1, 1024, 0, st>>>(bsum, nb);
-    k_scan_final<<<nb, SCAN_THREADS, 0, st>>>(cnt, ncnt, bsum, cnt);
+    scan_counts(cnt, ncnt, bsum, st);
     sort_place(pl, pl.W, digits, segs, cnt, tix, tlo, offsets, sorted, st);
     CSK_CHECK_LAUNCH();
     const uint32_t TB = g2 ? 128 : 256;
@@ -1211,10 +1347,7 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
       k_accumulate29_g2<F><<<ga, TB, 0, st>>>(segs, pl.K, sorted, offsets, Ktot, pl.L, pts29, b29, cr29, carry_key);
     CSK_CHECK_LAUNCH();
     if (tm) tm->mark(2, st);
-    // chains can be at most max_chunks long
-    for (uint64_t step = 1; step < pl.max_chunks; step *= 8)
-      k_carry_round<F><<<grp_blocks<F>(pl.max_chunks), 256, 0, st>>>(offsets, Ktot, pl.L, cr29, carry_key,
-                                                                               (uint32_t)step);
+    carry_chains<F>(offsets, Ktot, pl, cr29, carry_key, st);
     CSK_CHECK_LAUNCH();
     k_fixup<F><<<(Ktot + TB - 1) / TB, TB, 0, st>>>(offsets, Ktot, pl.L, b29, cr29);
     CSK_CHECK_LAUNCH();
@@ -1428,9 +1561,7 @@ int msm_run_table(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArg
   k_put_outs<<<1, 128, 0, st>>>(args, count, osegs);
   k_digits_tab<<<dim3(max_nt, count), 256, Wt * HB * 4, st>>>(args, segs, pl.c, Wt, sb, pl.st, HB, digits, cnt);
   CSK_CHECK_LAUNCH();
-  k_scan_reduce<<<nb, SCAN_THREADS, 0, st>>>(cnt, ncnt, bsum);
-  k_scan_blocks<<<1, 1024, 0, st>>>(bsum, nb);
-  k_scan_final<<<nb, SCAN_THREADS, 0, st>>>(cnt, ncnt, bsum, cnt);
+  scan_counts(cnt, ncnt, bsum, st);
   sort_place(pl, Wt, digits, segs, cnt, tix, tlo, offsets, sorted, st);
   CSK_CHECK_LAUNCH();
   const uint32_t TB = g2 ? 128 : 256;
@@ -1441,9 +1572,7 @@ int msm_run_table(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArg
     k_accumulate29_g2<F><<<ga, TB, 0, st>>>(segs, pl.K, sorted, offsets, Ktot, pl.L, nullptr, b29, cr29,
                                              carry_key);
   CSK_CHECK_LAUNCH();
-  for (uint64_t step = 1; step < pl.max_chunks; step *= 8)
-    k_carry_round<F><<<grp_blocks<F>(pl.max_chunks), 256, 0, st>>>(offsets, Ktot, pl.L, cr29, carry_key,
-                                                                             (uint32_t)step);
+  carry_chains<F>(offsets, Ktot, pl, cr29, carry_key, st);
   CSK_CHECK_LAUNCH();
   k_fixup<F><<<(Ktot + TB - 1) / TB, TB, 0, st>>>(offsets, Ktot, pl.L, b29, cr29);
   k_merge_members<F><<<dim3((pl.B + TB - 1) / TB, count), TB, 0, st>>>(offsets, b29, Wt, pl.B, merged);

@@ -6,9 +6,11 @@ import pytest
 
 import oracle as O
 from cusnarks_amd import inputs
-from cusnarks_amd.msm import msm_host
+from cusnarks_amd import _capi
+from cusnarks_amd.device import DeviceBuffer
+from cusnarks_amd.msm import fixed_base, msm_device, msm_host
 from oracle import pyoracle as P
-from tests.gpu_util import gen_mul
+from tests.gpu_util import dot_mod_r, gen_mul
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +67,23 @@ def test_reduction_shapes(g2, c, reduce_seg):
     pts = np.stack([base[e] for e in exps])
     want = gen_mul(sum(k * e for k, e in zip(inputs.to_ints(ks), exps)) % P.RR, g2)
     assert np.array_equal(msm_host(ks, pts, g2=g2, window_bits=c, reduce_seg=min(reduce_seg, 1 << (c - 1))), want)
+
+
+@pytest.mark.parametrize("n,g2", [(9000, False), (33000, False), (150001, False), (40001, True)])
+def test_wire_value_scalars(n, g2):
+    # one bucket holds most of the entries: long first-pass bins (a launch of
+    # their own above 4 tiles) and carry chains of more than 64 chunks
+    ctx = _capi.default_context()
+    rng = np.random.default_rng(n)
+    k = inputs.field_elements(50, n, nonzero=True)
+    sc = inputs.field_elements(51, n)
+    u = rng.random(n)
+    sc[u < 0.9, 1:] = 0
+    sc[u < 0.7, 0] = 1
+    d_k, d_s = DeviceBuffer.from_array(ctx, k), DeviceBuffer.from_array(ctx, sc)
+    pts, out = DeviceBuffer(ctx, n * (128 if g2 else 64)), DeviceBuffer(ctx, 128)
+    fixed_base(d_k, n, pts, g2=g2)
+    want = gen_mul(dot_mod_r(k, sc), g2)
+    for c in (0, 9):
+        msm_device(d_s, pts, n, out, g2=g2, window_bits=c)
+        assert np.array_equal(out.download((32 if g2 else 16,)), want)
