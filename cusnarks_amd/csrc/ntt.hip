@@ -266,9 +266,26 @@ k_ntt_r4(const uint32_t *__restrict__ src_in, uint32_t *__restrict__ dst_in, uin
     sh[4 * RS + p] = y.x; sh[5 * RS + p] = y.y; sh[6 * RS + p] = y.z; sh[7 * RS + p] = y.w;
   }
   __syncthreads();
-  // stages on t-bits b = R-1 .. 0, two at a time; an odd R ends with one radix-2 stage
+  // stages on t-bits b = R-1 .. 0, two at a time; an odd R begins with one radix-2
+  // stage, so that the transform's last pair is always stages 1 and 0
   int b = (int)R - 1;
-  for (; b >= 1; b -= 2) {
+  if (R & 1) {  // radix-2 stage s_lo + b: pairs (t, t + 2^b)
+    const uint32_t qb = R - 1, h = 1u << b;
+#pragma unroll 1
+    for (uint32_t idx = threadIdx.x; idx < TILE / 2; idx += NTT_THREADS) {
+      const uint32_t g = LAST ? idx >> qb : idx & (G - 1), t = LAST ? idx & (h - 1) : idx >> lgG;
+      const uint64_t jm = ((uint64_t)t << s_lo) + (LAST ? 0u : low0 + g);
+      Fr w;
+      ld8(w.v, T + 8 * ((1ull << (s_lo + b)) + jm));
+      const uint32_t pa = pos(g, t), pc = pos(g, t + h);
+      const Fr a = lds_ld(sh, RS, pa), c = lds_ld(sh, RS, pc);
+      lds_st(sh, RS, pa, Fr::add_lazy(a, c));
+      lds_st(sh, RS, pc, Fr::mul_lazy(Fr::sub_lazy(a, c), w));
+    }
+    __syncthreads();
+    b--;
+  }
+  for (; b >= (LAST ? 3 : 1); b -= 2) {
     const uint32_t h = 1u << (b - 1);
     const uint32_t s = s_lo + b;  // the upper stage of the pair
     const uint32_t qb = R - 2;    // q < 2^(R-2)
@@ -302,19 +319,22 @@ k_ntt_r4(const uint32_t *__restrict__ src_in, uint32_t *__restrict__ dst_in, uin
     }
     __syncthreads();
   }
-  if (b == 0) {  // radix-2 stage s_lo on t-bit 0: pairs (t, t+1)
-    const uint32_t qb = R - 1;
+  if constexpr (LAST) {
+    // stages 1 and 0 of the transform: every twiddle is 1 but w_4, so one
+    // product in place of four (10 products per element become 9.25 at 2^20)
+    Fr w4;
+    ld8(w4.v, T + 8 * 3);
 #pragma unroll 1
-    for (uint32_t idx = threadIdx.x; idx < TILE / 2; idx += NTT_THREADS) {
-      const uint32_t g = LAST ? idx >> qb : idx & (G - 1), q = LAST ? idx & ((1u << qb) - 1) : idx >> lgG;
-      const uint32_t t = q << 1;
-      const uint64_t jm = LAST ? 0u : low0 + g;  // t mod 2^0 = 0
-      Fr w;
-      ld8(w.v, T + 8 * ((1ull << s_lo) + jm));
-      const uint32_t pa = pos(g, t), pc = pos(g, t + 1);
-      const Fr a = lds_ld(sh, RS, pa), c = lds_ld(sh, RS, pc);
-      lds_st(sh, RS, pa, Fr::add_lazy(a, c));
-      lds_st(sh, RS, pc, Fr::mul_lazy(Fr::sub_lazy(a, c), w));
+    for (uint32_t idx = threadIdx.x; idx < TILE / 4; idx += NTT_THREADS) {
+      const uint32_t p0 = 4 * idx;  // position (g << R) | 4 q
+      const Fr a0 = lds_ld(sh, RS, p0), a1 = lds_ld(sh, RS, p0 + 1);
+      const Fr a2 = lds_ld(sh, RS, p0 + 2), a3 = lds_ld(sh, RS, p0 + 3);
+      const Fr u0 = Fr::add_lazy(a0, a2), u1 = Fr::add_lazy(a1, a3), v0 = Fr::sub_lazy(a0, a2);
+      const Fr v1 = Fr::mul_lazy(Fr::sub_lazy(a1, a3), w4);
+      lds_st(sh, RS, p0, Fr::add_lazy(u0, u1));
+      lds_st(sh, RS, p0 + 1, Fr::sub_lazy(u0, u1));
+      lds_st(sh, RS, p0 + 2, Fr::add_lazy(v0, v1));
+      lds_st(sh, RS, p0 + 3, Fr::sub_lazy(v0, v1));
     }
     __syncthreads();
   }
