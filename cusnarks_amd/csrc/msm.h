@@ -71,13 +71,14 @@ struct TabArgs {
   const uint32_t *live[kTabBatch];
   uint64_t n[kTabBatch];
 };
-// hsegs: host descriptors of the count * Wt members (m = p * Wt + w: window w
-// of run p, n = the table's n_pad, points = that window's slice), copied into
-// the workspace; max_nt: the largest n_pad / 4096 among the runs.
+// hsegs: host descriptors of the members, copied into the workspace: count (run
+// p's Wt windows together, n = Wt * n_pad, points = the table) or count * Wt
+// (m = p * Wt + w: window w of run p, n = n_pad, points = that window's slice);
+// max_nt: the largest n_pad / 4096 among the runs.
 int msm_run_table_g1(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArgs &args, uint32_t count,
-                     uint32_t max_nt, uint32_t Lrm, hipStream_t st);
+                     uint32_t Wt, uint32_t max_nt, uint32_t Lrm, hipStream_t st);
 int msm_run_table_g2(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArgs &args, uint32_t count,
-                     uint32_t max_nt, uint32_t Lrm, hipStream_t st);
+                     uint32_t Wt, uint32_t max_nt, uint32_t Lrm, hipStream_t st);
 size_t msm_table_ws_bytes(const MsmPlan &pl, bool g2, uint32_t count);
 
 // looks up this device's copy of the no-allocation scratch array (the device current)

@@ -362,24 +362,43 @@ struct csk_msm_table {
 
 namespace csk {
 
-// group plan of the count * Wt one-window members of runs over count scalar
-// vectors on a table of n_pad points
-static MsmPlan table_plan(uint32_t c, uint64_t n_pad, uint32_t Wt, uint32_t count) {
+// Whether a run's windows are sorted together, as one member of Wt * n_pad
+// points (a table's slices follow each other, and window w of scalar i is an
+// entry for point w * n_pad + i), so that all of a bucket's entries are
+// adjacent.  As members of one window each, every window has its own copy of
+// the buckets, carried, fixed up and merged: at 100003 points, c = 16, 524288
+// buckets of 3 entries instead of 32768 of 49, 582 -> 449 us; 500 points
+// 411 -> 219, 2^20 1661 -> 1500, 2.2M (2^25 entries) 3267 -> 2993 us; G2 5000 868 ->
+// 454, 2^20 4828 -> 3999 us.  A member has at most 256 second-pass workgroups, so
+// larger runs keep the members: 2^22 points 5886 us joint, 5829 as members.
+static constexpr uint64_t kJointMax = 1ull << 25;
+static bool table_joint(uint64_t n_pad, uint32_t Wt) { return n_pad * Wt <= kJointMax; }
+
+// group plan of the runs over tables of n_pad[0..count) points: count members of
+// Wt * n_pad points, or count * Wt one-window members
+static MsmPlan table_plan(uint32_t c, const uint64_t *n_pad, uint32_t count, uint32_t Wt) {
   MsmPlan pl = {};
+  uint64_t most = 0;
+  for (uint32_t p = 0; p < count; p++) {
+    pl.n += n_pad[p] * Wt;
+    if (n_pad[p] > most) most = n_pad[p];
+  }
+  const bool joint = table_joint(most, Wt);
   pl.c = c;
   pl.E = 1;
   pl.bits = kScalarBits;
   pl.W = 1;
   pl.B = 1u << (c - 1);
   pl.K = pl.B;
-  pl.J = Wt * count;
-  pl.n = n_pad * pl.J;
-  pl.most = n_pad;
-  pl.tiles = pl.J * (n_pad / kSortTile);
+  pl.J = joint ? count : Wt * count;
+  pl.most = joint ? most * Wt : most;
+  pl.tiles = pl.n / kSortTile;
   pl.max_entries = pl.n;
-  pl.hb = plan_hi_bits(c, n_pad);
+  pl.hb = plan_hi_bits(c, pl.n / pl.J);
   pl.st = plan_top_bits(pl.bits, c, pl.hb);
-  uint64_t l = pl.max_entries >> 18;
+  // two waves of chunks per SIMD: with few buckets a shorter chunk only makes
+  // more carries
+  uint64_t l = pl.max_entries >> (joint ? 17 : 18);
   if (l < 8) l = 8;
   if (l > 256) l = 256;
   pl.L = (uint32_t)l;
@@ -420,28 +439,18 @@ static int table_run(csk_ctx *ctx, uint32_t count, csk_msm_table *const *t, cons
                      uint32_t *const *d_out, hipStream_t st) {
   const csk_msm_table *t0 = t[0];
   const uint32_t Wt = t0->Wt, c = t0->c;
-  MsmPlan pl = table_plan(c, t0->n_pad, Wt, 1);  // B, K, hb, L are set below for the whole group
-  pl.J = count * Wt;
-  pl.n = 0;
-  pl.tiles = 0;
   uint32_t max_nt = 0;
+  uint64_t pads[kTabBatch];
   for (uint32_t p = 0; p < count; p++) {
     if (t[p]->ec2 != t0->ec2 || t[p]->c != c || t[p]->ctx->device != ctx->device) {
       set_error("msm_table_run: the tables of one run must share curve, window width and device");
       return CSK_ERR_ARG;
     }
+    pads[p] = t[p]->n_pad;
     const uint32_t nt = (uint32_t)(t[p]->n_pad / kSortTile);
-    pl.n += (uint64_t)Wt * t[p]->n_pad;
-    if (t[p]->n_pad > pl.most) pl.most = t[p]->n_pad;
-    pl.tiles += (uint64_t)Wt * nt;
     if (nt > max_nt) max_nt = nt;
   }
-  pl.max_entries = pl.n;
-  pl.hb = plan_hi_bits(c, pl.n / pl.J);
-  pl.st = plan_top_bits(pl.bits, c, pl.hb);
-  uint64_t l = pl.max_entries >> 18;
-  pl.L = (uint32_t)(l < 8 ? 8 : l > 256 ? 256 : l);
-  pl.max_chunks = (pl.max_entries + pl.L - 1) / pl.L;
+  const MsmPlan pl = table_plan(c, pads, count, Wt);
   if (!msm_plan_ok(pl)) {
     set_error("msm_table_run: " + std::to_string(count) + " runs of up to " + std::to_string(max_nt * kSortTile) +
               " points exceed the multiexp's index range");
@@ -449,13 +458,14 @@ static int table_run(csk_ctx *ctx, uint32_t count, csk_msm_table *const *t, cons
   }
   CSK_HIP(hipSetDevice(ctx->device));
   const uint64_t PW = t0->ec2 ? 32 : 16;
+  const uint32_t per = pl.J / count;  // members of a run
   std::vector<uint64_t> ns(pl.J);
   std::vector<const uint32_t *> sc(pl.J, nullptr), pts(pl.J);
   std::vector<uint32_t *> outs(pl.J, nullptr);
   for (uint32_t m = 0; m < pl.J; m++) {
-    const csk_msm_table *tp = t[m / Wt];
-    ns[m] = tp->n_pad;
-    pts[m] = tp->table + (uint64_t)(m % Wt) * tp->n_pad * PW;
+    const csk_msm_table *tp = t[m / per];
+    ns[m] = tp->n_pad * (Wt / per);
+    pts[m] = tp->table + (uint64_t)(m % per) * tp->n_pad * PW;
   }
   std::vector<MsmSeg> segs(pl.J + 1);
   msm_fill_segs(pl, ns.data(), sc.data(), pts.data(), outs.data(), segs.data());
@@ -468,8 +478,8 @@ static int table_run(csk_ctx *ctx, uint32_t count, csk_msm_table *const *t, cons
     args.live[p] = t[p]->live;
     args.n[p] = t[p]->n;
   }
-  return t0->ec2 ? msm_run_table_g2(ctx->ws.ptr, pl, segs.data(), args, count, max_nt, t0->Lrm, st)
-                 : msm_run_table_g1(ctx->ws.ptr, pl, segs.data(), args, count, max_nt, t0->Lrm, st);
+  return t0->ec2 ? msm_run_table_g2(ctx->ws.ptr, pl, segs.data(), args, count, Wt, max_nt, t0->Lrm, st)
+                 : msm_run_table_g1(ctx->ws.ptr, pl, segs.data(), args, count, Wt, max_nt, t0->Lrm, st);
 }
 
 }  // namespace csk
@@ -498,7 +508,7 @@ extern "C" int csk_msm_table_create(csk_ctx *ctx, int ec2, const uint32_t *d_poi
   }
   const uint32_t Wt = 254 / c + 1;
   const uint64_t n_pad = (n + kSortTile - 1) / kSortTile * kSortTile;
-  MsmPlan pl = table_plan(c, n_pad, Wt, 1);
+  MsmPlan pl = table_plan(c, &n_pad, 1, Wt);
   if (!msm_plan_ok(pl)) {
     set_error("msm_table_create: " + std::to_string(n) + " points x " + std::to_string(Wt) +
               " windows exceed the multiexp's index range");
@@ -589,7 +599,7 @@ extern "C" int csk_msm_table_run_multi(csk_ctx *ctx, uint32_t count, csk_msm_tab
 
 extern "C" int csk_msm_table_info(const csk_msm_table *t, uint64_t *out, int n) {
   if (!t || !out || n < 1) return CSK_ERR_ARG;
-  const MsmPlan pl = table_plan(t->c, t->n_pad, t->Wt, 1);
+  const MsmPlan pl = table_plan(t->c, &t->n_pad, 1, t->Wt);
   const uint64_t v[5] = {t->n, t->c, t->Wt, t->table_bytes, msm_table_ws_bytes(pl, t->ec2 != 0, 1)};
   for (int i = 0; i < n && i < 5; i++) out[i] = v[i];
   return CSK_OK;

@@ -10,7 +10,7 @@ int msm_table_build_g2(const uint32_t *pts, uint64_t n, uint64_t n_pad, uint32_t
   return msm_table_build<Fq2>(pts, n, n_pad, c, Wt, table, live, st);
 }
 int msm_run_table_g2(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArgs &args, uint32_t count,
-                     uint32_t max_nt, uint32_t Lrm, hipStream_t st) {
-  return msm_run_table<Fq2>(ws, pl, hsegs, args, count, max_nt, Lrm, st);
+                     uint32_t Wt, uint32_t max_nt, uint32_t Lrm, hipStream_t st) {
+  return msm_run_table<Fq2>(ws, pl, hsegs, args, count, Wt, max_nt, Lrm, st);
 }
 }  // namespace csk

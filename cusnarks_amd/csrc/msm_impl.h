@@ -908,18 +908,23 @@ template <> struct Acc29<Fq2> {
 };
 
 // Carries of one bucket occupy the consecutive chunk slots t0+1 .. t1 of a
-// bucket [s, e) (t0 = s/L, t1 = (e-1)/L).  A bucket far larger than a chunk
-// (skewed digits: small witness values, a narrow top window) gives a long
-// chain, so chains are summed by log-depth radix-8 rounds: in the round of
-// step 8^r the slot at chain index i (i % 8^(r+1) == 0) adds the slots at
-// i + k*8^r, k = 1..7, that lie in the chain.  The slots read are never
-// written in the same round.  Slots are 29-bit (SW words).
+// bucket [s, e) (t0 = s/L, t1 = (e-1)/L), chain index 0 .. t1-t0-1.  k_fixup adds
+// up to `keep` slots of its bucket's chain to the bucket: one with a lane per
+// bucket, where a second would keep whole waves for a few lanes (the G1 fix-up of a
+// 50000-constraint proof 113 -> 163 us), eight with a group per bucket, where the
+// buckets are few and their chains long.  Longer
+// chains are thinned first (a bucket far larger than a chunk: skewed digits,
+// small witness values, a narrow top window): in the round of step 8^r the slot
+// at chain index i (i % 8^(r+1) == 0) adds the slots at i + k*8^r, k = 1..7, that
+// lie in the chain, if the chain has more than keep * 8^r of them.  The slots read
+// are never written in the same round.  Slots are 29-bit (SW words).
 // A group of lanes per slot (quad29.h): a round is a chain of up to seven
 // additions, and few slots of a round head one.
 template <class F>
 __global__ void __launch_bounds__(256) k_carry_round(const uint32_t *__restrict__ off, uint32_t K, uint32_t L,
                                                      uint32_t *__restrict__ carry,
-                                                     const uint32_t *__restrict__ carry_key, uint32_t step) {
+                                                     const uint32_t *__restrict__ carry_key, uint32_t step,
+                                                     uint32_t keep) {
   constexpr int SW = Slot29<F>::SW;
   constexpr uint32_t GN = Grp<F>::N;
   const uint64_t u = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / GN;
@@ -933,7 +938,8 @@ __global__ void __launch_bounds__(256) k_carry_round(const uint32_t *__restrict_
       len = t1 - t0;
     }
   }
-  const bool head = ((uint64_t)i & (8ull * step - 1)) == 0 && (uint64_t)i + step < len;
+  const bool head = ((uint64_t)i & (8ull * step - 1)) == 0 && (uint64_t)i + step < len &&
+                    len > (uint64_t)keep * step;
   if (!__any(head)) return;
   Fq29 a = {};
   if (head) grp_load<F>(carry + u * SW, a);
@@ -949,14 +955,13 @@ __global__ void __launch_bounds__(256) k_carry_round(const uint32_t *__restrict_
 }
 
 // The slots kCarryTail apart that the rounds of step 1 .. kCarryTail / 8 leave in a
-// longer chain, summed by the wave that finds the chain's head: its groups take
-// every NG-th slot each, then join.  Chains this long are few (a bucket of more
-// than kCarryTail L entries), so one launch that looks for them costs less than a
-// launch per round.
+// chain of more than keep * kCarryTail, summed by the wave that finds the chain's
+// head: its groups take every NG-th slot each, then join.  Chains this long are
+// few, so one launch that looks for them costs less than a launch per round.
 static constexpr uint32_t kCarryTail = 64;
 template <class F>
 __global__ void __launch_bounds__(256) k_carry_tail(const uint32_t *__restrict__ off, uint32_t K, uint32_t L,
-                                                    uint32_t *carry, const uint32_t *__restrict__ carry_key) {
+                                                    uint32_t *carry, const uint32_t *__restrict__ carry_key, uint32_t keep) {
   constexpr uint32_t SW = Slot29<F>::SW, GN = Grp<F>::N, NG = 64 / GN;
   const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
   uint32_t len = 0;
@@ -967,7 +972,7 @@ __global__ void __launch_bounds__(256) k_carry_tail(const uint32_t *__restrict__
       if (u == t0 + 1) len = t1 - t0;
     }
   }
-  uint64_t heads = __ballot(len > kCarryTail);
+  uint64_t heads = __ballot(len > keep * kCarryTail);
   const uint32_t lane = threadIdx.x & 63, grp = lane / GN;
   for (; heads; heads &= heads - 1) {
     const uint32_t h = __builtin_ctzll(heads);
@@ -994,17 +999,14 @@ __global__ void __launch_bounds__(256) k_carry_tail(const uint32_t *__restrict__
   }
 }
 
-// every chain's sum into its head slot
-template <class F>
-static void carry_chains(const uint32_t *off, uint32_t K, const MsmPlan &pl, uint32_t *carry,
-                         const uint32_t *carry_key, hipStream_t st) {
-  for (uint64_t step = 1; step < kCarryTail && step < pl.max_chunks; step *= 8)
-    k_carry_round<F><<<grp_blocks<F>(pl.max_chunks), 256, 0, st>>>(off, K, pl.L, carry, carry_key, (uint32_t)step);
-  if (pl.max_chunks > kCarryTail)
-    k_carry_tail<F><<<(uint32_t)((pl.max_chunks + 255) / 256), 256, 0, st>>>(off, K, pl.L, carry, carry_key);
+// the slots apart that the rounds leave of a chain with keep = 8: at most eight, or
+// its head
+__device__ __forceinline__ uint32_t chain_stride(uint32_t len) {
+  return len <= 8 ? 1 : len <= 64 ? 8 : len <= 512 ? 64 : len;
 }
+static_assert(kCarryTail == 64, "chain_stride");
 
-// One thread per bucket: add the (reduced) chain head at slot t0+1.
+// every bucket gets its chain: a lane per bucket, or (k_fixup_groups) a group
 template <class F>
 __global__ void __launch_bounds__(256) k_fixup(const uint32_t *__restrict__ off, uint32_t K, uint32_t L,
                                                uint32_t *__restrict__ buckets,
@@ -1015,13 +1017,59 @@ __global__ void __launch_bounds__(256) k_fixup(const uint32_t *__restrict__ off,
   if (key >= K) return;
   const uint32_t s = off[key], e = off[key + 1];
   if (e == s) return;
-  const uint32_t t0 = s / L, t1 = (e - 1) / L;
-  if (t1 == t0) return;
+  const uint32_t t0 = s / L, len = (e - 1) / L - t0;
+  if (len == 0) return;
   A acc, c;
   load29(buckets + (uint64_t)key * SW, acc);
   load29(carry + (uint64_t)(t0 + 1) * SW, c);
   xadd29(acc, c);
   store29(buckets + (uint64_t)key * SW, acc);
+}
+template <class F>
+__global__ void __launch_bounds__(256) k_fixup_groups(const uint32_t *__restrict__ off, uint32_t K, uint32_t L,
+                                                      uint32_t *__restrict__ buckets,
+                                                      const uint32_t *__restrict__ carry) {
+  constexpr uint32_t SW = Slot29<F>::SW, GN = Grp<F>::N;
+  const uint32_t key = (uint32_t)(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / GN);
+  uint32_t t0 = 0, len = 0;
+  if (key < K) {
+    const uint32_t s = off[key], e = off[key + 1];
+    if (e != s) {
+      t0 = s / L;
+      len = (e - 1) / L - t0;
+    }
+  }
+  if (!__any(len != 0)) return;
+  const uint32_t stride = chain_stride(len);
+  Fq29 acc = {};
+  if (len) grp_load<F>(buckets + (uint64_t)key * SW, acc);
+#pragma unroll 1
+  for (uint32_t k = 0; __any(k < len); k += stride) {
+    Fq29 c = {};
+    if (k < len) grp_load<F>(carry + (uint64_t)(t0 + 1 + k) * SW, c);
+    grp_add<F>(acc, c);
+  }
+  if (len) grp_store<F>(buckets + (uint64_t)key * SW, acc);
+}
+
+// the carries into their buckets
+template <class F>
+static void carry_chains(const uint32_t *off, uint32_t K, const MsmPlan &pl, uint32_t *buckets, uint32_t *carry,
+                         const uint32_t *carry_key, hipStream_t st) {
+  // from two waves of buckets per SIMD on a lane each fills the chip, and chains are
+  // few or short; below, the chains are what is waited for.  Rounds and fix-up
+  // together, keep = 1 with lanes against 8 with groups: 32768 G1 buckets of 49
+  // entries 112 against 47 us, 262144 of 52 equal within 2% of the multiexp
+  const bool lanes = K >= 1u << 17;
+  const uint32_t keep = lanes ? 1 : 8;
+  for (uint32_t step = 1; step < kCarryTail && keep * step < pl.max_chunks; step *= 8)
+    k_carry_round<F><<<grp_blocks<F>(pl.max_chunks), 256, 0, st>>>(off, K, pl.L, carry, carry_key, step, keep);
+  if (pl.max_chunks > keep * kCarryTail)
+    k_carry_tail<F><<<(uint32_t)((pl.max_chunks + 255) / 256), 256, 0, st>>>(off, K, pl.L, carry, carry_key, keep);
+  if (lanes)
+    k_fixup<F><<<(K + 127) / 128, 128, 0, st>>>(off, K, pl.L, buckets, carry);
+  else
+    k_fixup_groups<F><<<grp_blocks<F>(K), 256, 0, st>>>(off, K, pl.L, buckets, carry);
 }
 
 // ------------------------------------------------------------ window sums
@@ -1347,9 +1395,7 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
       k_accumulate29_g2<F><<<ga, TB, 0, st>>>(segs, pl.K, sorted, offsets, Ktot, pl.L, pts29, b29, cr29, carry_key);
     CSK_CHECK_LAUNCH();
     if (tm) tm->mark(2, st);
-    carry_chains<F>(offsets, Ktot, pl, cr29, carry_key, st);
-    CSK_CHECK_LAUNCH();
-    k_fixup<F><<<(Ktot + TB - 1) / TB, TB, 0, st>>>(offsets, Ktot, pl.L, b29, cr29);
+    carry_chains<F>(offsets, Ktot, pl, b29, cr29, carry_key, st);
     CSK_CHECK_LAUNCH();
     window_sums<F>(offsets, b29, Wtot, pl.B, pl.Lr, wsum, st);
     CSK_CHECK_LAUNCH();
@@ -1366,11 +1412,12 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
 // 2^(c w) P_i for w < Wt = floor(254 / c) + 1 (n_pad = n rounded up to the
 // sort tile), in the 2^261 form the bucket loops read, and a bit per point,
 // 1 unless P_i is at infinity.  With the signed c-bit digits d_(i,w) of k_i,
-// sum_i k_i P_i = sum_(w, i) d_(i,w) Q[w * n_pad + i]: the multiexp runs as a
-// group of Wt one-window members (member w: digit w of every scalar, points
-// Q[w * n_pad ..]), which sorts and accumulates exactly as a plain group;
-// then bucket b of the sum is the sum over w of member w's bucket b, reduced
-// once, and no doublings are needed between windows.
+// sum_i k_i P_i = sum_(w, i) d_(i,w) Q[w * n_pad + i]: the multiexp runs as one
+// member of Wt * n_pad points and one window, which sorts, accumulates and
+// reduces exactly as a plain one; or, when large, as a group of Wt one-window
+// members (member w: digit w of every scalar, points Q[w * n_pad ..]), whose
+// buckets b are then summed over w and reduced once.  No doublings are needed
+// between windows.
 
 // one thread per point: its Wt table entries (an inversion each) and its bit;
 // grid covers n_pad (a multiple of the sort tile) exactly
@@ -1406,16 +1453,19 @@ namespace {  // curve-independent table kernels: one private copy per translatio
 // + w * n_pad (as k_digits writes a one-window member at its concatenated
 // points), empty (0xFFFFFFFF) for a zero digit, a point at infinity or i >= n.
 // Counts go to cnt[cbase_m + hi * NT + tile], cbase_m = cbase_(p*Wt) + w * HB
-// * NT, the member's pass-1 counters.
-__global__ void __launch_bounds__(256) k_digits_tab(TabArgs args, const MsmSeg *__restrict__ segs, uint32_t c,
-                                                    uint32_t Wt, uint32_t s, uint32_t ts, uint32_t HB,
+// * NT, the member's pass-1 counters.  With a run's windows together (per = 1) it is
+// member p, window w's tiles are w * NT + tile of it, and every window splits
+// its buckets at s bits.
+__global__ void __launch_bounds__(256) k_digits_tab(TabArgs args, const MsmSeg *__restrict__ segs, uint32_t per,
+                                                    uint32_t c, uint32_t Wt, uint32_t s, uint32_t ts, uint32_t HB,
                                                     uint32_t *__restrict__ digits, uint32_t *__restrict__ cnt) {
   extern __shared__ uint32_t hist[];  // Wt * HB counters
   const uint32_t tile = blockIdx.x, p = blockIdx.y;
-  const MsmSeg &g0 = segs[p * Wt];
-  const uint32_t NT = g0.NT;
+  const MsmSeg &g0 = segs[p * per];
+  const uint64_t n = args.n[p];
+  const uint32_t NT = (uint32_t)((n + kSortTile - 1) / kSortTile);
   if (tile >= NT) return;  // the whole workgroup: this run's table has fewer tiles
-  const uint64_t n = args.n[p], n_pad = g0.n;
+  const uint64_t n_pad = (uint64_t)NT * kSortTile;
   const uint32_t *__restrict__ scalars = args.s[p];
   const uint32_t *__restrict__ live = args.live[p];
   digits += g0.pbase;
@@ -1442,7 +1492,10 @@ __global__ void __launch_bounds__(256) k_digits_tab(TabArgs args, const MsmSeg *
     }
   }
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < Wt * HB; i += blockDim.x) cnt[(uint64_t)i * NT + tile] = hist[i];
+  for (uint32_t i = threadIdx.x; i < Wt * HB; i += blockDim.x) {
+    const uint32_t w = i / HB, hi = i - w * HB;
+    cnt[per == 1 ? ((uint64_t)hi * Wt + w) * NT + tile : (uint64_t)i * NT + tile] = hist[i];
+  }
 }
 
 // merged[p * B + b] = sum over the J members of vector p (blockIdx.y) of their
@@ -1510,8 +1563,10 @@ inline size_t msm_table_workspace_bytes(const MsmPlan &pl, bool g2, uint32_t cou
   b += Carver::round(nb * 4);
   b += Carver::round((Ktot + 1) * 4);
   b += Carver::round(pl.max_chunks * 4);
-  b += Carver::round((uint64_t)count * pl.B * sb);        // merged buckets
-  b += Carver::round(((uint64_t)count * pl.B + 1) * 4);   // iota offsets
+  if (pl.J != count) {
+    b += Carver::round((uint64_t)count * pl.B * sb);       // merged buckets
+    b += Carver::round(((uint64_t)count * pl.B + 1) * 4);  // iota offsets
+  }
   b += Carver::round((uint64_t)count * sb);               // their sums
   b += Carver::round((uint64_t)(count + 1) * sizeof(MsmSeg));  // output descriptors
   b += Carver::round(((uint64_t)pl.J + 1) * sizeof(MsmSeg));   // member descriptors
@@ -1519,13 +1574,13 @@ inline size_t msm_table_workspace_bytes(const MsmPlan &pl, bool g2, uint32_t cou
 }
 
 // Enqueue count table multiexps (run p: scalar vector args.s[p] over its
-// table -> args.o[p]): pl is the group plan of the count * Wt one-window
-// members m = p * Wt + w (J = count * Wt, W = 1), hsegs their host
-// descriptors (member m reads its table's slice of window w through its points
-// pointer), Lrm the buckets a reduction quad sums of a merged window.
+// table -> args.o[p]): pl is the group plan of the runs as count members of all
+// their windows, or as count * Wt one-window members m = p * Wt + w (W = 1),
+// hsegs their host descriptors (a member reads its table, or the slice of its
+// window, through its points pointer), Lrm the buckets of a reduction segment.
 template <class F>
 int msm_run_table(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArgs &args, uint32_t count,
-                  uint32_t max_nt, uint32_t Lrm, hipStream_t st) {
+                  uint32_t Wt, uint32_t max_nt, uint32_t Lrm, hipStream_t st) {
   const bool g2 = FieldIO<F>::NW == 16;
   constexpr int SW = Slot29<F>::SW;
   Carver cv(ws);
@@ -1550,19 +1605,24 @@ int msm_run_table(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArg
   uint32_t *bsum = cv.take<uint32_t>(nb);
   uint32_t *offsets = cv.take<uint32_t>((size_t)Ktot + 1);
   uint32_t *carry_key = cv.take<uint32_t>(pl.max_chunks);
-  uint32_t *merged = cv.take<uint32_t>((size_t)count * pl.B * SW);
-  uint32_t *iota = cv.take<uint32_t>((size_t)count * pl.B + 1);
+  const uint32_t per = pl.J / count;  // members of a run
+  uint32_t *merged = b29, *moff = offsets;
+  if (per > 1) {
+    merged = cv.take<uint32_t>((size_t)count * pl.B * SW);
+    moff = cv.take<uint32_t>((size_t)count * pl.B + 1);
+  }
   uint32_t *wsum = cv.take<uint32_t>((size_t)count * SW);
   MsmSeg *osegs = cv.take<MsmSeg>(count + 1);
   MsmSeg *segs = cv.take<MsmSeg>(pl.J + 1);
-  const uint32_t Wt = pl.J / count;
 
   CSK_HIP(hipMemcpyAsync(segs, hsegs, ((size_t)pl.J + 1) * sizeof(MsmSeg), hipMemcpyHostToDevice, st));
   k_put_outs<<<1, 128, 0, st>>>(args, count, osegs);
-  k_digits_tab<<<dim3(max_nt, count), 256, Wt * HB * 4, st>>>(args, segs, pl.c, Wt, sb, pl.st, HB, digits, cnt);
+  k_digits_tab<<<dim3(max_nt, count), 256, Wt * HB * 4, st>>>(args, segs, per, pl.c, Wt, sb, per > 1 ? pl.st : sb, HB,
+                                                                          digits, cnt);
   CSK_CHECK_LAUNCH();
   scan_counts(cnt, ncnt, bsum, st);
-  sort_place(pl, Wt, digits, segs, cnt, tix, tlo, offsets, sorted, st);
+  // no window of a member of all windows is the top one
+  sort_place(pl, per > 1 ? Wt : 0xFFFFFFFFu, digits, segs, cnt, tix, tlo, offsets, sorted, st);
   CSK_CHECK_LAUNCH();
   const uint32_t TB = g2 ? 128 : 256;
   const uint32_t ga = (uint32_t)((pl.max_chunks + TB - 1) / TB);
@@ -1572,13 +1632,14 @@ int msm_run_table(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArg
     k_accumulate29_g2<F><<<ga, TB, 0, st>>>(segs, pl.K, sorted, offsets, Ktot, pl.L, nullptr, b29, cr29,
                                              carry_key);
   CSK_CHECK_LAUNCH();
-  carry_chains<F>(offsets, Ktot, pl, cr29, carry_key, st);
+  carry_chains<F>(offsets, Ktot, pl, b29, cr29, carry_key, st);
   CSK_CHECK_LAUNCH();
-  k_fixup<F><<<(Ktot + TB - 1) / TB, TB, 0, st>>>(offsets, Ktot, pl.L, b29, cr29);
-  k_merge_members<F><<<dim3((pl.B + TB - 1) / TB, count), TB, 0, st>>>(offsets, b29, Wt, pl.B, merged);
-  k_iota<<<(uint32_t)(((uint64_t)count * pl.B + 1 + 255) / 256), 256, 0, st>>>(iota, count * pl.B + 1);
+  if (per > 1) {
+    k_merge_members<F><<<dim3((pl.B + TB - 1) / TB, count), TB, 0, st>>>(offsets, b29, Wt, pl.B, merged);
+    k_iota<<<(uint32_t)(((uint64_t)count * pl.B + 1 + 255) / 256), 256, 0, st>>>(moff, count * pl.B + 1);
+  }
   CSK_CHECK_LAUNCH();
-  window_sums<F>(iota, merged, count, pl.B, Lrm, wsum, st);
+  window_sums<F>(moff, merged, count, pl.B, Lrm, wsum, st);
   k_final<F><<<count, kChainThreads, 0, st>>>(osegs, wsum, 1, pl.c);
   CSK_CHECK_LAUNCH();
   return CSK_OK;

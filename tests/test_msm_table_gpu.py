@@ -208,3 +208,19 @@ def test_run_multi_over_different_tables(g2, c):
         MsmTable.run_multi([tabs[0], other], [scl[0], scl[0]], outs[:2])
     for t in tabs + [other]:
         t.close()
+
+
+@pytest.mark.parametrize("g2,n", [(False, 1 << 20), (False, (1 << 20) + 1), (True, 1 << 20), (True, (1 << 20) + 1)])
+def test_joint_and_separate_windows(g2, n):
+    # c = 8 has 32 windows: 2^25 entries are the largest run whose windows are
+    # sorted together, one more tile takes a member per window
+    ctx = _capi.default_context()
+    k, sc = inputs.field_elements(61, n, nonzero=True), inputs.field_elements(62, n)
+    sc[: n // 2, 1:] = 0  # chains of carries in the low windows' buckets
+    d_k, ds = DeviceBuffer.from_array(ctx, k), DeviceBuffer.from_array(ctx, sc)
+    pts, out = DeviceBuffer(ctx, n * (128 if g2 else 64)), DeviceBuffer(ctx, 128)
+    fixed_base(d_k, n, pts, g2=g2)
+    t = MsmTable(pts, n, g2=g2, window_bits=8, ctx=ctx)
+    t.run(ds, out)
+    assert np.array_equal(out.download((32 if g2 else 16,)), gen_mul(dot_mod_r(k, sc), g2))
+    t.close()
