@@ -1,0 +1,44 @@
+// Entries per thread of the multiexp's bucket loops.
+#pragma once
+#include <stdint.h>
+
+namespace csk {
+
+// Sorted entries per accumulation thread, from the entries there are (digits that
+// are not 0; a witness has half as many as its size allows) and the buckets K: fixed
+// when the caller says so, otherwise what fills whole rounds of 2^17 threads, the two
+// waves per SIMD that the bucket loops run.  One round up to 2^23 entries, two up to
+// 2^26 (64 to 256 entries a thread), then as many as hold 256 entries a thread.  A
+// length rounded down leaves a last round nearly empty: 2.2M G1 points, 262687 threads
+// of 134 entries 4.00 ms, 3.44 by 135; 2^18 G2 points, 233017 threads of 18 entries
+// 2.00 ms, 1.88 by 32.  From 64 to 256 entries a round more or less makes 1%.  With K
+// below 2^17, where the fix-up adds up to eight carries a bucket itself, a bucket is to
+// span no more chunks than that (10000 G2 points, c = 11, 39 entries a bucket: 0.76 ms
+// by 4, 0.60 by 8), unless the threads are so few that a longer chunk is what is waited
+// for (a table of 500 G1 points, 125 entries a bucket: 267 us by 20, 220 by 8).  Chunks
+// below 8 entries make more carries than their threads are worth.
+struct ChunkLen {
+  uint32_t fixed, least;
+  static constexpr uint32_t rounds(uint32_t entries) {
+    return entries <= 1u << 23 ? 1 : entries <= 1u << 26 ? 2 : (entries + (1u << 25) - 1) >> 25;
+  }
+  constexpr uint32_t operator()(uint32_t entries, uint32_t K) const {
+    if (fixed) return fixed;
+    const uint32_t threads = rounds(entries) << 17;
+    uint32_t l = (entries + threads - 1) / threads;
+    if (l < least) l = least;
+    if (K < 1u << 17 && entries >> 16) {
+      const uint32_t span = (entries / 13 * 2 + K - 1) / K;
+      if (l < span) l = span;
+    }
+    return l;
+  }
+  // chunks of at most `entries` entries, however many there are
+  constexpr uint64_t most(uint32_t entries) const {
+    const uint64_t l = fixed ? fixed : least, n = (entries + l - 1) / l;
+    const uint64_t r = fixed ? n : (uint64_t)rounds(entries) << 17;
+    return n < r ? n : r;
+  }
+};
+
+}  // namespace csk

@@ -5,6 +5,7 @@
 #include <stddef.h>
 #include <string>
 #include <mutex>
+#include "chunk.h"
 #include "../../include/csk.h"
 
 namespace csk {
@@ -67,13 +68,14 @@ struct MsmPlan {
   uint32_t J;            // members
   uint32_t hb;           // bucket bits the sort's first pass bins by (the second takes the other c-1-hb)
   uint32_t st;           // low bucket bits the second pass sorts the top window by (<= c-1-hb)
-  uint32_t L;            // sorted entries per accumulation thread
+  ChunkLen chunk;        // sorted entries per accumulation thread
+  uint32_t L;            // the same with every digit nonzero
   uint32_t Lr;           // buckets per reduction thread
   uint32_t S;            // reduction segments per window, B / Lr
   uint64_t n;            // points over all members, E for each of the caller's
   uint64_t most;         // points of the largest member
   uint64_t max_entries;  // n * W (upper bound on nonzero digits)
-  uint64_t max_chunks;   // ceil(max_entries / L)
+  uint64_t max_chunks;   // chunks at most, whatever the digits
   uint64_t tiles;        // sum over members of ceil(n_j / 4096) (sort tiles per window)
 };
 

@@ -80,6 +80,14 @@ static uint32_t plan_top_bits(uint32_t bits, uint32_t c, uint32_t hb) {
   return t > hb ? t - hb : 0;
 }
 
+static void plan_chunks(MsmPlan &pl, uint32_t fixed) {
+  const uint64_t K = (uint64_t)pl.J * pl.K;
+  pl.chunk = {fixed, 8};
+  if (pl.max_entries >> 31 || K == 0 || K >> 32) return;  // a plan that msm_plan_ok refuses
+  pl.L = pl.chunk((uint32_t)pl.max_entries, (uint32_t)K);
+  pl.max_chunks = pl.chunk.most((uint32_t)pl.max_entries);
+}
+
 MsmPlan msm_group_plan(uint32_t c, uint32_t E, const uint64_t *n, uint32_t J, bool g2, uint32_t chunk,
                        uint32_t reduce_seg) {
   (void)g2;
@@ -99,12 +107,6 @@ MsmPlan msm_group_plan(uint32_t c, uint32_t E, const uint64_t *n, uint32_t J, bo
   pl.max_entries = pl.n * pl.W;
   pl.hb = plan_hi_bits(c, J ? pl.n / J : 0);
   pl.st = plan_top_bits(pl.bits, c, pl.hb);
-  // chunk length: aim for ~2^18 accumulation threads (a few waves per SIMD)
-  // so small inputs are not latency bound; at most 256 entries per thread
-  uint64_t l = pl.max_entries >> 18;
-  if (l < 8) l = 8;
-  if (l > 256) l = 256;
-  pl.L = chunk ? chunk : (uint32_t)l;
   // buckets per reduction thread: aim for ~2^15 reduction threads
   const uint64_t Ktot = (uint64_t)J * pl.K;
   uint32_t lr = 16;
@@ -114,7 +116,7 @@ MsmPlan msm_group_plan(uint32_t c, uint32_t E, const uint64_t *n, uint32_t J, bo
   if (lr > pl.B) lr = pl.B;
   pl.Lr = lr;
   pl.S = pl.B / pl.Lr;
-  pl.max_chunks = (pl.max_entries + pl.L - 1) / pl.L;
+  plan_chunks(pl, chunk);
   return pl;
 }
 
@@ -367,9 +369,9 @@ namespace csk {
 // entry for point w * n_pad + i), so that all of a bucket's entries are
 // adjacent.  As members of one window each, every window has its own copy of
 // the buckets, carried, fixed up and merged: at 100003 points, c = 16, 524288
-// buckets of 3 entries instead of 32768 of 49, 582 -> 449 us; 500 points
-// 411 -> 219, 2^20 1661 -> 1500, 2.2M (2^25 entries) 3267 -> 2993 us; G2 5000 868 ->
-// 454, 2^20 4828 -> 3999 us.  A member has at most 256 second-pass workgroups, so
+// buckets of 3 entries instead of 32768 of 49, 582 -> 410 us; 500 points
+// 411 -> 219, 2^20 1661 -> 1475, 2.2M (2^25 entries) 3267 -> 3002 us; G2 5000 868 ->
+// 455, 2^20 4828 -> 3999 us.  A member has at most 256 second-pass workgroups, so
 // larger runs keep the members: 2^22 points 5886 us joint, 5829 as members.
 static constexpr uint64_t kJointMax = 1ull << 25;
 static bool table_joint(uint64_t n_pad, uint32_t Wt) { return n_pad * Wt <= kJointMax; }
@@ -396,15 +398,9 @@ static MsmPlan table_plan(uint32_t c, const uint64_t *n_pad, uint32_t count, uin
   pl.max_entries = pl.n;
   pl.hb = plan_hi_bits(c, pl.n / pl.J);
   pl.st = plan_top_bits(pl.bits, c, pl.hb);
-  // two waves of chunks per SIMD: with few buckets a shorter chunk only makes
-  // more carries
-  uint64_t l = pl.max_entries >> (joint ? 17 : 18);
-  if (l < 8) l = 8;
-  if (l > 256) l = 256;
-  pl.L = (uint32_t)l;
   pl.Lr = pl.B < 16 ? pl.B : 16;
   pl.S = pl.B / pl.Lr;
-  pl.max_chunks = (pl.max_entries + pl.L - 1) / pl.L;
+  plan_chunks(pl, 0);
   return pl;
 }
 

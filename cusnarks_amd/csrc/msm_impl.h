@@ -716,14 +716,14 @@ __device__ __forceinline__ XYZZ29 inf29() { return {Fq29{}, f29_const(Q29::one),
 template <class F>
 __global__ void __launch_bounds__(256) k_accumulate29(const MsmSeg *__restrict__ segs, uint32_t Kj,
                                                       const uint32_t *__restrict__ sorted,
-                                                      const uint32_t *__restrict__ off, uint32_t K, uint32_t L,
+                                                      const uint32_t *__restrict__ off, uint32_t K, ChunkLen chunk,
                                                       const uint32_t *__restrict__ pts29,
                                                       uint32_t *__restrict__ buckets29,
                                                       uint32_t *__restrict__ carry29,
                                                       uint32_t *__restrict__ carry_key) {
   static_assert(std::is_same<F, Fq>::value, "29-bit limbs are for the base field");
   const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t E = off[K];
+  const uint32_t E = off[K], L = chunk(E, K);
   const uint64_t e0l = (uint64_t)t * L;
   if (e0l >= E) return;
   const uint32_t e0 = (uint32_t)e0l;
@@ -812,12 +812,12 @@ __device__ __forceinline__ void load2_29(const uint32_t *points, uint32_t v, Fq2
 template <class F>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 k_accumulate29_g2(const MsmSeg *__restrict__ segs, uint32_t Kj, const uint32_t *__restrict__ sorted,
-                  const uint32_t *__restrict__ off, uint32_t K, uint32_t L, const uint32_t *__restrict__ pts29,
+                  const uint32_t *__restrict__ off, uint32_t K, ChunkLen chunk, const uint32_t *__restrict__ pts29,
                   uint32_t *__restrict__ buckets29, uint32_t *__restrict__ carry29,
                   uint32_t *__restrict__ carry_key) {
   static_assert(std::is_same<F, Fq2>::value, "the G2 loop");
   const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t E = off[K];
+  const uint32_t E = off[K], L = chunk(E, K);
   const uint64_t e0l = (uint64_t)t * L;
   if (e0l >= E) return;
   const uint32_t e0 = (uint32_t)e0l;
@@ -912,23 +912,22 @@ template <> struct Acc29<Fq2> {
 // up to `keep` slots of its bucket's chain to the bucket: one with a lane per
 // bucket, where a second would keep whole waves for a few lanes (the G1 fix-up of a
 // 50000-constraint proof 113 -> 163 us), eight with a group per bucket, where the
-// buckets are few and their chains long.  Longer
-// chains are thinned first (a bucket far larger than a chunk: skewed digits,
-// small witness values, a narrow top window): in the round of step 8^r the slot
-// at chain index i (i % 8^(r+1) == 0) adds the slots at i + k*8^r, k = 1..7, that
+// buckets are few and their chains long.  Longer chains are thinned first (a
+// bucket far larger than a chunk: skewed digits, small witness values, a narrow top
+// window): in the round of step 8^r the slot at chain index i (i % 8^(r+1) == 0) adds the slots at i + k*8^r, k = 1..7, that
 // lie in the chain, if the chain has more than keep * 8^r of them.  The slots read
 // are never written in the same round.  Slots are 29-bit (SW words).
 // A group of lanes per slot (quad29.h): a round is a chain of up to seven
 // additions, and few slots of a round head one.
 template <class F>
-__global__ void __launch_bounds__(256) k_carry_round(const uint32_t *__restrict__ off, uint32_t K, uint32_t L,
+__global__ void __launch_bounds__(256) k_carry_round(const uint32_t *__restrict__ off, uint32_t K, ChunkLen chunk,
                                                      uint32_t *__restrict__ carry,
                                                      const uint32_t *__restrict__ carry_key, uint32_t step,
                                                      uint32_t keep) {
   constexpr int SW = Slot29<F>::SW;
   constexpr uint32_t GN = Grp<F>::N;
   const uint64_t u = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / GN;
-  const uint32_t E = off[K];
+  const uint32_t E = off[K], L = chunk(E, K);
   uint32_t i = 0, len = 0;
   if (u * L < E) {
     const uint32_t key = carry_key[u];
@@ -960,12 +959,13 @@ __global__ void __launch_bounds__(256) k_carry_round(const uint32_t *__restrict_
 // few, so one launch that looks for them costs less than a launch per round.
 static constexpr uint32_t kCarryTail = 64;
 template <class F>
-__global__ void __launch_bounds__(256) k_carry_tail(const uint32_t *__restrict__ off, uint32_t K, uint32_t L,
+__global__ void __launch_bounds__(256) k_carry_tail(const uint32_t *__restrict__ off, uint32_t K, ChunkLen chunk,
                                                     uint32_t *carry, const uint32_t *__restrict__ carry_key, uint32_t keep) {
   constexpr uint32_t SW = Slot29<F>::SW, GN = Grp<F>::N, NG = 64 / GN;
   const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t E = off[K], L = chunk(E, K);
   uint32_t len = 0;
-  if ((uint64_t)u * L < off[K]) {
+  if ((uint64_t)u * L < E) {
     const uint32_t key = carry_key[u];
     if (key != 0xFFFFFFFFu) {
       const uint32_t t0 = off[key] / L, t1 = (off[key + 1] - 1) / L;
@@ -1008,7 +1008,7 @@ static_assert(kCarryTail == 64, "chain_stride");
 
 // every bucket gets its chain: a lane per bucket, or (k_fixup_groups) a group
 template <class F>
-__global__ void __launch_bounds__(256) k_fixup(const uint32_t *__restrict__ off, uint32_t K, uint32_t L,
+__global__ void __launch_bounds__(256) k_fixup(const uint32_t *__restrict__ off, uint32_t K, ChunkLen chunk,
                                                uint32_t *__restrict__ buckets,
                                                const uint32_t *__restrict__ carry) {
   constexpr int SW = Slot29<F>::SW;
@@ -1017,7 +1017,7 @@ __global__ void __launch_bounds__(256) k_fixup(const uint32_t *__restrict__ off,
   if (key >= K) return;
   const uint32_t s = off[key], e = off[key + 1];
   if (e == s) return;
-  const uint32_t t0 = s / L, len = (e - 1) / L - t0;
+  const uint32_t L = chunk(off[K], K), t0 = s / L, len = (e - 1) / L - t0;
   if (len == 0) return;
   A acc, c;
   load29(buckets + (uint64_t)key * SW, acc);
@@ -1026,11 +1026,12 @@ __global__ void __launch_bounds__(256) k_fixup(const uint32_t *__restrict__ off,
   store29(buckets + (uint64_t)key * SW, acc);
 }
 template <class F>
-__global__ void __launch_bounds__(256) k_fixup_groups(const uint32_t *__restrict__ off, uint32_t K, uint32_t L,
+__global__ void __launch_bounds__(256) k_fixup_groups(const uint32_t *__restrict__ off, uint32_t K, ChunkLen chunk,
                                                       uint32_t *__restrict__ buckets,
                                                       const uint32_t *__restrict__ carry) {
   constexpr uint32_t SW = Slot29<F>::SW, GN = Grp<F>::N;
   const uint32_t key = (uint32_t)(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / GN);
+  const uint32_t L = chunk(off[K], K);
   uint32_t t0 = 0, len = 0;
   if (key < K) {
     const uint32_t s = off[key], e = off[key + 1];
@@ -1063,13 +1064,13 @@ static void carry_chains(const uint32_t *off, uint32_t K, const MsmPlan &pl, uin
   const bool lanes = K >= 1u << 17;
   const uint32_t keep = lanes ? 1 : 8;
   for (uint32_t step = 1; step < kCarryTail && keep * step < pl.max_chunks; step *= 8)
-    k_carry_round<F><<<grp_blocks<F>(pl.max_chunks), 256, 0, st>>>(off, K, pl.L, carry, carry_key, step, keep);
+    k_carry_round<F><<<grp_blocks<F>(pl.max_chunks), 256, 0, st>>>(off, K, pl.chunk, carry, carry_key, step, keep);
   if (pl.max_chunks > keep * kCarryTail)
-    k_carry_tail<F><<<(uint32_t)((pl.max_chunks + 255) / 256), 256, 0, st>>>(off, K, pl.L, carry, carry_key, keep);
+    k_carry_tail<F><<<(uint32_t)((pl.max_chunks + 255) / 256), 256, 0, st>>>(off, K, pl.chunk, carry, carry_key, keep);
   if (lanes)
-    k_fixup<F><<<(K + 127) / 128, 128, 0, st>>>(off, K, pl.L, buckets, carry);
+    k_fixup<F><<<(K + 127) / 128, 128, 0, st>>>(off, K, pl.chunk, buckets, carry);
   else
-    k_fixup_groups<F><<<grp_blocks<F>(K), 256, 0, st>>>(off, K, pl.L, buckets, carry);
+    k_fixup_groups<F><<<grp_blocks<F>(K), 256, 0, st>>>(off, K, pl.chunk, buckets, carry);
 }
 
 // ------------------------------------------------------------ window sums
@@ -1390,9 +1391,9 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
     uint32_t ga = (uint32_t)((pl.max_chunks + TB - 1) / TB);
     if (tm) tm->mark(1, st);
     if constexpr (std::is_same<F, Fq>::value)
-      k_accumulate29<F><<<ga, TB, 0, st>>>(segs, pl.K, sorted, offsets, Ktot, pl.L, pts29, b29, cr29, carry_key);
+      k_accumulate29<F><<<ga, TB, 0, st>>>(segs, pl.K, sorted, offsets, Ktot, pl.chunk, pts29, b29, cr29, carry_key);
     else
-      k_accumulate29_g2<F><<<ga, TB, 0, st>>>(segs, pl.K, sorted, offsets, Ktot, pl.L, pts29, b29, cr29, carry_key);
+      k_accumulate29_g2<F><<<ga, TB, 0, st>>>(segs, pl.K, sorted, offsets, Ktot, pl.chunk, pts29, b29, cr29, carry_key);
     CSK_CHECK_LAUNCH();
     if (tm) tm->mark(2, st);
     carry_chains<F>(offsets, Ktot, pl, b29, cr29, carry_key, st);
@@ -1627,9 +1628,9 @@ int msm_run_table(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArg
   const uint32_t TB = g2 ? 128 : 256;
   const uint32_t ga = (uint32_t)((pl.max_chunks + TB - 1) / TB);
   if constexpr (std::is_same<F, Fq>::value)
-    k_accumulate29<F><<<ga, TB, 0, st>>>(segs, pl.K, sorted, offsets, Ktot, pl.L, nullptr, b29, cr29, carry_key);
+    k_accumulate29<F><<<ga, TB, 0, st>>>(segs, pl.K, sorted, offsets, Ktot, pl.chunk, nullptr, b29, cr29, carry_key);
   else
-    k_accumulate29_g2<F><<<ga, TB, 0, st>>>(segs, pl.K, sorted, offsets, Ktot, pl.L, nullptr, b29, cr29,
+    k_accumulate29_g2<F><<<ga, TB, 0, st>>>(segs, pl.K, sorted, offsets, Ktot, pl.chunk, nullptr, b29, cr29,
                                              carry_key);
   CSK_CHECK_LAUNCH();
   carry_chains<F>(offsets, Ktot, pl, b29, cr29, carry_key, st);

@@ -60,7 +60,7 @@ def apply(ctx) -> list[str]:
 
 
 def default_chunk(n: int, c: int) -> int:
-    """The library's built-in chunk length for one multiexp of n points."""
+    """The chunk length the sweep starts from, for one multiexp of n points."""
     return max(8, min(256, (n * (254 // c + 1)) >> 18))
 
 
@@ -102,11 +102,11 @@ def autotune(g2: bool, lgs, ctx=None, reps: int = 3, log=print) -> dict:
             sweep[c] = _measure(ctx, g2, sc, pts, n, out, MsmCfg(c, 0, 0, 0), reps)
         c = min(sweep, key=sweep.get)
         l0 = default_chunk(n, c)
-        chunks = {}
-        for L in sorted({max(4, l0 // 2), l0, min(1024, 2 * l0)}):
+        chunks = {}  # 0: the library's own rule
+        for L in sorted({0, max(4, l0 // 2), l0, min(1024, 2 * l0)}):
             chunks[L] = _measure(ctx, g2, sc, pts, n, out, MsmCfg(c, L, 0, 0), reps)
         L = min(chunks, key=chunks.get)
-        classes[str(lg)] = {"window_bits": c, "chunk": L if L != l0 else 0, "reduce_seg": 0,
+        classes[str(lg)] = {"window_bits": c, "chunk": L, "reduce_seg": 0,
                             "n": n, "ms": round(chunks[L], 4),
                             "sweep_c_ms": {str(a): round(b, 4) for a, b in sweep.items()},
                             "sweep_chunk_ms": {str(a): round(b, 4) for a, b in chunks.items()}}

@@ -65,3 +65,26 @@ def test_scalar_split(tmp_path):
         assert (k1 + k2 * LAMBDA - k) % R == 0 and abs(k1) < 1 << 126 and abs(k2) < 1 << 126, hex(k)
         if k < 1 << 100:
             assert (k1, k2) == (k, 0)  # small scalars (most wire values) stay small
+
+
+@pytest.mark.parametrize("least", [4, 8])
+@pytest.mark.parametrize("buckets", [2, 128, 2048, 40960, (1 << 17) - 1, 1 << 17, 1 << 18, 3 << 20])
+def test_chunk_length(tmp_path, buckets, least):
+    # however many of a plan's entries there are, the chunks fit the slots it has
+    L = compiled(tmp_path, "chunk.h", "uint32_t len(uint32_t f, uint32_t l, uint32_t e, uint32_t k) "
+                                      "{ return csk::ChunkLen{f, l}(e, k); }\n"
+                                      'extern "C" uint64_t most(uint32_t f, uint32_t l, uint32_t e) '
+                                      "{ return csk::ChunkLen{f, l}.most(e); }")
+    L.len.restype, L.most.restype = ctypes.c_uint32, ctypes.c_uint64
+    rng = random.Random(buckets)
+    es = {0, 1, 2, 2**31 - 1}
+    for k in range(3, 32):
+        es |= {min(max(0, (m << k >> 1) + d), 2**31 - 1) for m in (2, 3) for d in (-2, -1, 0, 1, 2)}
+    es |= {rng.randrange(1 << rng.randrange(1, 32)) % 2**31 for _ in range(300)}
+    for fixed in (0, 1, 5, 300):
+        peak = 0
+        for e in sorted(es):
+            n = L.len(fixed, least, e, buckets)
+            assert n >= (fixed or least)
+            peak = max(peak, -(-e // n))
+            assert peak <= L.most(fixed, least, e), (e, n)
