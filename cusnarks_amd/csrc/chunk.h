@@ -14,9 +14,12 @@ namespace csk {
 // 2.00 ms, 1.88 by 32.  From 64 to 256 entries a round more or less makes 1%.  With K
 // below 2^17, where the fix-up adds up to eight carries a bucket itself, a bucket is to
 // span no more chunks than that (10000 G2 points, c = 11, 39 entries a bucket: 0.76 ms
-// by 4, 0.60 by 8), unless the threads are so few that a longer chunk is what is waited
-// for (a table of 500 G1 points, 125 entries a bucket: 267 us by 20, 220 by 8).  Chunks
-// below 8 entries make more carries than their threads are worth.
+// by 4, 0.60 by 8), in fewer rounds if need be (2^19 G2 points, c = 13: 4.00 ms in two
+// rounds of 40, 3.00 in one of 80), unless the threads are so few that a longer chunk
+// is what is waited for (a table of 500 G1 points, 125 entries a bucket: 267 us by 20,
+// 220 by 8).  Chunks below 8 entries make more carries than their threads are worth,
+// below 4 where a chunk's entry takes longest (5003 G2 points in quarters: 568 us by 3,
+// 539 by 4, 565 by 8).
 struct ChunkLen {
   uint32_t fixed, least;
   static constexpr uint32_t rounds(uint32_t entries) {
@@ -24,13 +27,13 @@ struct ChunkLen {
   }
   constexpr uint32_t operator()(uint32_t entries, uint32_t K) const {
     if (fixed) return fixed;
-    const uint32_t threads = rounds(entries) << 17;
-    uint32_t l = (entries + threads - 1) / threads;
+    const uint32_t span = K < 1u << 17 && entries >> 16 ? (entries / 13 * 2 + K - 1) / K : 1;
+    uint32_t r = rounds(entries);
+    if (r > entries / span >> 17) r = entries / span >> 17;
+    if (r == 0) r = 1;
+    uint32_t l = (entries + (r << 17) - 1) / (r << 17);
+    if (l < span) l = span;
     if (l < least) l = least;
-    if (K < 1u << 17 && entries >> 16) {
-      const uint32_t span = (entries / 13 * 2 + K - 1) / K;
-      if (l < span) l = span;
-    }
     return l;
   }
   // chunks of at most `entries` entries, however many there are

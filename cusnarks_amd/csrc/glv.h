@@ -18,18 +18,34 @@
 //   k1 = k - c1 s - c2 n2,  k2 = c1 n1 - c2 s,
 // at most (1/2 + 2^-33)(s + n2) < 2^126 in size.  c1 and c2 come from
 // products by round(2^288 s / r) and round(2^288 n1 / r).
+//
+// On the twist psi(x, y) = (conj(x) gx, conj(y) gy), the q-power Frobenius seen
+// through the twist (gx = (9 + u)^((q - 1) / 3), gy = (9 + u)^((q - 1) / 2)), is the
+// multiplication by mu = q mod r = 6 x^2, x the curve's parameter, and psi^2 = -phi:
+// k = k0 + k1 mu + k2 mu^2 + k3 mu^3 with |ki| < 2^64 (Galbraith and Scott,
+// "Exponentiation in pairing-friendly groups using homomorphisms", 2008).  A reduced
+// basis of the lattice of (a0, .., a3) with sum a_i mu^i = 0 mod r:
+//   (2x, x + 1, -x, x), (x, -x, x, 2x + 1), (x + 1, x, x, -2x), (2x + 1, -x, -x - 1, -x)
+// (k, 0, 0, 0) is the sum of the rows times k (6x^3 - x) / r, k (6x^3 + 6x^2 + 2x) / r,
+// k (6x^3 + 6x^2 + 4x + 1) / r and k (6x^3 + 6x^2 + x) / r.  Their nearest whole numbers
+// c_j leave k0 .. k3, at most half the sums of the columns: 0.81 2^64.
 #pragma once
 #include <stdint.h>
 
 namespace csk {
 
-// bits of a half (its size is below 2^kGlvBits) and of a whole scalar
-static constexpr uint32_t kGlvBits = 126, kScalarBits = 254;
+// bits of a half (its size is below 2^kGlvBits), of a quarter and of a whole scalar
+static constexpr uint32_t kGlvBits = 126, kGlsBits = 64, kScalarBits = 254;
 
 namespace glv_detail {
 struct K {
   static constexpr uint32_t g1[4] = {1857668884u, 3353392087u, 3642565422u, 2u};
   static constexpr uint32_t g2[6] = {2783153403u, 958312845u, 2054937044u, 2809385679u, 1288630292u, 2u};
+  static constexpr uint32_t h0[7] = {2099248942u, 2513771441u, 1190444457u, 4235297966u, 149281382u, 2967022483u, 2659201418u};
+  static constexpr uint32_t h1[7] = {893176993u, 853813032u, 771696917u, 2749716351u, 1437911675u, 2967022485u, 2659201418u};
+  static constexpr uint32_t h2[7] = {2750845877u, 4207205119u, 119295043u, 2749716354u, 1437911675u, 2967022485u, 2659201418u};
+  static constexpr uint32_t h3[7] = {587435050u, 3472084287u, 3245381501u, 2749716349u, 1437911675u, 2967022485u, 2659201418u};
+  static constexpr uint64_t x = 4965661367192848881ull;
   static constexpr uint32_t s[2] = {2496795619u, 2312316264u};
   static constexpr uint32_t n1[4] = {2102333736u, 2182200299u, 4005059068u, 1867350600u};
   static constexpr uint32_t n2[4] = {304162059u, 199549268u, 4005059069u, 1867350600u};
@@ -115,6 +131,36 @@ __device__ __forceinline__ uint32_t glv_split(const uint32_t *k, uint32_t *k1, u
   mul_add<4, 2, true>(k2, c2, K::s);
   const uint32_t a = size_sign(k1), b = size_sign(k2);
   return a | (b << 1);
+}
+
+// k < r (8 words) -> |k0| .. |k3| (2 words each); bit i of the result is set when
+// k_i is negative.  All modulo 2^128: c_j has up to 190 bits, but k_i is small.
+__device__ __forceinline__ uint32_t gls_split(const uint32_t *k, uint32_t (*o)[2]) {
+  using namespace glv_detail;
+  typedef unsigned __int128 u128;
+  uint32_t w[4][4];
+  mul_hi<7, 4>(k, K::h0, w[0]);
+  mul_hi<7, 4>(k, K::h1, w[1]);
+  mul_hi<7, 4>(k, K::h2, w[2]);
+  mul_hi<7, 4>(k, K::h3, w[3]);
+  auto u = [](const uint32_t *v) {
+    return ((u128)((uint64_t)v[3] << 32 | v[2]) << 64) | ((uint64_t)v[1] << 32 | v[0]);
+  };
+  const u128 c0 = u(w[0]), c1 = u(w[1]), c2 = u(w[2]), c3 = u(w[3]);
+  const u128 d = c0 - c1, e = c2 - c3;
+  uint32_t neg = 0;
+  auto put = [&](int i, u128 r) {
+    const bool n = (r >> 127) != 0;
+    const uint64_t v = n ? 0 - (uint64_t)r : (uint64_t)r;
+    o[i][0] = (uint32_t)v;
+    o[i][1] = (uint32_t)(v >> 32);
+    neg |= (uint32_t)n << i;
+  };
+  put(0, u(k) - (K::x * (c0 + c0 + c1 + c2 + c3 + c3) + c2 + c3));
+  put(1, 0 - (K::x * (d + e) + c0));
+  put(2, K::x * (d - e) + c3);
+  put(3, 0 - (K::x * (c0 + c1 + c1 - c2 - c2 - c3) + c1));
+  return neg;
 }
 
 }  // namespace csk

@@ -60,8 +60,8 @@ struct Carver {
 // [j*K, (j+1)*K); every stage runs once over the whole group.
 struct MsmPlan {
   uint32_t c;            // window bits
-  uint32_t E;            // scalars' parts: 2 with the scalars split along the endomorphism (glv.h), else 1
-  uint32_t bits;         // size of a part in bits: 126 or 254
+  uint32_t E;            // scalars' parts: 2, on G2 also 4, with the scalars split along the endomorphisms (glv.h), else 1
+  uint32_t bits;         // size of a part in bits: 126, 64 or 254
   uint32_t W;            // windows: floor(bits / c) + 1 signed-digit windows cover a part
   uint32_t B;            // buckets per window, 2^(c-1) (signed digits)
   uint32_t K;            // W * B bucket keys per member

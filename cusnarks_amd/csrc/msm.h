@@ -41,7 +41,7 @@ inline uint64_t msm_sortbuf_bytes(const MsmPlan &pl, bool g2) {
 
 uint32_t msm_choose_c(uint64_t n, bool g2, const csk_ctx *ctx, const csk_msm_cfg *cfg);
 // group plan for members of sizes n[0..J) sharing window width c, the scalars
-// taken whole or split (E = 1 or 2)
+// taken whole or split (E = 1, 2 or, on G2, 4)
 MsmPlan msm_group_plan(uint32_t c, uint32_t E, const uint64_t *n, uint32_t J, bool g2, uint32_t chunk,
                        uint32_t reduce_seg);
 // the plan a group runs by: split scalars, or whole ones where only their

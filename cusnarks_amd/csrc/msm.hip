@@ -8,8 +8,8 @@
 //
 // Pipeline (all on one stream, no host round trip):
 //   1. k_digits      one thread per point: k mod r, split in two halves along
-//                    the endomorphism (glv.h), signed c-bit digits of each for
-//                    W windows; (window, |digit|) -> bucket key; histogram.
+//                    the endomorphism (on G2 in four quarters, glv.h), signed
+//                    c-bit digits of each for W windows; (window, |digit|) -> bucket key; histogram.
 //   2. scan          exclusive prefix sum of the histogram -> bucket offsets.
 //   3. k_scatter     counting-sort placement of (point index | sign) by key.
 //   4. k_accumulate  each thread folds a fixed-length chunk of the sorted
@@ -42,15 +42,11 @@ uint32_t msm_choose_c(uint64_t n, bool g2, const csk_ctx *ctx, const csk_msm_cfg
   if (cfg && cfg->window_bits) return cfg->window_bits;
   const uint32_t lg = floor_log2(n);
   if (ctx && lg < 64 && ctx->tune[g2][lg].window_bits) return ctx->tune[g2][lg].window_bits;
-  // windows whose top window keeps most of its bits (126 = (W-1) c + t with t
-  // close to c): a narrow top window puts every point in a few buckets
-  uint32_t c;
-  if (lg <= 11) c = 8;
-  else if (lg <= 14) c = 13;
-  else if (lg <= 22) c = 16;
-  else c = 19;
-  if (g2 && c > 16) c = 16;
-  return c;
+  // windows whose top window keeps most of its bits (126, on G2 64 for c <= 13, is
+  // (W-1) c + t with t close to c): a narrow top window puts every point in a few
+  // buckets
+  if (g2) return lg <= 7 ? 5 : lg <= 13 ? 11 : lg <= 18 ? 13 : 16;
+  return lg <= 11 ? 8 : lg <= 14 ? 13 : lg <= 22 ? 16 : 19;
 }
 
 // Bits of the bucket index the sort's first pass bins by: the top 8 (at most
@@ -68,8 +64,8 @@ static uint32_t plan_hi_bits(uint32_t c, uint64_t n_avg) {
 }
 
 // Low bucket bits the second pass sorts the top window by.  That window
-// holds only the top t = bits mod c bits of a scalar or of its half (below
-// 2^bits, bits = 254 or 126), and its digit, at most 2^t <= 2^(c-1), has no
+// holds only the top t = bits mod c bits of a scalar or of its half or
+// quarter (below 2^bits, bits = 254, 126 or 64), and its digit, at most 2^t <= 2^(c-1), has no
 // carry out, so its buckets are below 2^t: its first pass bins by the top hb of those t bits
 // (all HB bins filled, as for the other windows) or, when t <= hb, by all of
 // them, and each of its first-pass bins is then a single bucket.  Binning it
@@ -82,7 +78,7 @@ static uint32_t plan_top_bits(uint32_t bits, uint32_t c, uint32_t hb) {
 
 static void plan_chunks(MsmPlan &pl, uint32_t fixed) {
   const uint64_t K = (uint64_t)pl.J * pl.K;
-  pl.chunk = {fixed, 8};
+  pl.chunk = {fixed, pl.E == 4 ? 4u : 8u};
   if (pl.max_entries >> 31 || K == 0 || K >> 32) return;  // a plan that msm_plan_ok refuses
   pl.L = pl.chunk((uint32_t)pl.max_entries, (uint32_t)K);
   pl.max_chunks = pl.chunk.most((uint32_t)pl.max_entries);
@@ -94,7 +90,7 @@ MsmPlan msm_group_plan(uint32_t c, uint32_t E, const uint64_t *n, uint32_t J, bo
   MsmPlan pl = {};
   pl.c = c;
   pl.E = E;
-  pl.bits = E == 2 ? kGlvBits : kScalarBits;
+  pl.bits = E == 4 ? kGlsBits : E == 2 ? kGlvBits : kScalarBits;
   pl.W = pl.bits / c + 1;
   pl.B = 1u << (c - 1);
   pl.K = pl.W * pl.B;
@@ -120,9 +116,18 @@ MsmPlan msm_group_plan(uint32_t c, uint32_t E, const uint64_t *n, uint32_t J, bo
   return pl;
 }
 
+// G2 scalars are taken in quarters where these have no more entries at the width
+// than halves have: they have half the buckets and half the doublings.  5003 points
+// 757 us in halves (c = 13), 538 in quarters (c = 11), 2^18 points 1.88 (c = 16) and
+// 1.78 ms (c = 13).  At other widths the top window of a quarter is a waste: c = 16,
+// 5 windows of 4 against 8 of 2 per scalar, 5.9 against 5.0 ms at 2^20 points.
 MsmPlan msm_split_plan(const MsmPlan &whole, const uint64_t *n, bool g2, uint32_t chunk, uint32_t reduce_seg) {
-  const MsmPlan pl = msm_group_plan(whole.c, 2, n, whole.J, g2, chunk, reduce_seg);
-  return msm_plan_ok(pl) ? pl : whole;
+  const MsmPlan half = msm_group_plan(whole.c, 2, n, whole.J, g2, chunk, reduce_seg);
+  if (g2) {
+    const MsmPlan quarter = msm_group_plan(whole.c, 4, n, whole.J, g2, chunk, reduce_seg);
+    if (quarter.max_entries <= half.max_entries && msm_plan_ok(quarter)) return quarter;
+  }
+  return msm_plan_ok(half) ? half : whole;
 }
 
 bool msm_plan_ok(const MsmPlan &pl) {

@@ -77,21 +77,59 @@ template <> struct Beta29<Fq2> {
                                     69340804u,  535036287u, 352865610u, 1478937u};
 };
 
+// psi of the twist, (x, y) -> (conj(x) gx, conj(y) gy) (glv.h): both components and
+// the first's negative
+struct Psi29 {
+  static constexpr uint32_t x0[9] = {77959568u, 116720857u, 200831163u, 387972444u, 449106301u,
+                                     79574741u, 198110247u, 444835091u, 2396851u};
+  static constexpr uint32_t x1[9] = {286535409u, 187804871u, 492312764u, 403373079u, 442701694u,
+                                     360078139u, 294614062u, 104485018u, 1269326u};
+  static constexpr uint32_t nx0[9] = {332884919u, 437214173u, 276443795u, 196420980u, 448858106u,
+                                      505219562u, 349697305u, 332955936u, 774554u};
+  static constexpr uint32_t y0[9] = {455018104u, 57932550u, 320278461u, 408777911u, 37819167u,
+                                     383878197u, 519288526u, 32534274u, 1918653u};
+  static constexpr uint32_t y1[9] = {430327765u, 436072363u, 496131354u, 220163167u, 145517765u,
+                                     530932250u, 323946238u, 161949718u, 1410845u};
+  static constexpr uint32_t ny0[9] = {492697295u, 496002479u, 156996497u, 175615513u, 323274328u,
+                                      200916107u, 28519026u, 208385841u, 1252753u};
+};
+
+__device__ __forceinline__ void store29(uint32_t *d, const Fq29 &v) {
+  uint32_t o[8];
+  pack29(canon29(v), o);
+  st8(d, o);
+}
+
 // the point in the 2^261 form (field29.h), packed words, component by
-// component; with E = 2 followed by phi of it
+// component; with E = 2 followed by phi of it; with E = 4 by psi, -psi^2 = phi and
+// -psi^3 of it
 template <class F, int E> __device__ __forceinline__ void store_point29(uint32_t *d, const uint32_t *comps) {
   constexpr int NC = FieldIO<F>::NW / 8, PW = 2 * FieldIO<F>::NW;  // components per coordinate, words per point
+  Fq29 v[2 * NC];
 #pragma unroll
   for (int k = 0; k < 2 * NC; k++) {
-    uint32_t in[8], o[8];
+    uint32_t in[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) in[i] = comps[8 * k + i];
-    const Fq29 v = mul29(unpack29(in), f29_const(Q29::to));
-    pack29(canon29(v), o);
-    st8(d + 8 * k, o);
-    if (E == 2) {
-      if (k < NC) pack29(canon29(mul29(v, f29_const(Beta29<F>::v))), o);
-      st8(d + PW + 8 * k, o);
+    v[k] = mul29(unpack29(in), f29_const(Q29::to));
+    store29(d + 8 * k, v[k]);
+    if (E > 1) {
+      Fq29 t = v[k];
+      if (k < NC) t = mul29(t, f29_const(Beta29<F>::v));
+      store29(d + (E / 2) * PW + 8 * k, t);
+    }
+  }
+  if constexpr (E == 4) {
+    const Fq29 s[4] = {dot29(v[0], f29_const(Psi29::x0), v[1], f29_const(Psi29::x1)),
+                       dot29(v[0], f29_const(Psi29::x1), v[1], f29_const(Psi29::nx0)),
+                       dot29(v[2], f29_const(Psi29::y0), v[3], f29_const(Psi29::y1)),
+                       dot29(v[2], f29_const(Psi29::y1), v[3], f29_const(Psi29::ny0))};
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      store29(d + PW + 8 * k, s[k]);
+      Fq29 t = s[k];
+      if (k < 2) t = mul29(t, f29_const(Beta29<F>::v));
+      store29(d + 3 * PW + 8 * k, t);
     }
   }
 }
@@ -122,8 +160,12 @@ template <int E> __device__ __forceinline__ void store_point29(uint32_t *d, cons
 // whether d is negative.
 template <int NW> struct Digits {
   uint32_t k[NW + 1];
-  uint32_t c, B, mask, carry = 0;
-  __device__ __forceinline__ Digits(const uint32_t *v, uint32_t c_) : c(c_), B(1u << (c_ - 1)), mask((1u << c_) - 1) {
+  uint32_t c, B, mask, carry;
+  __device__ __forceinline__ void set(const uint32_t *v, uint32_t c_) {
+    c = c_;
+    B = 1u << (c - 1);
+    mask = (1u << c) - 1;
+    carry = 0;
 #pragma unroll
     for (int i = 0; i < NW; i++) k[i] = v[i];
     k[NW] = 0;
@@ -141,7 +183,8 @@ template <int NW> struct Digits {
 
 // One workgroup per (member j, tile) of kSortTile points, E of them for each of
 // the caller's (E = 2: P_i and phi(P_i) with the halves of k_i, glv.h; points
-// 2i and 2i + 1 of the member); block b covers the tiles in member order
+// 2i and 2i + 1 of the member; E = 4 on G2: P_i, psi(P_i) and so on with the
+// quarters); block b covers the tiles in member order
 // (member j's tiles start at b = tbase_j / W).  Member j's digits occupy
 // D[W*pbase_j + w*n_j + i], b | neg << 31 for the nonzero signed digit d of
 // window w (b = |d| - 1 < B), or 0xFFFFFFFF when d == 0 or the point is at
@@ -153,7 +196,9 @@ template <int NW> struct Digits {
 //
 // Splitting halves the windows and doubles the points: as many entries, half
 // the buckets to reduce and half the doublings of the window combination, for
-// one product more per point and the second point's 64 B (128 B on G2) here.
+// one product more per point and the second point's 64 B (128 B on G2) here.  G2's
+// quarters halve them again for 14 products and 256 B more a point (5003 points: 46
+// -> 55 us here, 757 -> 538 us in all).
 template <class F, int E>
 __global__ void __launch_bounds__(1024) k_digits(const MsmSeg *__restrict__ segs, uint32_t J, uint32_t c,
                                                  uint32_t W, uint32_t s, uint32_t ts, uint32_t HB,
@@ -182,23 +227,26 @@ __global__ void __launch_bounds__(1024) k_digits(const MsmSeg *__restrict__ segs
       if (live) atomicAdd(&hist[w * HB + (b >> (w == W - 1 ? ts : s))], 1u);
       return live ? b | ((uint32_t)neg << 31) : 0xFFFFFFFFu;
     };
-    if constexpr (E == 2) {
-      uint32_t k1[4], k2[4];
-      const uint32_t sg = glv_split(k, k1, k2);
-      Digits<4> d1(k1, c), d2(k2, c);
-      for (uint32_t w = 0; w < W; w++) {
-        bool n1, n2;
-        const uint32_t b1 = d1.take(n1), b2 = d2.take(n2);
-        *reinterpret_cast<uint2 *>(dj + (uint64_t)w * n + 2 * i) =
-            make_uint2(entry(w, b1, n1 != (bool)(sg & 1)), entry(w, b2, n2 != (bool)(sg >> 1)));
-      }
-    } else {
-      Digits<8> d(k, c);
-      for (uint32_t w = 0; w < W; w++) {
+    uint32_t parts[E][8 / E], sg = 0;
+    if constexpr (E == 4) sg = gls_split(k, parts) ^ 12u;  // points 2 and 3 are -psi^2 and -psi^3
+    else if constexpr (E == 2) sg = glv_split(k, parts[0], parts[1]);
+    else
+      for (int e = 0; e < 8; e++) parts[0][e] = k[e];
+    Digits<8 / E> d[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) d[e].set(parts[e], c);
+    for (uint32_t w = 0; w < W; w++) {
+      uint32_t o[E];
+#pragma unroll
+      for (int e = 0; e < E; e++) {
         bool neg;
-        const uint32_t b = d.take(neg);
-        dj[(uint64_t)w * n + i] = entry(w, b, neg);
+        const uint32_t b = d[e].take(neg);
+        o[e] = entry(w, b, neg != (bool)((sg >> e) & 1));
       }
+      uint32_t *q = dj + (uint64_t)w * n + E * i;
+      if constexpr (E == 4) *reinterpret_cast<uint4 *>(q) = make_uint4(o[0], o[1], o[2], o[3]);
+      else if constexpr (E == 2) *reinterpret_cast<uint2 *>(q) = make_uint2(o[0], o[1]);
+      else *q = o[0];
     }
   }
   __syncthreads();
@@ -1377,12 +1425,10 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
   if (pl.n > 0) {
     // few tiles leave most of the GPU idle: more threads share a tile's points
     const uint32_t DT = pl.tiles >= 1024 ? 256 : 1024;
-    if (pl.E == 2)
-      k_digits<F, 2><<<(uint32_t)pl.tiles, DT, pl.W * HB * 4, st>>>(segs, pl.J, pl.c, pl.W, sb, pl.st, HB, digits,
-                                                                    cnt, pts29);
-    else
-      k_digits<F, 1><<<(uint32_t)pl.tiles, DT, pl.W * HB * 4, st>>>(segs, pl.J, pl.c, pl.W, sb, pl.st, HB, digits,
-                                                                    cnt, pts29);
+    auto *kd = pl.E == 2 ? k_digits<F, 2> : k_digits<F, 1>;
+    if constexpr (std::is_same<F, Fq2>::value)
+      if (pl.E == 4) kd = k_digits<F, 4>;
+    kd<<<(uint32_t)pl.tiles, DT, pl.W * HB * 4, st>>>(segs, pl.J, pl.c, pl.W, sb, pl.st, HB, digits, cnt, pts29);
     CSK_CHECK_LAUNCH();
     scan_counts(cnt, ncnt, bsum, st);
     sort_place(pl, pl.W, digits, segs, cnt, tix, tlo, offsets, sorted, st);
@@ -1483,7 +1529,8 @@ __global__ void __launch_bounds__(256) k_digits_tab(TabArgs args, const MsmSeg *
     ld8(k, scalars + i * 8);
     reduce_mod_r(k);
     const bool zero = ((live[i >> 5] >> (i & 31)) & 1u) == 0;
-    Digits<8> d(k, c);
+    Digits<8> d;
+    d.set(k, c);
     for (uint32_t w = 0; w < Wt; w++) {
       bool neg;
       const uint32_t b = d.take(neg);

@@ -88,3 +88,24 @@ def test_chunk_length(tmp_path, buckets, least):
             assert n >= (fixed or least)
             peak = max(peak, -(-e // n))
             assert peak <= L.most(fixed, least, e), (e, n)
+def test_quarter_scalars(tmp_path):
+    L = compiled(tmp_path, "glv.h", "uint32_t split(const uint32_t *k, uint32_t *o) "
+                                    "{ return csk::gls_split(k, (uint32_t(*)[2])o); }")
+    x = 4965661367192848881
+    mu = Q % R
+    assert mu == 6 * x * x and pow(mu, 2, R) == R - LAMBDA
+    rng = random.Random(7)
+    ks = [0, 1, 2, R - 1, R - 2, R // 2, R // 2 + 1, R // 3, mu, mu - 1, mu + 1, R - mu, pow(mu, 3, R), (1 << 253)]
+    ks += [rng.randrange(R) for _ in range(5000)] + [rng.randrange(1 << rng.randrange(1, 253)) for _ in range(500)]
+    # where a multiple of a basis vector is half way between two whole numbers
+    for a in (6 * x**3 - x, 6 * x**3 + 6 * x**2 + 2 * x, 6 * x**3 + 6 * x**2 + 4 * x + 1, 6 * x**3 + 6 * x**2 + x):
+        ks += [v for c in (0, 1, 12345, a // 2, a - 1) for d in range(-2, 3) for v in [(2 * c + 1) * R // (2 * a) + d]
+               if 0 <= v < R]
+    for k in ks:
+        o = W8()
+        neg = L.split(words(k), o)
+        v = [int(o[2 * i]) | int(o[2 * i + 1]) << 32 for i in range(4)]
+        v = [-t if neg >> i & 1 else t for i, t in enumerate(v)]
+        assert (sum(t * pow(mu, i, R) for i, t in enumerate(v)) - k) % R == 0, hex(k)
+        if k < 1 << 63:
+            assert v == [k, 0, 0, 0]
