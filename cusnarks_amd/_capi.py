@@ -55,6 +55,7 @@ _SIGS = {
     "csk_stream_sync": ([P, P], INT),
     "csk_host_alloc": ([P, ctypes.POINTER(P), U64], INT),
     "csk_host_free": ([P, P], INT),
+    "csk_msm_multi": ([P, INT, U32, P, P, P, P, P], INT),
     "csk_msm_g1": ([P, P, P, U64, P, P, P], INT),
     "csk_msm_g2": ([P, P, P, U64, P, P, P], INT),
     "csk_msm_g1_host": ([P, P, P, U64, P, P], INT),

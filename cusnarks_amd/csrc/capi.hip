@@ -475,6 +475,14 @@ int csk_event_elapsed(csk_ctx *ctx, void *start, void *end, float *ms) {
   return CSK_OK;
 }
 
+int csk_msm_multi(csk_ctx *ctx, int ec2, uint32_t count, const uint32_t *const *d_scalars,
+                  const uint32_t *const *d_points, const uint64_t *n, uint32_t *const *d_out, void *stream) {
+  if (!ctx || !count || count > 64 || !d_scalars || !d_points || !n || !d_out) {
+    set_error("msm_multi: null argument or more than 64 members");
+    return CSK_ERR_ARG;
+  }
+  return csk::msm_multi(ctx, ec2 != 0, count, d_scalars, d_points, n, d_out, (hipStream_t)stream);
+}
 int csk_msm_g1(csk_ctx *ctx, const uint32_t *d_scalars, const uint32_t *d_points, uint64_t n, uint32_t *d_out,
                const csk_msm_cfg *cfg, void *stream) {
   if (!ctx) return CSK_ERR_ARG;

@@ -43,6 +43,17 @@ def msm_device(d_scalars, d_points, n: int, d_out, g2: bool = False, ctx=None, s
     check(fn(ctx.ptr, dptr(d_scalars), dptr(d_points), int(n), dptr(d_out), _cfg(**cfg), stream), "csk_msm")
 
 
+def msm_multi(members, g2: bool = False, ctx=None, stream=None) -> None:
+    """Enqueue several multiexps, members = [(scalars, points, n, out), ...] on the
+    device (no synchronisation)."""
+    ctx = ctx or _capi.default_context()
+    k = len(members)
+    s, p, o = ((ctypes.c_void_p * k)(*[dptr(m[i]) or None for m in members]) for i in (0, 1, 3))
+    n = (ctypes.c_uint64 * k)(*[int(m[2]) for m in members])
+    check(lib().csk_msm_multi(ctx.ptr, int(bool(g2)), k, ctypes.cast(s, P), ctypes.cast(p, P), ctypes.cast(n, P),
+                              ctypes.cast(o, P), stream), "csk_msm_multi")
+
+
 def fixed_base(d_scalars, n: int, d_out, g2: bool = False, ctx=None, stream=None) -> None:
     """k_i * G for the G1 generator (1, 2) or the standard G2 generator."""
     ctx = ctx or _capi.default_context()

@@ -27,7 +27,7 @@ import numpy as np
 from . import _capi, inputs
 from ._capi import P, check, lib
 from .device import DeviceBuffer
-from .msm import fixed_base, msm_device
+from .msm import fixed_base, msm_device, msm_multi
 from .poly import interpolandmul_batch_device, interpolandmul_device, mpoly_eval_device, upload_csr
 from .synth import Circuit, KeyScalars
 
@@ -254,9 +254,10 @@ class ProofSlot:
 
 class GrothProver:
     """Plain per-request prover: every stage through the single-call entry
-    points, one after the other on one context and stream.  With the key's
-    fixed-base tables built (ProvingKey.build_tables) the five multiexps run
-    from them; the proof is the same."""
+    points, one after the other on one context and stream, but for the four G1
+    multiexps, which run as one call where their stages are not timed.  With the
+    key's fixed-base tables built (ProvingKey.build_tables) the five multiexps
+    run from them; the proof is the same."""
 
     def __init__(self, pk: ProvingKey, ctx=None, stream=None):
         self.pk = pk
@@ -283,6 +284,8 @@ class GrothProver:
         if tabs:
             self.pk.run_g1_tables(sl.g1_members(), ctx=c, stream=st)
             mark("msm_g1")
+        elif not timed:
+            msm_multi(sl.g1_members(), ctx=c, stream=st)
         else:
             for name, (ds, dp, n, do) in zip(names, sl.g1_members()):
                 msm_device(ds, dp, n, do, ctx=c, stream=st)

@@ -1,0 +1,45 @@
+"""csk_msm_multi: several multiexps in one call equal the single calls, bit for
+bit: members of one width and of several, more than a group holds, empty ones
+and members that overlap in scalars and points."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from cusnarks_amd import _capi, inputs
+from cusnarks_amd.device import DeviceBuffer
+from cusnarks_amd.msm import fixed_base, msm_device, msm_multi
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("g2", [False, True])
+@pytest.mark.parametrize("sizes", [
+    [1], [4, 1], [0, 5, 0, 7], [300, 4096, 4097, 2048, 2047],  # several widths
+    [50] * 17,                                                 # three groups
+    [9000, 12000, 8192, 16383],                                # a prover's four of one width
+])
+def test_multi_equals_single_calls(g2, sizes):
+    ctx = _capi.default_context()
+    nw, n = 32 if g2 else 16, max(sizes) + 8
+    pts = DeviceBuffer(ctx, n * nw * 4)
+    fixed_base(DeviceBuffer.from_array(ctx, inputs.field_elements(71, n, nonzero=True)), n, pts, g2=g2)
+    k = inputs.field_elements(72, n)
+    k[: n // 2, 1:] = 0
+    sc = DeviceBuffer.from_array(ctx, k)
+    outs, want = (DeviceBuffer(ctx, len(sizes) * nw * 4) for _ in range(2))
+    members = [(sc.ptr + (i % 8) * 32, pts.ptr + (i % 3) * nw * 4, m, outs.ptr + i * nw * 4) for i, m in enumerate(sizes)]
+    msm_multi(members, g2=g2)
+    for i, (s, p, m, _) in enumerate(members):
+        msm_device(s, p, m, want.ptr + i * nw * 4, g2=g2)
+    shape = (len(sizes), nw)
+    assert np.array_equal(outs.download(shape), want.download(shape))
+
+
+def test_refused():
+    ctx, L = _capi.default_context(), _capi.lib()
+    none = (ctypes.c_void_p * 65)()
+    n = (ctypes.c_uint64 * 65)(*[1] * 65)
+    p, q = ctypes.cast(none, _capi.P), ctypes.cast(n, _capi.P)
+    for count in (0, 1, 65):  # no member, null members, too many
+        assert L.csk_msm_multi(ctx.ptr, 0, count, p, p, q, p, None) != 0
