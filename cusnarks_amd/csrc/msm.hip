@@ -272,6 +272,20 @@ static bool multi_group(csk_ctx *ctx, bool g2, uint32_t c, uint32_t count, const
   return true;
 }
 
+// Width of a group of `count` G1 multiexps of n points in all, which single calls would
+// run at width c.  These weigh the buckets' reduction, which waits for chains of
+// additions, against launches and chains that a group shares; its cost is the work,
+// an addition per entry and about 2.8 per bucket, of 126 / c + 1 windows.  The four of
+// a 50000-constraint proof are at 3 entries a bucket by 16 and 25 by 13: 923 -> 791 us;
+// from 150000 points each 16 is the least again.
+static uint32_t multi_width(uint32_t c, uint32_t count, uint64_t n) {
+  auto work = [&](uint32_t w) { return (kGlvBits / w + 1) * (20 * n + 14ull * count * (1u << w)); };
+  uint32_t best = c;
+  for (uint32_t w : {16u, 13u, 8u})
+    if (w < c && work(w) < work(best)) best = w;
+  return best;
+}
+
 // The members a single call would give the same width run as one group: a stage is
 // one launch over all of them, and their window combinations, a chain of 126
 // doublings and an inversion that one workgroup each waits for, run side by side.
@@ -300,7 +314,7 @@ int msm_multi(csk_ctx *ctx, bool g2, uint32_t count, const uint32_t *const *scal
       go[k++] = out[j];
     }
     int rc = CSK_OK;
-    if (k > 1 && idx[0] == i && multi_group(ctx, g2, c, k, gn, gs, gp, go, st, &rc)) {
+    if (k > 1 && idx[0] == i && multi_group(ctx, g2, g2 ? c : multi_width(c, k, total), k, gn, gs, gp, go, st, &rc)) {
       for (uint32_t j = 0; j < k; j++) done |= 1ull << idx[j];
     } else {
       done |= 1ull << i;
