@@ -48,6 +48,7 @@ MsmPlan msm_group_plan(uint32_t c, uint32_t E, const uint64_t *n, uint32_t J, bo
 // entries fit the index range; whole is the plan with E = 1
 MsmPlan msm_split_plan(const MsmPlan &whole, const uint64_t *n, bool g2, uint32_t chunk, uint32_t reduce_seg);
 bool msm_plan_ok(const MsmPlan &pl);
+uint32_t multi_width(uint32_t c, uint32_t count, uint64_t n);
 int msm_multi(csk_ctx *ctx, bool g2, uint32_t count, const uint32_t *const *scalars, const uint32_t *const *points,
               const uint64_t *n, uint32_t *const *out, hipStream_t st);
 size_t msm_workspace_bytes(const MsmPlan &pl, bool g2);

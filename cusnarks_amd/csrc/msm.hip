@@ -278,7 +278,7 @@ static bool multi_group(csk_ctx *ctx, bool g2, uint32_t c, uint32_t count, const
 // an addition per entry and about 2.8 per bucket, of 126 / c + 1 windows.  The four of
 // a 50000-constraint proof are at 3 entries a bucket by 16 and 25 by 13: 923 -> 791 us;
 // from 150000 points each 16 is the least again.
-static uint32_t multi_width(uint32_t c, uint32_t count, uint64_t n) {
+uint32_t multi_width(uint32_t c, uint32_t count, uint64_t n) {
   auto work = [&](uint32_t w) { return (kGlvBits / w + 1) * (20 * n + 14ull * count * (1u << w)); };
   uint32_t best = c;
   for (uint32_t w : {16u, 13u, 8u})
