@@ -199,29 +199,43 @@ template <int NW> struct Digits {
 // one product more per point and the second point's 64 B (128 B on G2) here.  G2's
 // quarters halve them again for 14 products and 256 B more a point (5003 points: 46
 // -> 55 us here, 757 -> 538 us in all).
+//
+// The first `tiles` workgroups do this.  With more in the launch, the others write the
+// points, a thread each, and the first only the digits: few tiles leave most of the
+// CUs idle, and the products of 4096 points keep one CU's matter of 20 us and more.
 template <class F, int E>
 __global__ void __launch_bounds__(1024) k_digits(const MsmSeg *__restrict__ segs, uint32_t J, uint32_t c,
-                                                 uint32_t W, uint32_t s, uint32_t ts, uint32_t HB,
+                                                 uint32_t W, uint32_t s, uint32_t ts, uint32_t HB, uint32_t tiles,
                                                  uint32_t *__restrict__ digits, uint32_t *__restrict__ cnt,
                                                  uint32_t *__restrict__ pts29) {
   extern __shared__ uint32_t hist[];  // W * HB counters
+  constexpr uint32_t TS = kSortTile / E;  // scalars of a tile
+  constexpr int PW = 2 * FieldIO<F>::NW;
+  const bool both = gridDim.x == tiles;
+  if (blockIdx.x >= tiles) {
+    const uint32_t u = (blockIdx.x - tiles) * blockDim.x + threadIdx.x, g = u / TS;
+    const uint32_t j = member_of_tile(segs, J, W * g);
+    const uint64_t i = (uint64_t)(g - segs[j].tbase / W) * TS + u % TS;
+    if (E * i < segs[j].n)
+      store_point29<E>(pts29 + (segs[j].pbase + E * i) * PW, load_affine<F>(segs[j].points + i * PW));
+    return;
+  }
   const uint32_t j = member_of_tile(segs, J, W * blockIdx.x);
   const uint32_t tile = blockIdx.x - segs[j].tbase / W;
   const uint64_t pbase = segs[j].pbase, n = segs[j].n;
   const uint32_t NT = segs[j].NT;
   for (uint32_t i = threadIdx.x; i < W * HB; i += blockDim.x) hist[i] = 0;
   __syncthreads();
-  constexpr int PW = 2 * FieldIO<F>::NW;
   uint32_t *dj = digits + W * pbase;
-  for (uint32_t t = threadIdx.x; t < kSortTile / E; t += blockDim.x) {
-    const uint64_t i = (uint64_t)tile * (kSortTile / E) + t;
+  for (uint32_t t = threadIdx.x; t < TS; t += blockDim.x) {
+    const uint64_t i = (uint64_t)tile * TS + t;
     if (E * i >= n) break;
     uint32_t k[8];
     ld8(k, segs[j].scalars + i * 8);
     reduce_mod_r(k);
     const Affine<F> p = load_affine<F>(segs[j].points + i * PW);
     const bool zero = affine_is_inf(p);
-    store_point29<E>(pts29 + (pbase + E * i) * PW, p);
+    if (both) store_point29<E>(pts29 + (pbase + E * i) * PW, p);
     auto entry = [&](uint32_t w, uint32_t b, bool neg) -> uint32_t {
       const bool live = b != 0xFFFFFFFFu && !zero;
       if (live) atomicAdd(&hist[w * HB + (b >> (w == W - 1 ? ts : s))], 1u);
@@ -1423,12 +1437,15 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
 
   if (tm) tm->mark(0, st);
   if (pl.n > 0) {
-    // few tiles leave most of the GPU idle: more threads share a tile's points
-    const uint32_t DT = pl.tiles >= 1024 ? 256 : 1024;
+    // few tiles leave most of the GPU idle: more threads share a tile's points, and
+    // below 128 tiles other workgroups convert them: 5003 G2 points (5 tiles) 540 ->
+    // 509 us, 20011 G1 points (10) 465 -> 456, 200000 (98) 695 -> 689
+    const uint32_t tiles = (uint32_t)pl.tiles, DT = tiles >= 1024 ? 256 : tiles >= 128 ? 1024 : 512;
+    const uint32_t conv = tiles >= 128 ? 0 : tiles * (kSortTile / pl.E / DT);
     auto *kd = pl.E == 2 ? k_digits<F, 2> : k_digits<F, 1>;
     if constexpr (std::is_same<F, Fq2>::value)
       if (pl.E == 4) kd = k_digits<F, 4>;
-    kd<<<(uint32_t)pl.tiles, DT, pl.W * HB * 4, st>>>(segs, pl.J, pl.c, pl.W, sb, pl.st, HB, digits, cnt, pts29);
+    kd<<<tiles + conv, DT, pl.W * HB * 4, st>>>(segs, pl.J, pl.c, pl.W, sb, pl.st, HB, tiles, digits, cnt, pts29);
     CSK_CHECK_LAUNCH();
     scan_counts(cnt, ncnt, bsum, st);
     sort_place(pl, pl.W, digits, segs, cnt, tix, tlo, offsets, sorted, st);
