@@ -200,10 +200,10 @@ template <int NW> struct Digits {
 // quarters halve them again for 14 products and 256 B more a point (5003 points: 46
 // -> 55 us here, 757 -> 538 us in all).
 //
-// The first `tiles` workgroups do this.  With more in the launch, the others write the
-// points, a thread each, and the first only the digits: few tiles leave most of the
-// CUs idle, and the products of 4096 points keep one CU's matter of 20 us and more.
-template <class F, int E>
+// APART: the first `tiles` workgroups write only the digits and others the points, a
+// thread each.  Few tiles leave most of the CUs idle, and the products of 4096 points
+// keep one CU for 20 us and more.
+template <class F, int E, bool APART>
 __global__ void __launch_bounds__(1024) k_digits(const MsmSeg *__restrict__ segs, uint32_t J, uint32_t c,
                                                  uint32_t W, uint32_t s, uint32_t ts, uint32_t HB, uint32_t tiles,
                                                  uint32_t *__restrict__ digits, uint32_t *__restrict__ cnt,
@@ -211,8 +211,7 @@ __global__ void __launch_bounds__(1024) k_digits(const MsmSeg *__restrict__ segs
   extern __shared__ uint32_t hist[];  // W * HB counters
   constexpr uint32_t TS = kSortTile / E;  // scalars of a tile
   constexpr int PW = 2 * FieldIO<F>::NW;
-  const bool both = gridDim.x == tiles;
-  if (blockIdx.x >= tiles) {
+  if (APART && blockIdx.x >= tiles) {
     const uint32_t u = (blockIdx.x - tiles) * blockDim.x + threadIdx.x, g = u / TS;
     const uint32_t j = member_of_tile(segs, J, W * g);
     const uint64_t i = (uint64_t)(g - segs[j].tbase / W) * TS + u % TS;
@@ -235,7 +234,7 @@ __global__ void __launch_bounds__(1024) k_digits(const MsmSeg *__restrict__ segs
     reduce_mod_r(k);
     const Affine<F> p = load_affine<F>(segs[j].points + i * PW);
     const bool zero = affine_is_inf(p);
-    if (both) store_point29<E>(pts29 + (pbase + E * i) * PW, p);
+    if (!APART) store_point29<E>(pts29 + (pbase + E * i) * PW, p);
     auto entry = [&](uint32_t w, uint32_t b, bool neg) -> uint32_t {
       const bool live = b != 0xFFFFFFFFu && !zero;
       if (live) atomicAdd(&hist[w * HB + (b >> (w == W - 1 ? ts : s))], 1u);
@@ -266,6 +265,12 @@ __global__ void __launch_bounds__(1024) k_digits(const MsmSeg *__restrict__ segs
   __syncthreads();
   const uint32_t cb = segs[j].cbase + tile;
   for (uint32_t i = threadIdx.x; i < W * HB; i += blockDim.x) cnt[cb + (uint64_t)i * NT] = hist[i];
+}
+
+template <class F, bool APART> static auto digits_kernel(uint32_t E) {
+  if constexpr (std::is_same<F, Fq2>::value)
+    if (E == 4) return k_digits<F, 4, APART>;
+  return E == 2 ? k_digits<F, 2, APART> : k_digits<F, 1, APART>;
 }
 
 namespace {  // curve-independent kernels: one private copy per translation unit
@@ -1442,9 +1447,7 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
     // 509 us, 20011 G1 points (10) 465 -> 456, 200000 (98) 695 -> 689
     const uint32_t tiles = (uint32_t)pl.tiles, DT = tiles >= 1024 ? 256 : tiles >= 128 ? 1024 : 512;
     const uint32_t conv = tiles >= 128 ? 0 : tiles * (kSortTile / pl.E / DT);
-    auto *kd = pl.E == 2 ? k_digits<F, 2> : k_digits<F, 1>;
-    if constexpr (std::is_same<F, Fq2>::value)
-      if (pl.E == 4) kd = k_digits<F, 4>;
+    auto *kd = conv ? digits_kernel<F, true>(pl.E) : digits_kernel<F, false>(pl.E);
     kd<<<tiles + conv, DT, pl.W * HB * 4, st>>>(segs, pl.J, pl.c, pl.W, sb, pl.st, HB, tiles, digits, cnt, pts29);
     CSK_CHECK_LAUNCH();
     scan_counts(cnt, ncnt, bsum, st);

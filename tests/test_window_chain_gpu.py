@@ -87,3 +87,15 @@ def test_wire_value_scalars(n, g2):
     for c in (0, 9):
         msm_device(d_s, pts, n, out, g2=g2, window_bits=c)
         assert np.array_equal(out.download((32 if g2 else 16,)), want)
+
+
+@pytest.mark.parametrize("g2,n", [(False, 127 * 2048), (False, 127 * 2048 + 1), (True, 127 * 1024), (True, 127 * 1024 + 1)])
+def test_points_converted_apart(g2, n):
+    # 127 sort tiles: other workgroups write the points; 128: the digits' own
+    ctx = _capi.default_context()
+    k, sc = inputs.field_elements(52, n, nonzero=True), inputs.field_elements(53, n)
+    d_k, d_s = DeviceBuffer.from_array(ctx, k), DeviceBuffer.from_array(ctx, sc)
+    pts, out = DeviceBuffer(ctx, n * (128 if g2 else 64)), DeviceBuffer(ctx, 128)
+    fixed_base(d_k, n, pts, g2=g2)
+    msm_device(d_s, pts, n, out, g2=g2, window_bits=13)
+    assert np.array_equal(out.download((32 if g2 else 16,)), gen_mul(dot_mod_r(k, sc), g2))
