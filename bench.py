@@ -169,7 +169,7 @@ def main() -> int:
     ms_step = elapsed / args.steps * 1e3
     value = n / (elapsed / args.steps)
 
-    entries = n * W  # nonzero signed digits (zero digits occur with probability ~2^-c)
+    entries = plan[7]  # signed digits of the halves of the scalars (zero ones occur with probability ~2^-c)
     acc_mac = entries * 11 * 136
     achieved = acc_mac / (stage[1] * 1e-3)
     peak = min(mad_rate, ISSUE_PEAK)

@@ -9,7 +9,8 @@
 // Pipeline (all on one stream, no host round trip):
 //   1. k_digits      one thread per point: k mod r, split in two halves along
 //                    the endomorphism (on G2 in four quarters, glv.h), signed
-//                    c-bit digits of each for W windows; (window, |digit|) -> bucket key; histogram.
+//                    c-bit digits of each for W windows; (window, |digit|)
+//                    -> bucket key; histogram.
 //   2. scan          exclusive prefix sum of the histogram -> bucket offsets.
 //   3. k_scatter     counting-sort placement of (point index | sign) by key.
 //   4. k_accumulate  each thread folds a fixed-length chunk of the sorted
