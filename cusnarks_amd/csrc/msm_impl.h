@@ -1421,7 +1421,9 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
   const uint32_t nb = (ncnt + SCAN_TILE - 1) / SCAN_TILE;
   const uint32_t Ktot = pl.J * pl.K, Wtot = pl.J * pl.W;
   uint32_t *digits = cv.take<uint32_t>(pl.max_entries);
-  uint32_t *sorted = cv.take<uint32_t>(pl.max_entries + 4);  // + 4: quad loads
+  // not in the digits' place: the first pass writes it where a bin is one bucket.
+  // + 4: quad loads
+  uint32_t *sorted = cv.take<uint32_t>(pl.max_entries + 4);
   constexpr int PW = 2 * FieldIO<F>::NW, SW = Slot29<F>::SW;
   char *sortbuf = cv.take<char>(msm_sortbuf_bytes(pl, g2));
   Carver cs(sortbuf);
