@@ -109,3 +109,23 @@ def test_quarter_scalars(tmp_path):
         assert (sum(t * pow(mu, i, R) for i, t in enumerate(v)) - k) % R == 0, hex(k)
         if k < 1 << 63:
             assert v == [k, 0, 0, 0]
+
+
+@pytest.mark.parametrize("least", [4, 8])
+def test_chunk_length_keeps_threads(tmp_path, least):
+    # a chunk is longer than full rounds of 2^17 threads need only while it is
+    # short and 2^14 threads are left, and no number of entries and buckets asks
+    # for more than a plan takes (2^20 entries a chunk)
+    L = compiled(tmp_path, "chunk.h", "uint32_t len(uint32_t l, uint32_t e, uint32_t k) "
+                                      "{ return csk::ChunkLen{0, l}(e, k); }")
+    L.len.restype = ctypes.c_uint32
+    rng = random.Random(3)
+    es = [1 << k for k in range(31)] + [2**31 - 1] + [rng.randrange(1 << rng.randrange(1, 32)) % 2**31 for _ in range(400)]
+    for k in [1 << c for c in range(1, 20)] + [3 << c for c in range(1, 16)]:
+        for e in es:
+            n = L.len(least, e, k)
+            assert n <= 1 << 14, (e, k)
+            if n > max(least, -(-e // (1 << 17))):
+                assert n <= 48 and e // n >= 1 << 14, (e, k, n)
+    for n in range(1000, 4096):  # a table's 32 windows of 8 bits, sorted together
+        assert L.len(8, 32 * n, 128) == 8

@@ -12,7 +12,7 @@ import pytest
 import oracle as O
 from cusnarks_amd import _capi, inputs
 from cusnarks_amd.device import DeviceBuffer
-from cusnarks_amd.msm import MsmTable, fixed_base, msm_host
+from cusnarks_amd.msm import MsmTable, fixed_base, msm_device, msm_host
 from oracle import pyoracle as P
 from tests.gpu_util import dot_mod_r, g1_fixture, g2_fixture, gen_mul
 
@@ -224,3 +224,21 @@ def test_joint_and_separate_windows(g2, n):
     t.run(ds, out)
     assert np.array_equal(out.download((32 if g2 else 16,)), gen_mul(dot_mod_r(k, sc), g2))
     t.close()
+
+
+@pytest.mark.parametrize("c,n", [(2, 106497), (3, 327681), (4, 20001)])
+def test_narrow_windows_over_many_points(c, n):
+    # few buckets of very many entries: taken at every width, and the plain
+    # multiexp's result
+    ctx = _capi.default_context()
+    pts = DeviceBuffer(ctx, n * 64)
+    fixed_base(DeviceBuffer.from_array(ctx, inputs.field_elements(911, n, nonzero=True)), n, pts, ctx=ctx)
+    sc = DeviceBuffer.from_array(ctx, inputs.field_elements(912, n))
+    out, want, narrow = (DeviceBuffer(ctx, 64) for _ in range(3))
+    t = MsmTable(pts, n, window_bits=c, ctx=ctx)
+    t.run(sc, out)
+    msm_device(sc, pts, n, want, ctx=ctx)
+    msm_device(sc, pts, n, narrow, ctx=ctx, window_bits=c)
+    t.close()
+    assert np.array_equal(out.download((16,)), want.download((16,)))
+    assert np.array_equal(narrow.download((16,)), want.download((16,)))
