@@ -1,4 +1,4 @@
-// Entries per thread of the multiexp's bucket loops.
+// Entries per thread of the multiexp's bucket loops, and how a table run is sorted.
 #pragma once
 #include <stdint.h>
 
@@ -52,5 +52,28 @@ struct ChunkLen {
     return n < r ? n : r;
   }
 };
+
+// Whether a table run's windows are sorted together, as one member of Wt * n_pad
+// points (a table's slices follow each other, and window w of scalar i is an
+// entry for point w * n_pad + i), so that all of a bucket's entries are
+// adjacent.  As members of one window each, every window has its own copy of
+// the buckets, carried, fixed up and merged: at 100003 points, c = 16, 524288
+// buckets of 3 entries instead of 32768 of 49, 582 -> 410 us; 500 points
+// 411 -> 219, 2^20 1661 -> 1475, 2.2M (2^25 entries) 3267 -> 3002 us; G2 5000 868 ->
+// 455, 2^20 4828 -> 3999 us.  A member has at most 256 second-pass workgroups, so
+// larger runs keep the members: 2^22 points 5886 us joint, 5829 as members.
+// So do those whose top window (254 mod c bits) is no wider than what the second
+// pass sorts by (c - 9 bits): all its n_pad entries are then in one bin, and one
+// workgroup's walk through them, 1.3 ns each, is waited for, while a member's top
+// window has bins of its own.  The members' copies of the buckets cost 0.2 ns each
+// on G1 and 0.8 on G2; the line lies at about twice that and from 2^18 points, where
+// they win with wire values too (G1 2^20 points, c = 12: joint 3.66, members 2.26 ms;
+// c = 14 3.31 and 2.00; c = 18 2.92 and 2.00; G2 2^20, c = 14 6.88 and 5.72).
+constexpr bool table_joint(uint64_t n_pad, uint32_t c, uint32_t Wt, bool g2) {
+  if (n_pad * Wt > 1ull << 25) return false;
+  const bool one_bin = c > 9 && 254 % c <= c - 9;
+  const uint64_t copies = (uint64_t)Wt << (c - 1);
+  return !(one_bin && n_pad > 1u << 18 && 5 * n_pad > (g2 ? 3 : 2) * copies);
+}
 
 }  // namespace csk

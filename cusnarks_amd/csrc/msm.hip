@@ -455,28 +455,16 @@ struct csk_msm_table {
 
 namespace csk {
 
-// Whether a run's windows are sorted together, as one member of Wt * n_pad
-// points (a table's slices follow each other, and window w of scalar i is an
-// entry for point w * n_pad + i), so that all of a bucket's entries are
-// adjacent.  As members of one window each, every window has its own copy of
-// the buckets, carried, fixed up and merged: at 100003 points, c = 16, 524288
-// buckets of 3 entries instead of 32768 of 49, 582 -> 410 us; 500 points
-// 411 -> 219, 2^20 1661 -> 1475, 2.2M (2^25 entries) 3267 -> 3002 us; G2 5000 868 ->
-// 455, 2^20 4828 -> 3999 us.  A member has at most 256 second-pass workgroups, so
-// larger runs keep the members: 2^22 points 5886 us joint, 5829 as members.
-static constexpr uint64_t kJointMax = 1ull << 25;
-static bool table_joint(uint64_t n_pad, uint32_t Wt) { return n_pad * Wt <= kJointMax; }
-
 // group plan of the runs over tables of n_pad[0..count) points: count members of
 // Wt * n_pad points, or count * Wt one-window members
-static MsmPlan table_plan(uint32_t c, const uint64_t *n_pad, uint32_t count, uint32_t Wt) {
+static MsmPlan table_plan(bool g2, uint32_t c, const uint64_t *n_pad, uint32_t count, uint32_t Wt) {
   MsmPlan pl = {};
   uint64_t most = 0;
   for (uint32_t p = 0; p < count; p++) {
     pl.n += n_pad[p] * Wt;
     if (n_pad[p] > most) most = n_pad[p];
   }
-  const bool joint = table_joint(most, Wt);
+  const bool joint = table_joint(most, c, Wt, g2);
   pl.c = c;
   pl.E = 1;
   pl.bits = kScalarBits;
@@ -537,7 +525,7 @@ static int table_run(csk_ctx *ctx, uint32_t count, csk_msm_table *const *t, cons
     const uint32_t nt = (uint32_t)(t[p]->n_pad / kSortTile);
     if (nt > max_nt) max_nt = nt;
   }
-  const MsmPlan pl = table_plan(c, pads, count, Wt);
+  const MsmPlan pl = table_plan(t0->ec2 != 0, c, pads, count, Wt);
   if (!msm_plan_ok(pl)) {
     set_error("msm_table_run: " + std::to_string(count) + " runs of up to " + std::to_string(max_nt * kSortTile) +
               " points exceed the multiexp's index range");
@@ -595,7 +583,7 @@ extern "C" int csk_msm_table_create(csk_ctx *ctx, int ec2, const uint32_t *d_poi
   }
   const uint32_t Wt = 254 / c + 1;
   const uint64_t n_pad = (n + kSortTile - 1) / kSortTile * kSortTile;
-  MsmPlan pl = table_plan(c, &n_pad, 1, Wt);
+  MsmPlan pl = table_plan(ec2 != 0, c, &n_pad, 1, Wt);
   if (!msm_plan_ok(pl)) {
     set_error("msm_table_create: " + std::to_string(n) + " points x " + std::to_string(Wt) +
               " windows exceed the multiexp's index range");
@@ -686,7 +674,7 @@ extern "C" int csk_msm_table_run_multi(csk_ctx *ctx, uint32_t count, csk_msm_tab
 
 extern "C" int csk_msm_table_info(const csk_msm_table *t, uint64_t *out, int n) {
   if (!t || !out || n < 1) return CSK_ERR_ARG;
-  const MsmPlan pl = table_plan(t->c, &t->n_pad, 1, t->Wt);
+  const MsmPlan pl = table_plan(t->ec2 != 0, t->c, &t->n_pad, 1, t->Wt);
   const uint64_t v[5] = {t->n, t->c, t->Wt, t->table_bytes, msm_table_ws_bytes(pl, t->ec2 != 0, 1)};
   for (int i = 0; i < n && i < 5; i++) out[i] = v[i];
   return CSK_OK;

@@ -129,3 +129,21 @@ def test_chunk_length_keeps_threads(tmp_path, least):
                 assert n <= 48 and e // n >= 1 << 14, (e, k, n)
     for n in range(1000, 4096):  # a table's 32 windows of 8 bits, sorted together
         assert L.len(8, 32 * n, 128) == 8
+
+
+def test_table_windows_sorted_together(tmp_path):
+    # a top window that would sit in one bin of a large joint sort keeps the windows apart
+    L = compiled(tmp_path, "chunk.h", "int joint(uint64_t n, uint32_t c, uint32_t w, int g2) "
+                                      "{ return csk::table_joint(n, c, w, g2 != 0); }")
+    L.joint.argtypes = [ctypes.c_uint64, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_int]
+    joint = lambda n, c, g2=False: bool(L.joint(n, c, 254 // c + 1, int(g2)))
+    for c in range(2, 21):
+        w = 254 // c + 1
+        for g2 in (False, True):
+            assert joint(4096, c, g2)
+            assert not joint((1 << 25) // w // 4096 * 4096 + 4096, c, g2)
+            assert joint(min(1 << 18, (1 << 25) // w // 4096 * 4096), c, g2)
+    for c in (12, 14, 18):
+        assert not joint(1 << 20, c)
+    for c in (10, 13, 16, 17):
+        assert joint(1 << 20, c)

@@ -242,3 +242,22 @@ def test_narrow_windows_over_many_points(c, n):
     t.close()
     assert np.array_equal(out.download((16,)), want.download((16,)))
     assert np.array_equal(narrow.download((16,)), want.download((16,)))
+
+
+@pytest.mark.parametrize("g2,n,c", [(False, 1 << 18, 12), (False, (1 << 18) + 1, 12), (False, (1 << 18) + 1, 14),
+                                    (True, (1 << 18) + 1, 11)])
+def test_windows_apart_where_the_top_one_is_narrow(g2, n, c):
+    # 254 mod c is 2 or 1: the joint sort ends at 2^18 points
+    ctx = _capi.default_context()
+    k, sc = inputs.field_elements(63, n, nonzero=True), inputs.field_elements(64, n)
+    sc[: n // 2, 1:] = 0
+    ds = DeviceBuffer.from_array(ctx, sc)
+    pts, out = DeviceBuffer(ctx, n * (128 if g2 else 64)), DeviceBuffer(ctx, 128)
+    fixed_base(DeviceBuffer.from_array(ctx, k), n, pts, g2=g2)
+    t = MsmTable(pts, n, g2=g2, window_bits=c, ctx=ctx)
+    t.run(ds, out)
+    got = out.download((32 if g2 else 16,))
+    t.run_batch([ds, ds], [out, pts])
+    assert np.array_equal(out.download((32 if g2 else 16,)), got)
+    assert np.array_equal(got, gen_mul(dot_mod_r(k, sc), g2))
+    t.close()
