@@ -119,18 +119,29 @@ MsmPlan msm_group_plan(uint32_t c, uint32_t E, const uint64_t *n, uint32_t J, bo
   return pl;
 }
 
+// At widths where the halves have an entry more per point, whole scalars are the
+// fewer additions of a large multiexp: 2^24 G1 points, c = 17, 16 entries a point 23.6
+// ms, whole 15 and 21.9; c = 15 26.7 and 24.5.  The halves' fewer buckets, and half the
+// doublings, then count 10 entries each and 3 million: with 2^22 points they still win
+// or tie (c = 17 6.54 and 6.40 ms, wire values 3.75 and 3.92).  A whole scalar's narrow
+// top window (c = 14: 254 is 18 * 14 + 2) takes the gain back: 27.1 and 27.8 ms.
+static bool split_pays(const MsmPlan &split, const MsmPlan &whole) {
+  if (split.max_entries <= whole.max_entries || whole.bits % whole.c <= whole.c / 2) return true;
+  return split.max_entries - whole.max_entries <= whole.J * (10ull * (whole.K - split.K) + 3000000);
+}
+
 // G2 scalars are taken in quarters where these have no more entries at the width
 // than halves have: they have half the buckets and half the doublings.  5003 points
 // 757 us in halves (c = 13), 538 in quarters (c = 11), 2^18 points 1.88 (c = 16) and
 // 1.78 ms (c = 13).  At other widths the top window of a quarter is a waste: c = 16,
 // 5 windows of 4 against 8 of 2 per scalar, 5.9 against 5.0 ms at 2^20 points.
 MsmPlan msm_split_plan(const MsmPlan &whole, const uint64_t *n, bool g2, uint32_t chunk, uint32_t reduce_seg) {
-  const MsmPlan half = msm_group_plan(whole.c, 2, n, whole.J, g2, chunk, reduce_seg);
+  MsmPlan split = msm_group_plan(whole.c, 2, n, whole.J, g2, chunk, reduce_seg);
   if (g2) {
     const MsmPlan quarter = msm_group_plan(whole.c, 4, n, whole.J, g2, chunk, reduce_seg);
-    if (quarter.max_entries <= half.max_entries && msm_plan_ok(quarter)) return quarter;
+    if (quarter.max_entries <= split.max_entries && msm_plan_ok(quarter)) split = quarter;
   }
-  return msm_plan_ok(half) ? half : whole;
+  return msm_plan_ok(split) && split_pays(split, whole) ? split : whole;
 }
 
 bool msm_plan_ok(const MsmPlan &pl) {

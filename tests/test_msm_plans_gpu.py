@@ -1,0 +1,33 @@
+"""Which plan a multiexp runs by: whole scalars or split ones, and what is taken
+when a width or a workspace cannot be had.  The sum is the same by every plan."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from cusnarks_amd import _capi, inputs
+from cusnarks_amd.device import DeviceBuffer
+from cusnarks_amd.msm import fixed_base, msm_device
+
+pytestmark = pytest.mark.gpu
+
+
+def last_plan(ctx):
+    """(window bits, windows, points) of the context's last multiexp"""
+    plan = (ctypes.c_uint32 * 8)()
+    _capi.check(_capi.lib().csk_last_msm_plan(ctx.ptr, plan, 8), "csk_last_msm_plan")
+    return plan[0], plan[1], plan[6]
+
+
+@pytest.mark.parametrize("n,windows", [(4194304, 9), (4500000, 17)])
+def test_whole_scalars_of_large_multiexps(n, windows):
+    # c = 15: 18 entries a point in halves, 17 whole, which 4.3 million points and
+    # more take; the sum is the default width's
+    ctx = _capi.default_context()
+    pts, out, want = DeviceBuffer(ctx, n * 64), DeviceBuffer(ctx, 64), DeviceBuffer(ctx, 64)
+    sc = DeviceBuffer.from_array(ctx, inputs.field_elements(921, n))
+    fixed_base(sc, n, pts, ctx=ctx)
+    msm_device(sc, pts, n, want, ctx=ctx)
+    msm_device(sc, pts, n, out, ctx=ctx, window_bits=15)
+    assert last_plan(ctx) == (15, windows, n)
+    assert np.array_equal(out.download((16,)), want.download((16,)))
