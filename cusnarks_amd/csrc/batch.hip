@@ -59,7 +59,7 @@ struct csk_msm_batch {
 
 namespace {
 
-constexpr uint64_t kGroupEntryCap = 1ull << 30;  // entries per group (16 B of workspace each)
+constexpr uint64_t kGroupEntryCap = 1ull << 30;  // entries per group (10 B of workspace each, and their points)
 constexpr int kMaxStreams = 4;
 
 void destroy_batch(csk_msm_batch *b) {

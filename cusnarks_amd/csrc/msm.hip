@@ -164,8 +164,7 @@ size_t msm_workspace_bytes(const MsmPlan &pl, bool g2) {
   const uint64_t nb = (ncnt + SCAN_TILE - 1) / SCAN_TILE;
   const uint64_t Ktot = (uint64_t)pl.J * pl.K, Wtot = (uint64_t)pl.J * pl.W;
   size_t b = 0;
-  b += Carver::round(pl.max_entries * 4);       // digits
-  b += Carver::round((pl.max_entries + 4) * 4); // sorted (+ 4: quad loads)
+  b += Carver::round((pl.max_entries + 4) * 4); // digits, then sorted (+ 4: quad loads)
   b += Carver::round(msm_sortbuf_bytes(pl, g2)); // pass-1 entries, then 29-bit points and slots
   b += Carver::round((ncnt + 1) * 4);           // tile counts -> offsets
   b += Carver::round(nb * 4);                   // scan block sums
@@ -371,11 +370,11 @@ int msm_noalloc_setup(int device) {
 }
 
 // The bytes that decide which widths the array takes: the workspace of the
-// whole-scalar plan and a slot per reduction segment.  The pipeline that runs
-// needs no more, so a width is accepted or refused by n and cfg alone.
+// whole-scalar plan, its digits and a slot per reduction segment.  The pipeline
+// that runs needs no more, so a width is accepted or refused by n and cfg alone.
 static size_t noalloc_bytes(const MsmPlan &pl, uint32_t rseg) {
   const uint32_t seg = rseg && rseg < pl.Lr ? rseg : pl.Lr;
-  return msm_workspace_bytes(pl, false) + Carver::round((uint64_t)pl.J * pl.W * (pl.B / seg) * 144);
+  return msm_workspace_bytes(pl, false) + Carver::round(pl.max_entries * 4) + Carver::round((uint64_t)pl.J * pl.W * (pl.B / seg) * 144);
 }
 
 // out = (0, 1*R), the affine point at infinity of the empty sum

@@ -469,8 +469,8 @@ __device__ __forceinline__ TileRef tile_ref(const MsmSeg *segs, uint32_t J, uint
 // every scalar (global window index gw = j * W + w with gw mod Wwin = Wwin - 1:
 // w = W - 1 for multiexp members, every Wwin-th member for the one-window
 // members of table runs) splits its buckets at ts bits instead; with ts = 0
-// its bins are single buckets, the pass-1 ranges are the final ones, and the
-// entries go straight to `sorted`.
+// its bins are single buckets, the pass-1 ranges are the final ones, and pass 2
+// only copies the entries.
 // HOIST issues the tile's sixteen digit loads before the counts (unconditional,
 // the index clamped into the member's row; the tile's first index is < n);
 // otherwise each entry is one guarded load, wait and count.  Measured: HOIST
@@ -483,8 +483,7 @@ __global__ void __launch_bounds__(SORT_THREADS) k_sort_scatter1(const uint32_t *
                                                                 uint32_t s, uint32_t ts, uint32_t HB, uint32_t W,
                                                                 uint32_t Wwin, const uint32_t *__restrict__ goff,
                                                                 uint32_t *__restrict__ tix,
-                                                                uint16_t *__restrict__ tlo,
-                                                                uint32_t *__restrict__ sorted) {
+                                                                uint16_t *__restrict__ tlo) {
   __shared__ uint32_t h[256];
   __shared__ uint32_t base[256];
   __shared__ uint32_t scan_tmp[SORT_THREADS];
@@ -535,7 +534,7 @@ __global__ void __launch_bounds__(SORT_THREADS) k_sort_scatter1(const uint32_t *
   }
   __syncthreads();
   if (s == 0) {
-    for (uint32_t p = threadIdx.x; p < total; p += SORT_THREADS) sorted[h[sbin[p]] + p] = stage[p];
+    for (uint32_t p = threadIdx.x; p < total; p += SORT_THREADS) tix[h[sbin[p]] + p] = stage[p];
     return;
   }
   for (uint32_t p = threadIdx.x; p < total; p += SORT_THREADS) {
@@ -555,8 +554,9 @@ __global__ void __launch_bounds__(SORT_THREADS) k_sort_scatter1(const uint32_t *
 // faster for groups of 2^27 entries and more (2^24 x 15 windows), 4096 below.
 // A top window (see pass 1) partitions by its ts low bits into the buckets
 // gw*B + hi*2^ts + lo; its last segment also points the buckets it cannot
-// reach (from HB*2^ts on) at its end, and with ts = 0 pass 1 has placed its
-// entries already, so only the offsets are written.
+// reach (from HB*2^ts on) at its end, and with ts = 0 pass 1 has ordered its
+// entries already, so they are copied.  `sorted` takes the place of the digits,
+// which only pass 1 reads.
 // counter[key] += 1 for the live lanes, the count before this lane's: the lanes
 // that agree with the first one add once together.  For segments far above the
 // average, which hold a bucket of very many entries (the ones among wire
@@ -600,11 +600,22 @@ __global__ void __launch_bounds__(THREADS) k_sort_pass2(const uint32_t *__restri
   if (!LONG && seg == gridDim.x - 1 && threadIdx.x == 0) offsets[Ktot] = end;
   if (!LONG && hi == HB - 1)
     for (uint32_t k = key0 + L2 + threadIdx.x; k < (gw + 1) * B; k += THREADS) offsets[k] = end;
+  if (!LONG && s == 0 && threadIdx.x == 0) offsets[key0] = start;
+  if (!LONG && end - start > split) return;
   if (s == 0) {
-    if (threadIdx.x == 0) offsets[key0] = start;
+    for (uint32_t e0 = start; e0 < end; e0 += 8 * THREADS) {
+      uint32_t v[8];
+      for (int k = 0; k < 8; k++) {  // unconditional (clamped) loads, as below
+        const uint32_t e = e0 + k * THREADS + threadIdx.x;
+        v[k] = tix[e < end ? e : end - 1];
+      }
+      for (int k = 0; k < 8; k++) {
+        const uint32_t e = e0 + k * THREADS + threadIdx.x;
+        if (e < end) sorted[e] = v[k];
+      }
+    }
     return;
   }
-  if (!LONG && end - start > split) return;
   for (uint32_t i = threadIdx.x; i < L2; i += THREADS) cntv[i] = 0;
   __syncthreads();
   // eight unconditional (clamped) loads in flight per thread, then their counts
@@ -1384,10 +1395,10 @@ static inline void sort_place(const MsmPlan &pl, uint32_t Wwin, const uint32_t *
   const uint32_t nblk = (uint32_t)(pl.W * pl.tiles), Wtot = pl.J * pl.W, Ktot = pl.J * pl.K;
   if (pl.max_entries < (1ull << 27))
     k_sort_scatter1<true><<<nblk, SORT_THREADS, 0, st>>>(digits, segs, pl.J, sb, pl.st, HB, pl.W, Wwin, cnt, tix,
-                                                          tlo, sorted);
+                                                          tlo);
   else
     k_sort_scatter1<false><<<nblk, SORT_THREADS, 0, st>>>(digits, segs, pl.J, sb, pl.st, HB, pl.W, Wwin, cnt, tix,
-                                                           tlo, sorted);
+                                                           tlo);
   // the 8192-entry tile keeps 49 KB of staging in LDS beside 3 * 2^sb counter
   // words: used up to sb = 10 (61 KB); wider windows take the 4096 tile
   const uint32_t lds = 3 * (1u << sb) * 4;
@@ -1420,10 +1431,8 @@ int msm_run(void *ws, const MsmPlan &pl, const MsmSeg *segs, hipStream_t st, Sta
   const uint32_t ncnt = nblk * HB;
   const uint32_t nb = (ncnt + SCAN_TILE - 1) / SCAN_TILE;
   const uint32_t Ktot = pl.J * pl.K, Wtot = pl.J * pl.W;
-  uint32_t *digits = cv.take<uint32_t>(pl.max_entries);
-  // not in the digits' place: the first pass writes it where a bin is one bucket.
-  // + 4: quad loads
-  uint32_t *sorted = cv.take<uint32_t>(pl.max_entries + 4);
+  uint32_t *digits = cv.take<uint32_t>(pl.max_entries + 4);  // + 4: quad loads
+  uint32_t *sorted = digits;  // pass 2 of the sort, which writes it, no longer reads them
   constexpr int PW = 2 * FieldIO<F>::NW, SW = Slot29<F>::SW;
   char *sortbuf = cv.take<char>(msm_sortbuf_bytes(pl, g2));
   Carver cs(sortbuf);
@@ -1626,8 +1635,7 @@ inline size_t msm_table_workspace_bytes(const MsmPlan &pl, bool g2, uint32_t cou
   const uint64_t sort = Carver::round(pl.max_entries * 4) + pl.max_entries * 2;
   const uint64_t slots = Carver::round(Ktot * sb) + pl.max_chunks * sb;
   size_t b = 0;
-  b += Carver::round(pl.max_entries * 4);        // digits
-  b += Carver::round((pl.max_entries + 4) * 4);  // sorted
+  b += Carver::round((pl.max_entries + 4) * 4);  // digits, then sorted
   b += Carver::round(sort > slots ? sort : slots);
   b += Carver::round((ncnt + 1) * 4);
   b += Carver::round(nb * 4);
@@ -1660,8 +1668,8 @@ int msm_run_table(void *ws, const MsmPlan &pl, const MsmSeg *hsegs, const TabArg
   const uint32_t ncnt = nblk * HB;
   const uint32_t nb = (ncnt + SCAN_TILE - 1) / SCAN_TILE;
   const uint32_t Ktot = pl.J * pl.K;
-  uint32_t *digits = cv.take<uint32_t>(pl.max_entries);
-  uint32_t *sorted = cv.take<uint32_t>(pl.max_entries + 4);
+  uint32_t *digits = cv.take<uint32_t>(pl.max_entries + 4);
+  uint32_t *sorted = digits;  // as in msm_run
   const uint64_t sortb = Carver::round(pl.max_entries * 4) + pl.max_entries * 2;
   const uint64_t slotb = Carver::round((uint64_t)Ktot * SW * 4) + pl.max_chunks * SW * 4;
   char *sortbuf = cv.take<char>(sortb > slotb ? sortb : slotb);

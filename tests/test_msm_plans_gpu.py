@@ -31,3 +31,15 @@ def test_whole_scalars_of_large_multiexps(n, windows):
     msm_device(sc, pts, n, out, ctx=ctx, window_bits=15)
     assert last_plan(ctx) == (15, windows, n)
     assert np.array_equal(out.download((16,)), want.download((16,)))
+
+
+@pytest.mark.parametrize("lg,whole", [(18, 2531), (20, 1783), (22, 1483)])
+def test_split_plans_workspace(lg, whole):
+    # a proof's four G1 multiexps and the one on G2: points twice, on G2 up to four
+    # times, but not much more workspace than whole scalars took, in bytes a point
+    from cusnarks_amd.batch import MsmBatch
+    from cusnarks_amd.tune import apply
+    ctx, n = _capi.Context(0), 1 << lg
+    apply(ctx)
+    need = MsmBatch.workspace_bytes([n] * 4, ctx=ctx) + MsmBatch.workspace_bytes([n], g2=True, ctx=ctx)
+    assert need < 1.04 * whole * n
