@@ -9,7 +9,12 @@
 namespace csk {
 
 static thread_local std::string g_last_error;
-void set_error(const std::string &msg) { g_last_error = msg; }
+// an error reported here is not reported again by the next launch's check: a caller
+// may go on, with less memory for instance
+void set_error(const std::string &msg) {
+  g_last_error = msg;
+  (void)hipGetLastError();
+}
 
 int Workspace::ensure(size_t need) {
   if (need <= bytes) return CSK_OK;

@@ -43,3 +43,14 @@ def test_split_plans_workspace(lg, whole):
     apply(ctx)
     need = MsmBatch.workspace_bytes([n] * 4, ctx=ctx) + MsmBatch.workspace_bytes([n], g2=True, ctx=ctx)
     assert need < 1.04 * whole * n
+
+
+def test_launches_after_an_allocation_that_failed():
+    ctx = _capi.Context(0)
+    sc = DeviceBuffer.from_array(ctx, inputs.field_elements(923, 100))
+    pts, out = DeviceBuffer(ctx, 6400), DeviceBuffer(ctx, 64)
+    fixed_base(sc, 100, pts, ctx=ctx)
+    with pytest.raises(_capi.CskError):
+        DeviceBuffer(ctx, 1 << 46)
+    msm_device(sc, pts, 100, out, ctx=ctx)
+    out.download((16,))
