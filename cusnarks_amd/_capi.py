@@ -18,6 +18,7 @@ CSK_ERR_HIP = -2
 CSK_ERR_NOMEM = -3
 CSK_ERR_NODEV = -4
 BATCH_CTX_WORKSPACE = 1
+BATCH_LEAST_WORKSPACE = 2
 
 OP_MULM, OP_ADDM, OP_SUBM, OP_TOMONT, OP_FROMMONT, OP_INVM, OP_MULM_EXT = range(7)
 
@@ -74,6 +75,8 @@ _SIGS = {
     "csk_msm_set_tuning": ([P, INT, P, U32], INT),
     "csk_msm_batch_create": ([P, INT, U32, P, P, U32, ctypes.POINTER(P)], INT),
     "csk_msm_batch_bytes": ([P, INT, U32, P, P, ctypes.POINTER(U64)], INT),
+    "csk_msm_batch_least_bytes": ([P, INT, U32, P, P, ctypes.POINTER(U64)], INT),
+    "csk_ctx_limit_workspace": ([P, U64], INT),
     "csk_stream_create": ([P, ctypes.POINTER(P)], INT),
     "csk_stream_destroy": ([P, P], INT),
     "csk_stream_wait_event": ([P, P, P], INT),

@@ -31,7 +31,8 @@ class MsmBatch:
     integer device pointers); the buffers may change between runs.
     """
 
-    def __init__(self, sizes, g2: bool = False, window_bits=None, ctx=None, shared_workspace: bool = False):
+    def __init__(self, sizes, g2: bool = False, window_bits=None, ctx=None, shared_workspace: bool = False,
+                 least_workspace: bool = False):
         self.ctx = ctx or _capi.default_context()
         self.sizes = [int(x) for x in sizes]
         if not self.sizes:
@@ -43,20 +44,22 @@ class MsmBatch:
         if window_bits is not None and len(window_bits) != cnt:
             raise ValueError("window_bits length differs from sizes")
         self._ptr = P()
-        flags = _capi.BATCH_CTX_WORKSPACE if shared_workspace else 0
+        flags = (_capi.BATCH_CTX_WORKSPACE if shared_workspace else 0) | \
+            (_capi.BATCH_LEAST_WORKSPACE if least_workspace else 0)
         check(lib().csk_msm_batch_create(self.ctx.ptr, int(self.g2), cnt, ctypes.cast(n, P),
                                          ctypes.cast(wb, P) if wb is not None else None, flags,
                                          ctypes.byref(self._ptr)), "csk_msm_batch_create")
 
     @staticmethod
-    def workspace_bytes(sizes, g2: bool = False, ctx=None) -> int:
+    def workspace_bytes(sizes, g2: bool = False, ctx=None, least_workspace: bool = False) -> int:
         """Workspace bytes a batch of these sizes needs (planning only)."""
         ctx = ctx or _capi.default_context()
         sizes = [int(x) for x in sizes]
         n = (ctypes.c_uint64 * len(sizes))(*sizes)
         out = ctypes.c_uint64(0)
-        check(lib().csk_msm_batch_bytes(ctx.ptr, int(bool(g2)), len(sizes), ctypes.cast(n, P), None,
-                                        ctypes.byref(out)), "csk_msm_batch_bytes")
+        fn = lib().csk_msm_batch_least_bytes if least_workspace else lib().csk_msm_batch_bytes
+        check(fn(ctx.ptr, int(bool(g2)), len(sizes), ctypes.cast(n, P), None, ctypes.byref(out)),
+              "csk_msm_batch_bytes")
         return int(out.value)
 
     def __len__(self):

@@ -142,10 +142,28 @@ int csk_msm_set_tuning(csk_ctx *ctx, int ec2, const csk_msm_cfg *table, uint32_t
 
 namespace {
 
-// groups, plans and streams of a batch (no device memory yet)
-int plan_batch(csk_msm_batch *b, const uint64_t *n, const uint32_t *window_bits) {
+// The width of the least workspace for one member, from a coarse set up to c: a
+// narrower window has fewer buckets and more entries.
+uint32_t least_width(uint32_t c, uint64_t n, bool g2) {
+  uint32_t best = c;
+  size_t bytes = 0;
+  for (uint32_t w : {c, 16u, 13u, 11u, 8u}) {
+    const MsmPlan whole = msm_group_plan(w, 1, &n, 1, g2, 0, 0);
+    if (w > c || !msm_plan_ok(whole)) continue;
+    const size_t need = msm_workspace_bytes(msm_least_plan(whole, msm_split_plan(whole, &n, g2, 0, 0), g2), g2);
+    if (bytes && need >= bytes) continue;
+    bytes = need;
+    best = w;
+  }
+  return best;
+}
+
+// groups, plans and streams of a batch (no device memory yet); least: by the plans
+// and widths of least workspace
+int plan_batch(csk_msm_batch *b, const uint64_t *n, const uint32_t *window_bits, bool least) {
   const uint32_t count = b->count;
   const bool g2 = b->g2;
+  b->groups.clear();
   // window width per member, then groups of equal width in member order
   // Many members of one size (a cohort of proofs of one circuit) pay their
   // buckets' reduction, W * 2^(c-1) buckets each, beside n * W accumulations,
@@ -173,6 +191,7 @@ int plan_batch(csk_msm_batch *b, const uint64_t *n, const uint32_t *window_bits)
     } else if (!g2 && !cf.window_bits && per_class[lgs[i]] > 1) {
       cw[i] = multi_width(cw[i], 1, 3ull << lgs[i] >> 1);
     }
+    if (least && !cf.window_bits) cw[i] = least_width(cw[i], n[i], g2);
     if (cw[i] < 2 || cw[i] > kMaxWindowBits || n[i] * (254 / cw[i] + 1) >= (1ull << 31)) {
       set_error("msm_batch: member " + std::to_string(i) + " too large or bad window width");
       return CSK_ERR_ARG;
@@ -205,7 +224,8 @@ int plan_batch(csk_msm_batch *b, const uint64_t *n, const uint32_t *window_bits)
       set_error("msm_batch: unsupported group plan");
       return CSK_ERR_ARG;
     }
-    g.pl = msm_split_plan(g.pl, gn.data(), g2, 0, 0);
+    const MsmPlan split = msm_split_plan(g.pl, gn.data(), g2, 0, 0);
+    g.pl = least ? msm_least_plan(g.pl, split, g2) : split;
   }
   // largest groups first, dealt round-robin over the streams
   std::stable_sort(b->groups.begin(), b->groups.end(),
@@ -256,8 +276,8 @@ int bind_workspaces(csk_msm_batch *b) {
 
 extern "C" {
 
-int csk_msm_batch_bytes(csk_ctx *ctx, int ec2, uint32_t count, const uint64_t *n, const uint32_t *window_bits,
-                        uint64_t *bytes) {
+static int batch_bytes(csk_ctx *ctx, int ec2, uint32_t count, const uint64_t *n, const uint32_t *window_bits,
+                       bool least, uint64_t *bytes) {
   if (!ctx || !count || !n || !bytes) {
     set_error("msm_batch_bytes: bad arguments");
     return CSK_ERR_ARG;
@@ -266,15 +286,48 @@ int csk_msm_batch_bytes(csk_ctx *ctx, int ec2, uint32_t count, const uint64_t *n
   b.ctx = ctx;
   b.g2 = ec2 != 0;
   b.count = count;
-  int rc = plan_batch(&b, n, window_bits);
+  int rc = plan_batch(&b, n, window_bits, least);
   if (rc) return rc;
   *bytes = b.ws_bytes;
   return CSK_OK;
 }
 
+int csk_msm_batch_bytes(csk_ctx *ctx, int ec2, uint32_t count, const uint64_t *n, const uint32_t *window_bits,
+                        uint64_t *bytes) {
+  return batch_bytes(ctx, ec2, count, n, window_bits, false, bytes);
+}
+
+int csk_msm_batch_least_bytes(csk_ctx *ctx, int ec2, uint32_t count, const uint64_t *n, const uint32_t *window_bits,
+                              uint64_t *bytes) {
+  return batch_bytes(ctx, ec2, count, n, window_bits, true, bytes);
+}
+
+// the plan's device memory: descriptor tables and workspaces
+static int alloc_batch(csk_msm_batch *b) {
+  const size_t own = b->shared ? b->bytes - b->ws_bytes : b->bytes;
+  hipError_t e = hipMalloc(&b->mem, own);
+  if (e != hipSuccess) {
+    set_error(std::string("msm_batch_create: device memory (") + std::to_string(own >> 20) + " MiB): " +
+              hipGetErrorString(e));
+    b->mem = nullptr;
+    return CSK_ERR_NOMEM;
+  }
+  size_t off = 0;
+  for (auto &g : b->groups) {
+    g.d_segs = (MsmSeg *)((char *)b->mem + off);
+    off += Carver::round((g.pl.J + 1) * sizeof(MsmSeg));
+  }
+  const int rc = bind_workspaces(b);
+  if (rc) {
+    (void)hipFree(b->mem);
+    b->mem = nullptr;
+  }
+  return rc;
+}
+
 int csk_msm_batch_create(csk_ctx *ctx, int ec2, uint32_t count, const uint64_t *n,
                          const uint32_t *window_bits, uint32_t flags, csk_msm_batch **out) {
-  if (!ctx || !out || !count || !n || (flags & ~CSK_BATCH_CTX_WORKSPACE)) {
+  if (!ctx || !out || !count || !n || (flags & ~(CSK_BATCH_CTX_WORKSPACE | CSK_BATCH_LEAST_WORKSPACE))) {
     set_error("msm_batch_create: bad arguments");
     return CSK_ERR_ARG;
   }
@@ -286,26 +339,14 @@ int csk_msm_batch_create(csk_ctx *ctx, int ec2, uint32_t count, const uint64_t *
   b->count = count;
   b->n.assign(n, n + count);
   b->shared = (flags & CSK_BATCH_CTX_WORKSPACE) != 0;
-  int rc = plan_batch(b, n, window_bits);
-  if (rc) {
-    destroy_batch(b);
-    return rc;
+  const bool least = (flags & CSK_BATCH_LEAST_WORKSPACE) != 0;
+  int rc = plan_batch(b, n, window_bits, least);
+  if (rc == CSK_OK) rc = alloc_batch(b);
+  if (rc == CSK_ERR_NOMEM && !least) {  // what fits beside what else the device holds
+    rc = plan_batch(b, n, window_bits, true);
+    if (rc == CSK_OK) rc = alloc_batch(b);
+    if (rc == CSK_OK) set_error("");
   }
-  const size_t own = b->shared ? b->bytes - b->ws_bytes : b->bytes;
-  hipError_t e = hipMalloc(&b->mem, own);
-  if (e != hipSuccess) {
-    set_error(std::string("msm_batch_create: device memory (") + std::to_string(own >> 20) + " MiB): " +
-              hipGetErrorString(e));
-    b->mem = nullptr;
-    destroy_batch(b);
-    return CSK_ERR_NOMEM;
-  }
-  size_t off = 0;
-  for (auto &g : b->groups) {
-    g.d_segs = (MsmSeg *)((char *)b->mem + off);
-    off += Carver::round((g.pl.J + 1) * sizeof(MsmSeg));
-  }
-  rc = bind_workspaces(b);
   if (rc) {
     destroy_batch(b);
     return rc;

@@ -18,6 +18,10 @@ void set_error(const std::string &msg) {
 
 int Workspace::ensure(size_t need) {
   if (need <= bytes) return CSK_OK;
+  if (limit && need > limit) {
+    set_error("workspace of " + std::to_string(need) + " bytes: the context is limited to " + std::to_string(limit));
+    return CSK_ERR_NOMEM;
+  }
   if (ptr) {
     // work on any stream may still use the old buffer
     hipError_t e = hipDeviceSynchronize();
@@ -30,6 +34,7 @@ int Workspace::ensure(size_t need) {
     }
   }
   size_t want = need + need / 8;
+  if (limit && want > limit) want = limit;
   hipError_t e = hipMalloc(&ptr, want);
   if (e != hipSuccess) {
     ptr = nullptr;
@@ -337,6 +342,12 @@ int csk_last_msm_plan(csk_ctx *ctx, uint32_t *out, int n) {
   const csk::MsmPlan &p = ctx->last_plan;
   uint64_t v[8] = {p.c, p.W, p.B, p.L, p.Lr, p.S, p.n / (p.E ? p.E : 1), p.max_entries};
   for (int i = 0; i < n && i < 8; i++) out[i] = (uint32_t)v[i];
+  return CSK_OK;
+}
+
+int csk_ctx_limit_workspace(csk_ctx *ctx, uint64_t bytes) {
+  if (!ctx) return CSK_ERR_ARG;
+  ctx->ws.limit = ctx->batch_ws.limit = bytes;
   return CSK_OK;
 }
 

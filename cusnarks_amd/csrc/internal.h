@@ -38,6 +38,7 @@ struct Workspace {
   void *ptr = nullptr;
   size_t bytes = 0;
   uint64_t gen = 0;  // bumped on every reallocation
+  size_t limit = 0;  // bytes it may grow to, 0: the device's memory
   int ensure(size_t need);
   void release();
 };

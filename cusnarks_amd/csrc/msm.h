@@ -47,6 +47,8 @@ MsmPlan msm_group_plan(uint32_t c, uint32_t E, const uint64_t *n, uint32_t J, bo
 // the plan a group runs by: split scalars, or whole ones where only their
 // entries fit the index range; whole is the plan with E = 1
 MsmPlan msm_split_plan(const MsmPlan &whole, const uint64_t *n, bool g2, uint32_t chunk, uint32_t reduce_seg);
+// the one of the two that needs less workspace
+MsmPlan msm_least_plan(const MsmPlan &whole, const MsmPlan &split, bool g2);
 bool msm_plan_ok(const MsmPlan &pl);
 uint32_t multi_width(uint32_t c, uint32_t count, uint64_t n);
 int msm_multi(csk_ctx *ctx, bool g2, uint32_t count, const uint32_t *const *scalars, const uint32_t *const *points,

@@ -197,6 +197,10 @@ void msm_fill_segs(const MsmPlan &pl, const uint64_t *n, const uint32_t *const *
   }
 }
 
+MsmPlan msm_least_plan(const MsmPlan &whole, const MsmPlan &split, bool g2) {
+  return msm_workspace_bytes(whole, g2) < msm_workspace_bytes(split, g2) ? whole : split;
+}
+
 // writes the descriptor table (members + sentinel) of a call on the stream
 struct SegArgs {
   MsmSeg s[kMultiMembers + 1];
@@ -239,9 +243,17 @@ int msm_launch(csk_ctx *ctx, bool g2, const uint32_t *d_scalars, const uint32_t 
     set_error("msm: unsupported configuration (window/chunk/segment or size too large)");
     return CSK_ERR_ARG;
   }
-  pl = msm_split_plan(pl, &n, g2, chunk, rseg);
   const size_t seg_bytes = Carver::round(2 * sizeof(MsmSeg));
-  int rc = ctx->ws.ensure(seg_bytes + msm_workspace_bytes(pl, g2));
+  const MsmPlan split = msm_split_plan(pl, &n, g2, chunk, rseg), least = msm_least_plan(pl, split, g2);
+  int rc = ctx->ws.ensure(seg_bytes + msm_workspace_bytes(split, g2));
+  if (rc == CSK_ERR_NOMEM && least.E != split.E) {
+    // the split points do not fit: whole scalars need one copy of them
+    rc = ctx->ws.ensure(seg_bytes + msm_workspace_bytes(least, g2));
+    if (rc == CSK_OK) set_error("");
+    pl = least;
+  } else {
+    pl = split;
+  }
   if (rc) return rc;
   StageTimer *tm = nullptr;
   if (ctx->timing) {

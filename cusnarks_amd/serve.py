@@ -136,9 +136,13 @@ class _Circuit:
             self.msm_bytes = (max(self.tables[k].info()["workspace_bytes"] for k in ProofSlot.G1_TABLES)
                               + self.tables["B2"].info()["workspace_bytes"])
         else:
-            self.msm_bytes = (MsmBatch.workspace_bytes(self.g1_sizes, ctx=ctx)
-                              + MsmBatch.workspace_bytes([nv + 2], g2=True, ctx=ctx))
+            self.msm_bytes = self.batch_bytes(ctx, False)
+        self.least = False  # its cohorts run by the plans of least workspace
         self.idle: list[ProofSlot] = []
+
+    def batch_bytes(self, ctx, least: bool) -> int:
+        return (MsmBatch.workspace_bytes(self.g1_sizes, ctx=ctx, least_workspace=least)
+                + MsmBatch.workspace_bytes([self.pk.n_vars + 2], g2=True, ctx=ctx, least_workspace=least))
 
 
 class _Cohort:
@@ -181,14 +185,15 @@ class _Lane:
         self.cohorts = 0
         self.cohort_sizes: list[int] = []
 
-    def batch(self, sizes, g2: bool, pos: int) -> MsmBatch:
+    def batch(self, sizes, g2: bool, pos: int, least: bool = False) -> MsmBatch:
         # keyed by cohort position too: a batch rewrites its descriptor tables
         # only after its previous run ended, and the cohort in flight at the
         # other position may be that run
-        key = (g2, tuple(sizes), pos)
+        key = (g2, tuple(sizes), pos, least)
         b = self.batches.get(key)
         if b is None:
-            b = MsmBatch(sizes, g2=g2, ctx=self.ctx_g2 if g2 else self.ctx_g1, shared_workspace=True)
+            b = MsmBatch(sizes, g2=g2, ctx=self.ctx_g2 if g2 else self.ctx_g1, shared_workspace=True,
+                         least_workspace=least)
             b.uses = 0
             self.batches[key] = b
             while len(self.batches) > 32:  # each batch owns its streams and tables
@@ -219,6 +224,10 @@ class ProofServer:
         self.circuits = {name: _Circuit(name, pk, int(pk.log2m >= large_log2m), ctx, use_tables)
                          for name, pk in keys.items()}
         self.adm = Admission(budget_bytes, max_inflight, shares=(small_share, 1.0 - small_share))
+        for cc in self.circuits.values():
+            # a share too small for the fastest plans may still hold slower ones
+            if not cc.tables and self.adm.never_fits(cc.lane, cc.slot_bytes, cc.msm_bytes):
+                cc.msm_bytes, cc.least = cc.batch_bytes(ctx, True), True
         self.queues = [collections.deque(), collections.deque()]
         self.use_graph = use_graph
         self.done: list[Request] = []
@@ -348,8 +357,9 @@ class ProofServer:
         if plain:
             g1 = [m for req in plain for m in req.slot.g1_members()]
             g2 = [req.slot.g2_member() for req in plain]
-            b1 = lane.batch([m[2] for m in g1], False, pos)
-            b2 = lane.batch([m[2] for m in g2], True, pos)
+            least = any(self.circuits[req.circuit].least for req in plain)
+            b1 = lane.batch([m[2] for m in g1], False, pos, least)
+            b2 = lane.batch([m[2] for m in g2], True, pos, least)
             runs += [(b1, g1, lane.st_g1), (b2, g2, lane.st_g2)]
             ws += b1.info()["bytes"] + b2.info()["bytes"]
         fin = [req.slot.final_member() for req in ready]

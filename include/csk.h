@@ -54,6 +54,10 @@ int csk_device_count(int *count);
  * ms[1] bucket accumulation, ms[2] fix-up + reductions + final combine,
  * ms[3] total.  Missing values are -1. */
 int csk_ctx_set_timing(csk_ctx *ctx, int on);
+/* Multiexps grow the context's workspaces to at most `bytes` each (0, the default:
+ * as far as the device's memory goes).  One that would need more runs by a plan
+ * that needs less (the same result), or fails with CSK_ERR_NOMEM. */
+int csk_ctx_limit_workspace(csk_ctx *ctx, uint64_t bytes);
 int csk_last_stage_times(csk_ctx *ctx, float *ms, int n);
 /* Plan of the last single multiexp: c, W, buckets/window, chunk, reduce
  * segment, segments/window, n, entry bound (first n values written). */
@@ -156,10 +160,14 @@ int csk_msm_set_tuning(csk_ctx *ctx, int ec2, const csk_msm_cfg *table, uint32_t
  *   16 / 32 words), enqueued on stream.  Pointers may change between runs.
  *   use_graph != 0 replays a graph captured on the first such run (captured
  *   again if the shared workspace moved).  Runs of one batch must not overlap.
- * bytes: the workspace bytes such a batch needs (no allocation).
+ *   CSK_BATCH_LEAST_WORKSPACE plans whole scalars and narrower windows where
+ *   these need less workspace (slower); so does a batch whose memory cannot be had.
+ * bytes, least_bytes: the workspace bytes such a batch needs, without and with
+ *   CSK_BATCH_LEAST_WORKSPACE (no allocation).
  * info: out = {groups, device bytes, then per group: c, members, chunk,
  *   entry bound} (first n values). */
 #define CSK_BATCH_CTX_WORKSPACE 1u
+#define CSK_BATCH_LEAST_WORKSPACE 2u
 typedef struct csk_msm_batch csk_msm_batch;
 int csk_msm_batch_create(csk_ctx *ctx, int ec2, uint32_t count, const uint64_t *n,
                          const uint32_t *window_bits, uint32_t flags, csk_msm_batch **out);
@@ -168,6 +176,8 @@ int csk_msm_batch_run(csk_msm_batch *b, const uint32_t *const *d_scalars,
                       int use_graph, void *stream);
 int csk_msm_batch_bytes(csk_ctx *ctx, int ec2, uint32_t count, const uint64_t *n,
                         const uint32_t *window_bits, uint64_t *bytes);
+int csk_msm_batch_least_bytes(csk_ctx *ctx, int ec2, uint32_t count, const uint64_t *n,
+                              const uint32_t *window_bits, uint64_t *bytes);
 int csk_msm_batch_info(const csk_msm_batch *b, uint64_t *out, int n);
 void csk_msm_batch_destroy(csk_msm_batch *b);
 

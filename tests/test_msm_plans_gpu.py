@@ -45,6 +45,45 @@ def test_split_plans_workspace(lg, whole):
     assert need < 1.04 * whole * n
 
 
+@pytest.mark.parametrize("g2,n", [(False, 1), (False, 1 << 20), (True, 1 << 18), (True, 1 << 20)])
+def test_workspace_limit(g2, n):
+    # a context that the split plan does not fit in runs a plan that needs less;
+    # below that the call is refused, the context stays usable and nothing lingers
+    from cusnarks_amd.batch import MsmBatch
+    from cusnarks_amd.tune import apply
+    ctx, nw, L = _capi.Context(0), 32 if g2 else 16, _capi.lib()
+    apply(ctx)
+    limit = lambda b: _capi.check(L.csk_ctx_limit_workspace(ctx.ptr, int(b)), "limit")  # noqa: E731
+    pts, out, want = DeviceBuffer(ctx, n * nw * 4), DeviceBuffer(ctx, nw * 4), DeviceBuffer(ctx, nw * 4)
+    sc = DeviceBuffer.from_array(ctx, inputs.field_elements(922, n))
+    fixed_base(sc, n, pts, g2=g2, ctx=ctx)
+    msm_device(sc, pts, n, want, g2=g2, ctx=_capi.Context(0))
+    expected = want.download((nw,))
+    need = MsmBatch.workspace_bytes([n], g2=g2, ctx=ctx)
+    least = MsmBatch.workspace_bytes([n], g2=g2, ctx=ctx, least_workspace=True)
+    assert least <= need
+    limit(least // 2)
+    with pytest.raises(_capi.CskError):
+        MsmBatch([n], g2=g2, ctx=ctx, shared_workspace=True)
+    with pytest.raises(_capi.CskError):
+        msm_device(sc, pts, n, out, g2=g2, ctx=ctx)
+    limit(max(least, need - 1))
+    b = MsmBatch([n], g2=g2, ctx=ctx, shared_workspace=True)
+    assert least <= b.info()["bytes"] <= max(least, need - 1) + 4096
+    b.run([sc], [pts], [out])
+    assert np.array_equal(out.download((nw,)), expected)
+    if g2 and n == 1 << 20:  # whole scalars need less at the tuned width
+        msm_device(sc, pts, n, out, g2=g2, ctx=ctx)
+        assert last_plan(ctx)[1] == 254 // last_plan(ctx)[0] + 1 and L.csk_last_error() == b""
+        assert np.array_equal(out.download((nw,)), expected)
+    limit(0)
+    msm_device(sc, pts, n, out, g2=g2, ctx=ctx)
+    assert np.array_equal(out.download((nw,)), expected)
+    b2 = MsmBatch([n], g2=g2, ctx=ctx, least_workspace=True)
+    b2.run([sc], [pts], [out], use_graph=False)
+    assert np.array_equal(out.download((nw,)), expected)
+
+
 def test_launches_after_an_allocation_that_failed():
     ctx = _capi.Context(0)
     sc = DeviceBuffer.from_array(ctx, inputs.field_elements(923, 100))

@@ -123,3 +123,21 @@ def test_served_tiny_circuit_vs_python_oracle(keys):
         assert list(q.proof[0]) == P.g1_to_words(ea)
         assert list(q.proof[1]) == P.g2_to_words(eb)
         assert list(q.proof[2]) == P.g1_to_words(ec)
+
+
+def test_share_that_holds_only_the_least_workspace(keys):
+    # a request that its lane's share cannot hold by the fastest plans is admitted
+    # by those of least workspace, and its proof is the same
+    pks, wit = keys
+    only = {"c5000": pks["c5000"]}
+    cc = ProofServer(only, budget_bytes=1 << 30, small_share=1.0).circuits["c5000"]
+    assert not cc.least
+    least = ProofServer(only, budget_bytes=1, small_share=1.0).circuits["c5000"].msm_bytes
+    assert least < cc.msm_bytes
+    srv = ProofServer(only, budget_bytes=cc.slot_bytes + least, small_share=1.0)
+    reqs = [Request(i, "c5000", wit["c5000"], 11 + i, 13 + i) for i in range(3)]
+    srv.run(reqs)
+    pr = GrothProver(pks["c5000"])
+    assert not srv.rejected
+    for q in reqs:
+        assert all(np.array_equal(a, b) for a, b in zip(q.proof, pr.prove(q.witness, q.r, q.s)))
