@@ -214,6 +214,16 @@ static void put_segs(const MsmPlan &pl, const MsmSeg *segs, MsmSeg *dst, hipStre
   k_put_segs<<<1, 64, 0, st>>>(a, pl.J + 1, dst);
 }
 
+// a single call's whole-scalar plan and the settings it was made with
+static MsmPlan single_plan(const csk_ctx *ctx, bool g2, uint64_t n, const csk_msm_cfg *cfg, uint32_t &chunk,
+                           uint32_t &rseg) {
+  const uint32_t lg = floor_log2(n);
+  const csk_msm_cfg *tn = lg < 64 && !(cfg && cfg->window_bits) ? &ctx->tune[g2][lg] : nullptr;
+  chunk = cfg && cfg->chunk ? cfg->chunk : tn ? tn->chunk : 0;
+  rseg = cfg && cfg->reduce_seg ? cfg->reduce_seg : tn ? tn->reduce_seg : 0;
+  return msm_group_plan(msm_choose_c(n, g2, ctx, cfg), 1, &n, 1, g2, chunk, rseg);
+}
+
 int msm_launch(csk_ctx *ctx, bool g2, const uint32_t *d_scalars, const uint32_t *d_points, uint64_t n,
                uint32_t *d_out, const csk_msm_cfg *cfg, hipStream_t st) {
   if (!d_out) {
@@ -233,12 +243,8 @@ int msm_launch(csk_ctx *ctx, bool g2, const uint32_t *d_scalars, const uint32_t 
     set_error("msm: null input");
     return CSK_ERR_ARG;
   }
-  const uint32_t c = msm_choose_c(n, g2, ctx, cfg);
-  const uint32_t lg = floor_log2(n);
-  const csk_msm_cfg *tn = lg < 64 ? &ctx->tune[g2][lg] : nullptr;
-  const uint32_t chunk = cfg && cfg->chunk ? cfg->chunk : (tn && !(cfg && cfg->window_bits) ? tn->chunk : 0);
-  const uint32_t rseg = cfg && cfg->reduce_seg ? cfg->reduce_seg : (tn && !(cfg && cfg->window_bits) ? tn->reduce_seg : 0);
-  MsmPlan pl = msm_group_plan(c, 1, &n, 1, g2, chunk, rseg);
+  uint32_t chunk, rseg;
+  MsmPlan pl = single_plan(ctx, g2, n, cfg, chunk, rseg);
   if (!msm_plan_ok(pl)) {
     set_error("msm: unsupported configuration (window/chunk/segment or size too large)");
     return CSK_ERR_ARG;
@@ -317,6 +323,18 @@ uint32_t multi_width(uint32_t c, uint32_t count, uint64_t n) {
 // workspaces, which a group needs, is worth.
 int msm_multi(csk_ctx *ctx, bool g2, uint32_t count, const uint32_t *const *scalars, const uint32_t *const *points,
               const uint64_t *n, uint32_t *const *out, hipStream_t st) {
+  // what a single call would refuse is refused before anything is enqueued
+  uint32_t chunk, rseg;
+  for (uint32_t i = 0; i < count; i++) {
+    if (!out[i] || (n[i] && (!scalars[i] || !points[i]))) {
+      set_error("msm_multi: null pointer for member " + std::to_string(i));
+      return CSK_ERR_ARG;
+    }
+    if (n[i] && !msm_plan_ok(single_plan(ctx, g2, n[i], nullptr, chunk, rseg))) {
+      set_error("msm_multi: member " + std::to_string(i) + " too large");
+      return CSK_ERR_ARG;
+    }
+  }
   CSK_HIP(hipSetDevice(ctx->device));
   uint64_t done = 0;  // members enqueued, a bit each
   for (uint32_t i = 0; i < count; i++) {
@@ -327,7 +345,7 @@ int msm_multi(csk_ctx *ctx, bool g2, uint32_t count, const uint32_t *const *scal
     const uint32_t *gs[kMultiMembers], *gp[kMultiMembers];
     uint32_t *go[kMultiMembers];
     for (uint32_t j = i; j < count && k < kMultiMembers; j++) {
-      if ((done >> j & 1) || n[j] == 0 || !scalars[j] || !points[j] || !out[j]) continue;
+      if ((done >> j & 1) || n[j] == 0) continue;
       if (n[j] > kMultiPoints || total + n[j] > kMultiPoints || msm_choose_c(n[j], g2, ctx, nullptr) != c) continue;
       total += n[j];
       idx[k] = j;

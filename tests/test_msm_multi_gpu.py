@@ -43,3 +43,29 @@ def test_refused():
     p, q = ctypes.cast(none, _capi.P), ctypes.cast(n, _capi.P)
     for count in (0, 1, 65):  # no member, null members, too many
         assert L.csk_msm_multi(ctx.ptr, 0, count, p, p, q, p, None) != 0
+
+
+def _members(ctx, g2, sizes):
+    nw, n = 32 if g2 else 16, max(sizes)
+    pts, outs = DeviceBuffer(ctx, n * nw * 4), DeviceBuffer(ctx, len(sizes) * nw * 4)
+    sc = DeviceBuffer.from_array(ctx, inputs.field_elements(73, n, nonzero=True))
+    fixed_base(sc, n, pts, g2=g2, ctx=ctx)
+    keep = (sc, pts, outs)
+    return keep, [(sc.ptr, pts.ptr, m, outs.ptr + i * nw * 4) for i, m in enumerate(sizes)]
+
+
+@pytest.mark.parametrize("bad", [0, 1, 3])
+def test_refused_before_anything_is_enqueued(bad):
+    ctx, sizes = _capi.Context(0), [300, 400, 30000]
+    keep, members = _members(ctx, False, sizes)
+    mark = np.full((3, 16), 7, np.uint32)
+    keep[2].upload(mark)
+    last = list(members[2])
+    last[bad] = 0
+    with pytest.raises(_capi.CskError):
+        msm_multi(members[:2] + [tuple(last)], ctx=ctx)
+    last = members[2][:2] + ((1 << 31),) + members[2][3:]  # more entries than an index holds
+    with pytest.raises(_capi.CskError):
+        msm_multi(members[:2] + [last], ctx=ctx)
+    _capi.check(_capi.lib().csk_stream_sync(ctx.ptr, None), "sync")
+    assert np.array_equal(keep[2].download((3, 16)), mark)
