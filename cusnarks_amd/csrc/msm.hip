@@ -315,6 +315,12 @@ uint32_t multi_width(uint32_t c, uint32_t count, uint64_t n) {
   return best;
 }
 
+// out = (0, 1*R), the affine point at infinity of the empty sum; words 16 (G1), 32 (G2)
+__global__ void k_put_inf(uint32_t *out, uint32_t words) {
+  const uint32_t i = threadIdx.x, y = words / 2;
+  if (i < words) out[i] = i >= y && i < y + 8 ? FieldConst<0>::one[i - y] : 0u;
+}
+
 // The members a single call would give the same width run as one group: a stage is
 // one launch over all of them, and their window combinations, a chain of 126
 // doublings and an inversion that one workgroup each waits for, run side by side.
@@ -339,7 +345,12 @@ int msm_multi(csk_ctx *ctx, bool g2, uint32_t count, const uint32_t *const *scal
   uint64_t done = 0;  // members enqueued, a bit each
   for (uint32_t i = 0; i < count; i++) {
     if (done >> i & 1) continue;
-    const uint32_t c = msm_choose_c(n[i] ? n[i] : 1, g2, ctx, nullptr);
+    if (n[i] == 0) {
+      k_put_inf<<<1, 64, 0, st>>>(out[i], g2 ? 32 : 16);
+      CSK_CHECK_LAUNCH();
+      continue;
+    }
+    const uint32_t c = msm_choose_c(n[i], g2, ctx, nullptr);
     uint32_t idx[kMultiMembers], k = 0;
     uint64_t gn[kMultiMembers], total = 0;
     const uint32_t *gs[kMultiMembers], *gp[kMultiMembers];
@@ -407,12 +418,6 @@ static size_t noalloc_bytes(const MsmPlan &pl, uint32_t rseg) {
   return msm_workspace_bytes(pl, false) + Carver::round(pl.max_entries * 4) + Carver::round((uint64_t)pl.J * pl.W * (pl.B / seg) * 144);
 }
 
-// out = (0, 1*R), the affine point at infinity of the empty sum
-__global__ void k_put_inf_g1(uint32_t *out) {
-  uint32_t i = threadIdx.x;
-  if (i < 16) out[i] = i < 8 ? 0u : FieldConst<0>::one[i - 8];
-}
-
 }  // namespace csk
 
 using namespace csk;
@@ -438,7 +443,7 @@ extern "C" int csk_msm_g1_noalloc(csk_ctx *ctx, const uint32_t *d_scalars, const
   char *base = (char *)g_scratch_ptr[ctx->device];
   hipStream_t st = (hipStream_t)stream;
   if (n == 0) {
-    k_put_inf_g1<<<1, 64, 0, st>>>(d_out);
+    k_put_inf<<<1, 64, 0, st>>>(d_out, 16);
     CSK_CHECK_LAUNCH();
     return CSK_OK;
   }

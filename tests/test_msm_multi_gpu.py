@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from cusnarks_amd import _capi, inputs
-from cusnarks_amd.device import DeviceBuffer
+from cusnarks_amd.device import DeviceBuffer, Stream
 from cusnarks_amd.msm import fixed_base, msm_device, msm_multi
 
 pytestmark = pytest.mark.gpu
@@ -52,6 +52,31 @@ def _members(ctx, g2, sizes):
     fixed_base(sc, n, pts, g2=g2, ctx=ctx)
     keep = (sc, pts, outs)
     return keep, [(sc.ptr, pts.ptr, m, outs.ptr + i * nw * 4) for i, m in enumerate(sizes)]
+
+
+@pytest.mark.parametrize("g2", [False, True])
+def test_empty_members_do_not_wait(g2):
+    # a call with empty members is enqueued like any other: it can be captured, and
+    # every replay writes all outputs
+    hip = ctypes.CDLL("libamdhip64.so")
+    ctx, sizes = _capi.Context(0), [0, 300, 0, 5000, 200]
+    keep, members = _members(ctx, g2, sizes)
+    outs, shape = keep[2], (len(sizes), 32 if g2 else 16)
+    msm_multi(members, g2=g2, ctx=ctx)  # grows the workspace
+    want = outs.download(shape)
+    zero = np.zeros(shape, np.uint32)
+    st, graph, ex = Stream(ctx), ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamBeginCapture(st.ptr, 1) == 0
+    msm_multi(members, g2=g2, ctx=ctx, stream=st.ptr)
+    assert hip.hipStreamEndCapture(st.ptr, ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, 0) == 0
+    for _ in range(3):
+        outs.upload(zero)
+        assert hip.hipGraphLaunch(ex, st.ptr) == 0
+        _capi.check(_capi.lib().csk_stream_sync(ctx.ptr, st.ptr), "sync")
+        assert np.array_equal(outs.download(shape), want)
+    hip.hipGraphExecDestroy(ex)
+    hip.hipGraphDestroy(graph)
 
 
 @pytest.mark.parametrize("bad", [0, 1, 3])
