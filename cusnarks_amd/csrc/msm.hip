@@ -285,7 +285,10 @@ static bool multi_group(csk_ctx *ctx, bool g2, uint32_t c, uint32_t count, const
   if (!msm_plan_ok(pl)) return false;
   pl = msm_split_plan(pl, n, g2, 0, 0);
   const size_t seg_bytes = Carver::round((count + 1) * sizeof(MsmSeg));
-  if (ctx->ws.ensure(seg_bytes + msm_workspace_bytes(pl, g2)) != CSK_OK) return false;
+  if (ctx->ws.ensure(seg_bytes + msm_workspace_bytes(pl, g2)) != CSK_OK) {
+    set_error("");  // the single calls may fit
+    return false;
+  }
   StageTimer *tm = nullptr;
   if (ctx->timing) {
     ctx->timer.reset();

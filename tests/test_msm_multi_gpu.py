@@ -94,3 +94,16 @@ def test_refused_before_anything_is_enqueued(bad):
         msm_multi(members[:2] + [last], ctx=ctx)
     _capi.check(_capi.lib().csk_stream_sync(ctx.ptr, None), "sync")
     assert np.array_equal(keep[2].download((3, 16)), mark)
+
+
+def test_group_that_does_not_fit_runs_member_by_member():
+    ctx, sizes = _capi.Context(0), [40000] * 8
+    keep, members = _members(ctx, False, sizes)
+    msm_multi(members, ctx=_capi.Context(0))
+    want = keep[2].download((8, 16))
+    keep[2].upload(np.zeros((8, 16), np.uint32))
+    L = _capi.lib()
+    _capi.check(L.csk_ctx_limit_workspace(ctx.ptr, 60 << 20), "limit")
+    msm_multi(members, ctx=ctx)
+    assert L.csk_last_error() == b""
+    assert np.array_equal(keep[2].download((8, 16)), want)
