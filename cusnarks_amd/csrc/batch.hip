@@ -189,7 +189,8 @@ int plan_batch(csk_msm_batch *b, const uint64_t *n, const uint32_t *window_bits,
       const uint32_t cap = lg <= 12 ? 8 : lg <= 15 ? 11 : lg <= 17 ? 13 : lg <= 19 ? 15 : kMaxWindowBits;
       if (cw[i] > cap) cw[i] = cap;
     } else if (!g2 && !cf.window_bits && per_class[lgs[i]] > 1) {
-      cw[i] = multi_width(cw[i], 1, 3ull << lgs[i] >> 1);
+      const uint32_t w = multi_width(cw[i], 1, 3ull << lgs[i] >> 1);
+      if (n[i] * (254 / w + 1) < (1ull << 31)) cw[i] = w;  // what the single call takes is taken
     }
     if (least && !cf.window_bits) cw[i] = least_width(cw[i], n[i], g2);
     if (cw[i] < 2 || cw[i] > kMaxWindowBits || n[i] * (254 / cw[i] + 1) >= (1ull << 31)) {

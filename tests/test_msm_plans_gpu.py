@@ -93,3 +93,14 @@ def test_launches_after_an_allocation_that_failed():
         DeviceBuffer(ctx, 1 << 46)
     msm_device(sc, pts, 100, out, ctx=ctx)
     out.download((16,))
+
+
+def test_batch_takes_the_sizes_of_single_calls():
+    # two members of 2^27 points at a tuned width of 18: 15 windows fit the index
+    # range, the 16 of the next narrower width do not
+    from cusnarks_amd import tune
+    from cusnarks_amd.batch import MsmBatch
+    ctx = _capi.Context(0)
+    tune.install(ctx, False, {"classes": {"27": {"window_bits": 18}}})
+    one = MsmBatch.workspace_bytes([1 << 27], ctx=ctx)
+    assert MsmBatch.workspace_bytes([1 << 27] * 2, ctx=ctx) == 2 * one
