@@ -327,7 +327,7 @@ template <> struct RowAcc<Fq> {
     if (inf) {
       for (int i = 0; i < 8; i++) w[i] = l ? FieldConst<0>::one[i] : 0u;
     } else {
-      const uint32_t t = row_inverse(k, row_mul(k, p.ZZ, p.ZZZ));
+      const uint32_t t = row_inverse(row_mul(k, p.ZZ, p.ZZZ));
       const uint32_t i = row_mul(k, t, k.odd ? p.ZZ : p.ZZZ);  // 1/ZZ | 1/ZZZ
       const uint32_t v = row_mul(k, i, k.odd ? p.Y : p.X);
       row_words(row_mul(k, v, kRowFrom[l & 15]), w);
@@ -399,7 +399,7 @@ template <> struct RowAcc<Fq2> {
       const uint32_t zz0 = v(H_ZZ0), zz1 = v(H_ZZ1), z30 = v(H_ZZZ0), z31 = v(H_ZZZ1);
       uint32_t t0, t1, u0, u1, a0, a1, b0, b1;
       row_spread2(mul2(zz0, zz1, z30, z31, zz0, zz1, z30, z31), t0, t1);  // ZZ ZZZ
-      const uint32_t n = row_inverse(k, row_dot(k, t0, t0, t1, t1));       // its inverse: (t0 - t1 u) / (t0^2 + t1^2)
+      const uint32_t n = row_inverse(row_dot(k, t0, t0, t1, t1));       // its inverse: (t0 - t1 u) / (t0^2 + t1^2)
       row_spread2(row_mul(k, odd ? neg(t1) : t0, n), u0, u1);
       row_spread4(mul2(u0, u1, z30, z31, u0, u1, zz0, zz1), a0, a1, b0, b1);  // 1/ZZ, 1/ZZZ
       const uint32_t r = mul2(v(H_X0), v(H_X1), a0, a1, v(H_Y0), v(H_Y1), b0, b1);

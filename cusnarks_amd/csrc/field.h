@@ -30,8 +30,6 @@ template <> struct FieldConst<0> {  // q
                                       2021213740u, 1718526831u, 2584207151u, 235567041u};
   static constexpr uint32_t r2[8] = {1401617033u, 4079811675u, 3561292283u, 3051821329u,
                                      172064758u,  1202396927u, 3401069855u, 114859889u};
-  static constexpr uint32_t r3[8] = {3658821855u, 2983030191u, 2804432310u, 1660031206u,
-                                     182061819u,  4018080524u, 760816964u,  553479824u};
 };
 
 template <> struct FieldConst<1> {  // r
@@ -42,8 +40,6 @@ template <> struct FieldConst<1> {  // r
                                       2021213742u, 1718526831u, 2584207151u, 235567041u};
   static constexpr uint32_t r2[8] = {2921426343u, 465102405u,  3814480355u, 1409170097u,
                                      1404797061u, 2353627965u, 2135835813u, 35049649u};
-  static constexpr uint32_t r3[8] = {3032416320u, 1586813153u, 486258360u,  709401790u,
-                                     2711605229u, 2302461540u, 2144101756u, 217602379u};
 };
 
 template <int PIDX> struct Fp {
@@ -266,19 +262,18 @@ template <int PIDX> struct Fp {
     return mul(a, one_n);
   }
 
-  // Inverse in the Montgomery domain: (aR)^-1 R, 0 for a == 0.  The integer
-  // aR is inverted by division steps (inv30.h), then multiplied by R^3:
-  // (aR)^-1 R^3 R^-1 = a^-1 R.
+  // Inverse in the Montgomery domain, 0 for a == 0: R^2 / (aR) = a^-1 R by
+  // division steps (inv30.h).
   __device__ static Fp inv(const Fp &a) {
     if (a.is_zero()) return zero();
-    Fp p, r, r3;
+    Fp p, r, r2;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
       p.v[i] = C::p[i];
-      r3.v[i] = C::r3[i];
+      r2.v[i] = C::r2[i];
     }
-    i30_inverse<false>(a.v, p.v, C::np, r.v);
-    return mul(r, r3);
+    i30_inverse<false>(a.v, p.v, C::np, r.v, r2.v);
+    return r;
   }
 };
 

@@ -1,16 +1,24 @@
-// Modular inversion by division steps (Bernstein and Yang, "Fast
-// constant-time gcd computation and modular inversion", 2019; the variant
-// that starts at delta = 1/2), for the inversions that close a multiexp and
-// the per-point ones of the table builders.
+// Modular inversion by division steps, for the inversions that close a multiexp
+// and the per-point ones of the table builders.
 //
-// f = p, g = a and the cofactors d, e (d a = f, e a = g mod p) are signed
-// numbers of nine 30-bit limbs.  A batch takes 30 division steps on the low
-// words alone, several at a time where the low bits of g can be cleared
-// together, and collects them in a 2x2 matrix; f, g, d and e then take the
-// matrix once, exactly divided by 2^30 (d, e modulo p).  About 18 batches end
-// with g = 0, f = +-1.  A binary extended Euclid, which this replaced, shifted
-// and added whole numbers bit by bit (the window combination of a one-window
-// table run, an inversion and little else: 167 us, now 33).
+// Bernstein and Yang, "Fast constant-time gcd computation and modular
+// inversion" (2019), define for odd f the step
+//   (delta, f, g) -> (1 - delta, g, (g - f) / 2)                delta > 0, g odd
+//                    (1 + delta, f, (g + (g mod 2) f) / 2)      otherwise
+// and prove that from delta = 1 at most (49 b + 57) / 17 of them bring numbers of
+// b bits to g = 0, f = +-gcd: 741 for b = 256.
+//
+// A batch is 30 steps on the low 30 bits of f and g, which is all that they look
+// at, and its matrix (u v; q r), 2^30 (f', g') = (u f + v g, q f + r g), with
+// |u| + |v| and |q| + |r| at most 2^30.  A row is kept as one 64-bit number
+// u + 2^32 v: doubling, adding and subtracting rows are then single operations,
+// exact as long as the entries fit (they do), and the entries are read off at the
+// end.  f, g and the pair d, e with d a = s f, e a = s g mod p (s: the scale) are
+// nine 30-bit limbs, the top one signed, and take the matrix once a batch; for d and
+// e a multiple m p, |m| <= 2^29, makes the sum divisible by 2^30, so that they grow
+// by at most p / 2: after the 25 batches that can be needed both are within 13.5 p,
+// and only the result is brought to [0, p).  About 18 batches end with g = 0.  The
+// scale makes the caller's factor (Montgomery's) part of the inverse.
 #pragma once
 #include <stdint.h>
 
@@ -33,54 +41,6 @@ __device__ __forceinline__ I30 i30_from(const uint32_t *w) {
   return r;
 }
 
-// p^-1 mod 2^30 from np = -p^-1 mod 2^32
-__device__ __forceinline__ constexpr uint32_t i30_pinv(uint32_t np) { return (0u - np) & 0x3FFFFFFFu; }
-
-// 30 division steps on the low bits of f (odd) and g; eta = -2 delta.  The
-// matrix (u v; q r) satisfies 2^30 (f', g') = (u f + v g, q f + r g) with
-// |u| + |v| <= 2^30, |q| + |r| <= 2^30.
-__device__ __forceinline__ int32_t i30_divsteps(int32_t eta, uint32_t f, uint32_t g, int32_t &u, int32_t &v,
-                                                int32_t &q, int32_t &r) {
-  uint32_t uu = 1, vv = 0, qq = 0, rr = 1;
-  int32_t i = 30;
-  for (;;) {
-    // g even: halve it (a step with delta + 1 each); the sentinel stops at i
-    const int32_t z = __builtin_ctz(g | (0xFFFFFFFFu << i));
-    g >>= z;
-    uu <<= z;
-    vv <<= z;
-    eta -= 2 * z;
-    i -= z;
-    if (i == 0) break;
-    if (eta < 0) {  // delta > 0 and g odd: (f, g) <- (g, -f)
-      eta = -eta;
-      uint32_t t = f;
-      f = g;
-      g = 0u - t;
-      t = uu;
-      uu = qq;
-      qq = 0u - t;
-      t = vv;
-      vv = rr;
-      rr = 0u - t;
-    }
-    // the next (eta + 1) / 2 steps cannot swap: add the multiple w f of f
-    // that clears that many low bits of g (at most 6: 1/f = f (2 - f f) mod 64)
-    int32_t lim = (eta + 1) >> 1;
-    if (lim > i) lim = i;
-    if (lim > 6) lim = 6;
-    const uint32_t w = (f * g * (f * f - 2u)) & ((1u << lim) - 1u);
-    g += f * w;
-    qq += uu * w;
-    rr += vv * w;
-  }
-  u = (int32_t)uu;
-  v = (int32_t)vv;
-  q = (int32_t)qq;
-  r = (int32_t)rr;
-  return eta;
-}
-
 // the compiler knows the masked limbs to be nonnegative and would form their
 // signed products from unsigned ones and corrections
 #ifdef __HIP__
@@ -97,87 +57,119 @@ static inline int32_t i30_signed(int32_t x) { return x; }
 template <bool UNIFORM> static inline uint32_t i30_low(int32_t x) { return (uint32_t)x; }
 #endif
 
-// words of a^-1 mod p for 0 < a < 2^256 coprime to p (p odd, below 2^255);
-// pw: words of p, np = -p^-1 mod 2^32.  UNIFORM: every active lane has the same
-// a, so the division steps run on the scalar unit.
+struct I30Row {
+  int32_t x, y;  // x + 2^32 y
+};
+__device__ __forceinline__ I30Row i30_row(uint64_t r) {
+  const uint32_t lo = (uint32_t)r;
+  return {(int32_t)lo, (int32_t)((uint32_t)(r >> 32) + (lo >> 31))};
+}
+
+// 30 division steps; the rows of their matrix in top and bottom.  On the scalar unit a
+// step is five instructions, nine more where g is odd and up to five for a turn.
+// Unrolled, as one wave waits for them: a table run of 64 G1 points, an inversion and
+// little else, 177 us, 179 with five steps to a trip, 186 with one.
+__device__ __forceinline__ void i30_steps(int32_t &delta, uint32_t f, uint32_t g, I30Row &top, I30Row &bottom) {
+  uint64_t a = 1, b = 1ull << 32;
+#pragma unroll
+  for (int k = 0; k < 30; k++) {
+    if (g & 1) {
+      if (delta > 0) {  // a quarter turn: the sum below is then g - f, beside f = g
+        const uint32_t h = f;
+        const uint64_t c = a;
+        f = g;
+        g = 0 - h;
+        a = b;
+        b = 0 - c;
+        delta = -delta;
+      }
+      g += f;
+      b += a;
+    }
+    g >>= 1;
+    a += a;
+    delta++;
+  }
+  top = i30_row(a);
+  bottom = i30_row(b);
+}
+
+// (x X + y Y + m P) / 2^30, an exact division
+__device__ __forceinline__ I30 i30_combine(const I30Row &r, const I30 &X, const I30 &Y, int32_t m, const I30 &P) {
+  I30 o;
+  int64_t c = 0;
+#pragma unroll
+  for (int i = 0; i < 9; i++) {
+    c += (int64_t)r.x * X.l[i];
+    c += (int64_t)r.y * Y.l[i];
+    c += (int64_t)m * P.l[i];
+    if (i > 0) o.l[i - 1] = i30_signed((int32_t)c & 0x3FFFFFFF);
+    c >>= 30;
+  }
+  o.l[8] = (int32_t)c;
+  return o;
+}
+
+// the m of -2^29 .. 2^29 - 1 for which x X + y Y + m p is divisible by 2^30;
+// np = -1/p mod 2^32
+__device__ __forceinline__ int32_t i30_multiple(const I30Row &r, const I30 &X, const I30 &Y, uint32_t np) {
+  const uint32_t t = (uint32_t)r.x * (uint32_t)X.l[0] + (uint32_t)r.y * (uint32_t)Y.l[0];
+  return (int32_t)(t * np << 2) >> 2;
+}
+
+// words of scale / a mod p (scale below p, 1 if null) for 0 < a < 2^256 coprime to
+// p (p odd, below 2^255); pw: words of p, np = -1/p mod 2^32.  UNIFORM: every
+// active lane has the same a, so the division steps run on the scalar unit.
 template <bool UNIFORM>
-__device__ __forceinline__ void i30_inverse(const uint32_t *a, const uint32_t *pw, uint32_t np, uint32_t *out) {
-  constexpr int32_t M30 = 0x3FFFFFFF;
-  const uint32_t pinv = i30_pinv(np);
-  const I30 p = i30_from(pw);
+__device__ __forceinline__ void i30_inverse(const uint32_t *a, const uint32_t *pw, uint32_t np, uint32_t *out,
+                                            const uint32_t *scale = nullptr) {
+  const I30 p = i30_from(pw), zero = {};
   I30 f = p, g = i30_from(a), d = {}, e = {};
   e.l[0] = 1;
-  int32_t eta = -1;  // delta = 1/2
-  for (;;) {
-    int32_t u, v, q, r;
-    eta = i30_divsteps(eta, i30_low<UNIFORM>(f.l[0]), i30_low<UNIFORM>(g.l[0]), u, v, q, r);
-    // d, e in (-2p, p) stay there: a negative one counts as itself plus p, and
-    // the multiple of p that makes the sum divisible by 2^30 is taken in (-2^30, 0]
-    const int32_t sd = d.l[8] >> 31, se = e.l[8] >> 31;
-    int32_t md = (u & sd) + (v & se), me = (q & sd) + (r & se);
-    int64_t cd = (int64_t)u * d.l[0] + (int64_t)v * e.l[0], ce = (int64_t)q * d.l[0] + (int64_t)r * e.l[0];
-    md -= (int32_t)((pinv * (uint32_t)cd + (uint32_t)md) & (uint32_t)M30);
-    me -= (int32_t)((pinv * (uint32_t)ce + (uint32_t)me) & (uint32_t)M30);
-    cd += (int64_t)p.l[0] * md;
-    ce += (int64_t)p.l[0] * me;
-    int64_t cf = (int64_t)u * f.l[0] + (int64_t)v * g.l[0], cg = (int64_t)q * f.l[0] + (int64_t)r * g.l[0];
-    cd >>= 30;
-    ce >>= 30;
-    cf >>= 30;
-    cg >>= 30;
-    int32_t nz = 0;
+  if (scale) e = i30_from(scale);
+  int32_t delta = 1, left;
+  do {
+    I30Row t, b;
+    i30_steps(delta, i30_low<UNIFORM>(f.l[0]), i30_low<UNIFORM>(g.l[0]), t, b);
+    const I30 f1 = i30_combine(t, f, g, 0, zero), d1 = i30_combine(t, d, e, i30_multiple(t, d, e, np), p);
+    g = i30_combine(b, f, g, 0, zero);
+    e = i30_combine(b, d, e, i30_multiple(b, d, e, np), p);
+    f = f1;
+    d = d1;
+    left = 0;
 #pragma unroll
-    for (int i = 1; i < 9; i++) {
-      const int32_t di = d.l[i], ei = e.l[i], fi = f.l[i], gi = g.l[i];
-      cd += (int64_t)u * di + (int64_t)v * ei + (int64_t)p.l[i] * md;
-      ce += (int64_t)q * di + (int64_t)r * ei + (int64_t)p.l[i] * me;
-      cf += (int64_t)u * fi + (int64_t)v * gi;
-      cg += (int64_t)q * fi + (int64_t)r * gi;
-      d.l[i - 1] = i30_signed((int32_t)cd & M30);
-      e.l[i - 1] = i30_signed((int32_t)ce & M30);
-      f.l[i - 1] = i30_signed((int32_t)cf & M30);
-      g.l[i - 1] = i30_signed((int32_t)cg & M30);
-      nz |= g.l[i - 1];
-      cd >>= 30;
-      ce >>= 30;
-      cf >>= 30;
-      cg >>= 30;
-    }
-    d.l[8] = (int32_t)cd;
-    e.l[8] = (int32_t)ce;
-    f.l[8] = (int32_t)cf;
-    g.l[8] = (int32_t)cg;
-    nz |= g.l[8];
-    if (i30_low<UNIFORM>(nz) == 0) break;
-  }
-  // f = +-1 and d a = f: the inverse is f d in (-2p, 2p), brought to [0, p)
-  const int32_t sf = f.l[8] >> 31;
-#pragma unroll
-  for (int i = 0; i < 9; i++) d.l[i] = (d.l[i] ^ sf) - sf;
+    for (int i = 0; i < 9; i++) left |= g.l[i];
+  } while (i30_low<UNIFORM>(left) != 0);
+  // f = +-1: the result is f d, within 13.5 p; as a number of [0, 28 p) it loses 14 p,
+  // 7 p, 4 p, 2 p and p where it is at least that
+  const int32_t sign = f.l[8] < 0 ? -1 : 1;
+  int32_t k = 14;
 #pragma unroll 1
-  for (int k = 0; k < 5; k++) {  // + p twice, into (0, 4p); - p while it is at least p
-    const int32_t keep = k < 2 ? 0 : -1, sg = k < 2 ? 0 : -1;
-    int32_t x[9], c = 0;
+  for (int pass = 0; pass < 6; pass++) {
+    I30 x;
+    int64_t c = 0;
 #pragma unroll
     for (int i = 0; i < 9; i++) {
-      const int32_t t = d.l[i] + ((p.l[i] ^ sg) - sg) + c;
-      x[i] = i < 8 ? (t & M30) : t;
-      c = t >> 30;
+      c += pass == 0 ? (int64_t)sign * d.l[i] : (int64_t)d.l[i];
+      c += (int64_t)k * p.l[i];
+      x.l[i] = i < 8 ? (int32_t)c & 0x3FFFFFFF : (int32_t)c;
+      c >>= 30;
     }
-    const bool lt = (x[8] & keep) < 0;
+    const bool take = pass == 0 || x.l[8] >= 0;
 #pragma unroll
-    for (int i = 0; i < 9; i++) d.l[i] = lt ? d.l[i] : x[i];
+    for (int i = 0; i < 9; i++) d.l[i] = take ? x.l[i] : d.l[i];
+    k = pass == 0 ? -14 : pass == 1 ? -7 : pass == 2 ? -4 : k / 2;
   }
 #pragma unroll
-  for (int k = 0; k < 8; k++) {  // 30-bit limbs -> words
+  for (int k2 = 0; k2 < 8; k2++) {  // 30-bit limbs -> words
     uint32_t x = 0;
 #pragma unroll
     for (int i = 0; i < 9; i++) {
-      const int lo = 30 * i - 32 * k;
+      const int lo = 30 * i - 32 * k2;
       if (lo >= 32 || lo + 30 <= 0) continue;
       x |= lo >= 0 ? ((uint32_t)d.l[i] << lo) : ((uint32_t)d.l[i] >> -lo);
     }
-    out[k] = x;
+    out[k2] = x;
   }
 }
 

@@ -48,10 +48,7 @@ __constant__ uint32_t kRowD[6][16] = {
     {1424090310u, 1244383009u, 1551524116u, 1548966950u, 1463451310u, 1552975748u, 1183108232u, 1335459334u,
      31714062u}};
 
-// 2^783 mod q (2^261 cubed: from the inverse of a 2^261-form number to the
-// 2^261 form of the inverse) and 2^256 mod q (to the 2^256 form)
-__constant__ uint32_t kRowR3[16] = {237179570u, 381705378u, 197673865u, 484389131u, 296595421u,
-                                    53368462u,  493544588u, 282381599u, 2540242u};
+// 2^256 mod q (to the 2^256 form)
 __constant__ uint32_t kRowFrom[16] = {93261213u,  451550318u, 297979764u, 299258347u, 342016167u,
                                       297253948u, 482187706u, 406012155u, 920183u};
 
@@ -183,14 +180,22 @@ __device__ __forceinline__ uint32_t row_scatter(const Fq29 &a) {
 }
 // canonical words of each row's element (below 2q)
 __device__ __forceinline__ void row_words(uint32_t x, uint32_t (&w)[8]) { pack29(canon29(row_gather(x)), w); }
+// words of 2^522 mod q: over a 2^261-form number, the 2^261 form of its inverse
+struct Row522 {
+  static constexpr uint32_t v[8] = {1704700944u, 3785531508u, 1409679450u, 1670927750u,
+                                    759047730u,  4283745664u, 887776678u,  705799820u};
+};
 // the inverse of an element every row holds (2^261 form, below 2q, not 0)
-__device__ __forceinline__ uint32_t row_inverse(const RowK &k, uint32_t x) {
-  uint32_t w[8], p[8], o[8];
+__device__ __forceinline__ uint32_t row_inverse(uint32_t x) {
+  uint32_t w[8], p[8], s[8], o[8];
   row_words(x, w);
 #pragma unroll
-  for (int i = 0; i < 8; i++) p[i] = FieldConst<0>::p[i];
-  i30_inverse<true>(w, p, FieldConst<0>::np, o);
-  return row_mul(k, row_scatter(unpack29(o)), kRowR3[threadIdx.x & 15]);
+  for (int i = 0; i < 8; i++) {
+    p[i] = FieldConst<0>::p[i];
+    s[i] = Row522::v[i];
+  }
+  i30_inverse<true>(w, p, FieldConst<0>::np, o, s);
+  return row_scatter(unpack29(o));
 }
 
 // rows 0, 2 hold one value and rows 1, 3 another: both in every row

@@ -147,3 +147,17 @@ def test_table_windows_sorted_together(tmp_path):
         assert not joint(1 << 20, c)
     for c in (10, 13, 16, 17):
         assert joint(1 << 20, c)
+
+
+@pytest.mark.parametrize("p", [Q, R])
+def test_inverse_with_a_scale(tmp_path, p):
+    L = compiled(tmp_path, "inv30.h", "void inv(const uint32_t *a, const uint32_t *p, uint32_t np, uint32_t *o, "
+                                      "const uint32_t *s) { csk::i30_inverse<false>(a, p, np, o, s); }")
+    rng = random.Random(8)
+    np_ = -pow(p, -1, 1 << 32) % (1 << 32)
+    xs = [1, 2, p - 1, p - 2, (p + 1) // 2, p + 1, 2**256 - 1, 2**255, 3 << 200] + [rng.randrange(1, p) for _ in range(3000)]
+    for i, x in enumerate(xs):
+        s = (0, 1, p - 1, 1 << 253)[i % 8] if i % 8 < 4 else rng.randrange(p)
+        o = W8()
+        L.inv(words(x), words(p), np_, o, words(s))
+        assert value(o) == s * pow(x, -1, p) % p, (hex(x), hex(s))
