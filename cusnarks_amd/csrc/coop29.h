@@ -141,8 +141,6 @@ template <> struct Coop29<Fq2> {
   static constexpr int kRows = 16;
   static constexpr int kForm = E_NSLOT > D2_OZZZ1 + 1 ? E_NSLOT : D2_OZZZ1 + 1;
   static constexpr int kSlots = kForm + 6;
-  static constexpr int kDbl = sizeof(kG2Dbl) / sizeof(C29Op), kAdd1 = sizeof(kG2Add1) / sizeof(C29Op),
-                       kAdd2 = sizeof(kG2Add2) / sizeof(C29Op);
 
   // One row's operation of a round, as word offsets of its lane: fetched once
   // for the rounds of the doubling, which run back to back.

@@ -73,43 +73,6 @@ template <class F> __device__ __forceinline__ XYZZ<F> xyzz_madd_inl(const XYZZ<F
 }
 
 
-
-// a + b (add-2008-s); xyzz_add_inl is the always-inlined body
-template <class F> __device__ __forceinline__ XYZZ<F> xyzz_add_inl(const XYZZ<F> &a, const XYZZ<F> &b) {
-  if (a.is_inf()) return b;
-  if (b.is_inf()) return a;
-  F U1 = F::mul(a.X, b.ZZ);
-  F U2 = F::mul(b.X, a.ZZ);
-  F S1 = F::mul(a.Y, b.ZZZ);
-  F S2 = F::mul(b.Y, a.ZZZ);
-  F P = F::sub(U2, U1);
-  F R = F::sub(S2, S1);
-  if (P.is_zero()) {
-    if (R.is_zero()) return xyzz_dbl(a);
-    return XYZZ<F>::inf();
-  }
-  F PP = F::sqr(P);
-  F PPP = F::mul(P, PP);
-  F Qv = F::mul(U1, PP);
-  F X3 = F::sub(F::sub(F::sqr(R), PPP), F::dbl(Qv));
-  F Y3 = F::sub(F::mul(R, F::sub(Qv, X3)), F::mul(S1, PPP));
-  return {X3, Y3, F::mul(F::mul(a.ZZ, b.ZZ), PP), F::mul(F::mul(a.ZZZ, b.ZZZ), PPP)};
-}
-
-
-// k*p for a small non-negative k (bucket-segment offsets), left to right
-template <class F> __device__ __forceinline__ XYZZ<F> xyzz_mul_small_inl(const XYZZ<F> &p, uint32_t k) {
-  XYZZ<F> acc = XYZZ<F>::inf();
-  if (k == 0 || p.is_inf()) return acc;
-  int top = 31 - __builtin_clz(k);
-  acc = p;
-  for (int b = top - 1; b >= 0; b--) {
-    acc = xyzz_dbl(acc);
-    if ((k >> b) & 1u) acc = xyzz_add(acc, p);
-  }
-  return acc;
-}
-
 // canonical affine; infinity -> (0, 1) as the reference encodes it
 // (ec_jac2aff_h, cusnarks src/cuda/ec.cpp:963-1012)
 template <class F> __device__ __forceinline__ Affine<F> xyzz_to_affine_inl(const XYZZ<F> &p) {
@@ -126,8 +89,6 @@ template <class F> __device__ __forceinline__ Affine<F> xyzz_to_affine_inl(const
 template <class F> __device__ __noinline__ XYZZ<F> xyzz_dbl_affine_call(const Affine<F> &p) { return xyzz_dbl_affine_inl(p); }
 template <class F> __device__ __noinline__ XYZZ<F> xyzz_dbl_call(const XYZZ<F> &p) { return xyzz_dbl_inl(p); }
 template <class F> __device__ __noinline__ XYZZ<F> xyzz_madd_call(const XYZZ<F> &a, const Affine<F> &q) { return xyzz_madd_inl(a, q); }
-template <class F> __device__ __noinline__ XYZZ<F> xyzz_add_call(const XYZZ<F> &a, const XYZZ<F> &b) { return xyzz_add_inl(a, b); }
-template <class F> __device__ __noinline__ XYZZ<F> xyzz_mul_small_call(const XYZZ<F> &p, uint32_t k) { return xyzz_mul_small_inl(p, k); }
 template <class F> __device__ __noinline__ Affine<F> xyzz_to_affine_call(const XYZZ<F> &p) { return xyzz_to_affine_inl(p); }
 
 #define CSK_DISPATCH(F, name, ...) \
@@ -137,8 +98,6 @@ template <class F> __device__ __noinline__ Affine<F> xyzz_to_affine_call(const X
 template <class F> __device__ __forceinline__ XYZZ<F> xyzz_dbl_affine(const Affine<F> &p) { CSK_DISPATCH(F, xyzz_dbl_affine, p); }
 template <class F> __device__ __forceinline__ XYZZ<F> xyzz_dbl(const XYZZ<F> &p) { CSK_DISPATCH(F, xyzz_dbl, p); }
 template <class F> __device__ __forceinline__ XYZZ<F> xyzz_madd(const XYZZ<F> &a, const Affine<F> &q) { CSK_DISPATCH(F, xyzz_madd, a, q); }
-template <class F> __device__ __forceinline__ XYZZ<F> xyzz_add(const XYZZ<F> &a, const XYZZ<F> &b) { CSK_DISPATCH(F, xyzz_add, a, b); }
-template <class F> __device__ __forceinline__ XYZZ<F> xyzz_mul_small(const XYZZ<F> &p, uint32_t k) { CSK_DISPATCH(F, xyzz_mul_small, p, k); }
 template <class F> __device__ __forceinline__ Affine<F> xyzz_to_affine(const XYZZ<F> &p) { CSK_DISPATCH(F, xyzz_to_affine, p); }
 
 // ------------------------------------------------------------------ memory I/O

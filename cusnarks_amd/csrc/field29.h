@@ -18,7 +18,7 @@
 // Conversion.  Points enter as the library's 8 x u32 words in Montgomery
 // form for R = 2^256; a product by 2^266 mod q (x 2^256 x 2^266 /
 // 2^261 = x 2^261), stored packed back into 8 words (values are < q).
-// from29 multiplies by 2^256 mod q, which returns to R = 2^256 form.
+// A product by 2^256 mod q returns to the R = 2^256 form (row29.h).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -38,8 +38,6 @@ struct Q29 {
                                       490881230u, 299191303u, 86689704u,  903222u};  // 2^261 mod q
   static constexpr uint32_t to[9] = {322215073u, 442336424u, 171859116u, 268585440u, 314135016u,
                                      244503300u, 348886451u, 68918589u,  360451u};  // 2^266 mod q
-  static constexpr uint32_t from[9] = {93261213u,  451550318u, 297979764u, 299258347u, 342016167u,
-                                       297253948u, 482187706u, 406012155u, 920183u};  // 2^256 mod q
   static constexpr uint32_t p4[9] = {32765212u,  68256475u, 298487100u, 190090051u, 370632160u,
                                      191693570u, 43746564u, 426809552u, 12685625u};  // 4q
 };
@@ -485,11 +483,6 @@ __device__ __forceinline__ void pack29(const Fq29 &a, uint32_t (&w)[8]) {
   }
 }
 
-// 2^261 form (value below 8q) -> canonical R = 2^256 words
-__device__ __forceinline__ void from29_words(const Fq29 &a, uint32_t (&out)[8]) {
-  pack29(canon29(mul29(a, f29_const(Q29::from))), out);
-}
-
 struct XYZZ29 {
   Fq29 X, Y, ZZ, ZZZ;
 };
@@ -869,19 +862,6 @@ __device__ __forceinline__ void xadd29(XYZZ2_29 &a, const XYZZ2_29 &b) {
   a.Y = Y3;
   a.ZZ = ZZ3;
   a.ZZZ = ZZZ3;
-}
-
-// k a for a small k (bucket-segment offsets), left to right
-template <class A> __device__ __forceinline__ A xmul_small29(const A &p, uint32_t k, const A &inf) {
-  if (k == 0) return inf;
-  A acc = p;
-  const int top = 31 - __builtin_clz(k);
-#pragma unroll 1
-  for (int b = top - 1; b >= 0; b--) {
-    xdbl29(acc);
-    if ((k >> b) & 1u) xadd29(acc, p);
-  }
-  return acc;
 }
 
 }  // namespace csk

@@ -42,18 +42,6 @@ __device__ __forceinline__ void reduce_mod_r(uint32_t *k) {
 }
 
 // ------------------------------------------------------------------ members
-// largest j < J with segs[j].pbase <= g (the member holding concatenated point
-// g; empty members share their pbase with the next one and are skipped)
-__device__ __forceinline__ uint32_t member_of_point(const MsmSeg *segs, uint32_t J, uint64_t g) {
-  uint32_t lo = 0, hi = J;
-  while (hi - lo > 1) {
-    uint32_t mid = (lo + hi) >> 1;
-    if (segs[mid].pbase <= g) lo = mid;
-    else hi = mid;
-  }
-  return lo;
-}
-
 // largest j < J with segs[j].tbase <= b (the member of pass-1 workgroup b)
 __device__ __forceinline__ uint32_t member_of_tile(const MsmSeg *segs, uint32_t J, uint32_t b) {
   uint32_t lo = 0, hi = J;
@@ -786,11 +774,11 @@ __device__ __forceinline__ void store29(uint32_t *d, const XYZZ2_29 &a) {
 
 __device__ __forceinline__ XYZZ29 inf29() { return {Fq29{}, f29_const(Q29::one), Fq29{}, Fq29{}}; }
 
-// It is bound by power: 98% of the issue slots hold a vector instruction, and
-// the clock falls to 1.85 GHz under the 1485 multiply-adds per entry of its
-// 2150 instructions (1.92 GHz with 2364; 2^24 points, 2.35 * 10^8 entries: 16.5
-// ms, 1.42 * 10^10 entries/s).  A 9% shorter loop gained 1.5%; only fewer
-// multiply-adds per entry would gain more.
+// It is bound by power: 94% of the cycles issue a vector instruction, and the
+// clock falls to 1.95 GHz (2.25 in a loop of multiply-adds alone) under the 1485
+// multiply-adds per entry of its 2160 instructions (2^24 points, 2.35 * 10^8
+// entries: 16.2 ms, 1.45 * 10^10 entries/s).  A 9% shorter loop gained 1.5%; only
+// fewer multiply-adds per entry would gain more.
 template <class F>
 __global__ void __launch_bounds__(256) k_accumulate29(const MsmSeg *__restrict__ segs, uint32_t Kj,
                                                       const uint32_t *__restrict__ sorted,
