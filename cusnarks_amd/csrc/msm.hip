@@ -119,15 +119,17 @@ MsmPlan msm_group_plan(uint32_t c, uint32_t E, const uint64_t *n, uint32_t J, bo
   return pl;
 }
 
-// At widths where the halves have an entry more per point, whole scalars are the
-// fewer additions of a large multiexp: 2^24 G1 points, c = 17, 16 entries a point 23.6
-// ms, whole 15 and 21.9; c = 15 26.7 and 24.5.  The halves' fewer buckets, and half the
-// doublings, then count 10 entries each and 3 million: with 2^22 points they still win
-// or tie (c = 17 6.54 and 6.40 ms, wire values 3.75 and 3.92).  A whole scalar's narrow
-// top window (c = 14: 254 is 18 * 14 + 2) takes the gain back: 27.1 and 27.8 ms.
+// At widths where the parts have an entry more per point, whole scalars are the
+// fewer additions of a large multiexp: 2^24 G1 points, c = 17, 16 entries a point 22.6
+// ms, whole 15 and 21.2; c = 15 26.0 and 23.9; G2 c = 17 65.2 and 55.3.  The parts' fewer
+// buckets, and half the doublings, then count 4 entries each and 3.7 million, which is
+// where wire values, half of whose digits are 0, tie too: G1 c = 15 at 4.2 million
+// points (uniform ones at 1), c = 17 at 6 (3), c = 20 at 17 (12); G2 c = 17 at 4.3 (2.7).
+// A whole scalar's narrow top window (c = 14: 254 is 18 * 14 + 2) takes the gain back:
+// 27.1 and 27.8 ms.
 static bool split_pays(const MsmPlan &split, const MsmPlan &whole) {
   if (split.max_entries <= whole.max_entries || whole.bits % whole.c <= whole.c / 2) return true;
-  return split.max_entries - whole.max_entries <= whole.J * (10ull * (whole.K - split.K) + 3000000);
+  return split.max_entries - whole.max_entries <= whole.J * (4ull * (whole.K - split.K) + 3700000);
 }
 
 // G2 scalars are taken in quarters where these have no more entries at the width
