@@ -2,14 +2,19 @@
 
 For each size class lg (sizes with floor(log2 n) == lg) it times the Pippenger
 pipeline at n = 2^(lg + 1/2) over a sweep of window widths c, then of the
-accumulation chunk length, and keeps the fastest.  The table is persisted as
+accumulation chunk length, and takes the fastest; the width that the installed
+table has stays unless another is 2% faster, the library's own chunk rule
+(csrc/chunk.h, from the digits that are not zero, where a fixed length fits one kind
+of scalars) unless one is 10% faster.  With --change only the named classes may
+change: the others are timed and keep their widths, which neighbouring classes share
+so that a proof's multiexps run as one group.  The table is persisted as
 JSON under cusnarks_amd/tuning/ and installed into a context with
 csk_msm_set_tuning; single calls and batch plans then use it whenever the
 caller gives no explicit setting.  The reference fixes its launch geometry per
 multiexp batch instead (get_shfl_blockD, cusnarks
 src/python/cuda_wrapper.py:1570-1587).
 
-    python -m cusnarks_amd.tune --curve g1 --lg 10:25 --out cusnarks_amd/tuning/msm_g1.json
+    python -m cusnarks_amd.tune --curve g1 --lg 10:27 --out cusnarks_amd/tuning/msm_g1.json
 """
 from __future__ import annotations
 
@@ -60,7 +65,8 @@ def apply(ctx) -> list[str]:
 
 
 def default_chunk(n: int, c: int) -> int:
-    """The chunk length the sweep starts from, for one multiexp of n points."""
+    """A length for the chunk sweep to start from: entries of whole scalars over
+    2^18 threads, 8 to 256 (not the library's rule, which chunk 0 asks for)."""
     return max(8, min(256, (n * (254 // c + 1)) >> 18))
 
 
@@ -77,7 +83,13 @@ def _measure(ctx, g2, ds, dp, n, out, cfg, reps) -> float:
     return statistics.median(_time_once(ctx, g2, ds, dp, n, out, cfg) for _ in range(reps))
 
 
-def autotune(g2: bool, lgs, ctx=None, reps: int = 3, log=print) -> dict:
+def _pick(times: dict, present: int, keep: float) -> int:
+    """The fastest, or the present choice while that takes at most `keep` times as long."""
+    best = min(times, key=times.get)
+    return present if present in times and times[present] <= keep * times[best] else best
+
+
+def autotune(g2: bool, lgs, ctx=None, reps: int = 3, log=print, change=None) -> dict:
     """Sweep c, then the chunk length, for every class in lgs; returns the tuning document."""
     from .msm import fixed_base
     ctx = ctx or _capi.Context(0)
@@ -94,18 +106,23 @@ def autotune(g2: bool, lgs, ctx=None, reps: int = 3, log=print) -> dict:
     out = DeviceBuffer(ctx, 4 * (G2W if g2 else G1W))
     log("tune %s: %d points ready in %.1f s" % ("g2" if g2 else "g1", nmax, time.time() - t0))
     cmax = 18 if g2 else 20
+    present = {}
+    if os.path.exists(tuning_path(g2)):
+        with open(tuning_path(g2)) as fh:
+            present = json.load(fh)["classes"]
     classes = {}
     for lg in lgs:
         n = int(round(2 ** (lg + 0.5)))
         sweep = {}
         for c in range(max(4, lg - 10), min(lg + 1, cmax) + 1):
             sweep[c] = _measure(ctx, g2, sc, pts, n, out, MsmCfg(c, 0, 0, 0), reps)
-        c = min(sweep, key=sweep.get)
+        fixed = change is not None and lg not in change
+        c = _pick(sweep, int(present.get(str(lg), {}).get("window_bits", 0)), float("inf") if fixed else 1.02)
         l0 = default_chunk(n, c)
         chunks = {}  # 0: the library's own rule
         for L in sorted({0, max(4, l0 // 2), l0, min(1024, 2 * l0)}):
             chunks[L] = _measure(ctx, g2, sc, pts, n, out, MsmCfg(c, L, 0, 0), reps)
-        L = min(chunks, key=chunks.get)
+        L = _pick(chunks, 0, float("inf") if fixed else 1.1)
         classes[str(lg)] = {"window_bits": c, "chunk": L, "reduce_seg": 0,
                             "n": n, "ms": round(chunks[L], 4),
                             "sweep_c_ms": {str(a): round(b, 4) for a, b in sweep.items()},
@@ -116,7 +133,8 @@ def autotune(g2: bool, lgs, ctx=None, reps: int = 3, log=print) -> dict:
         b.close()
     check(lib().csk_ctx_set_timing(ctx.ptr, 0), "csk_ctx_set_timing")
     return {"curve": "g2" if g2 else "g1", "device": "gfx950", "reps": reps,
-            "method": "median device time of the full pipeline (HIP events); c swept, then chunk",
+            "method": "median device time of the full pipeline (HIP events), uniform scalars; c swept, then "
+                      "chunk (0: the library's rule)",
             "classes": classes}
 
 
@@ -125,11 +143,13 @@ def main(argv=None) -> int:
     ap.add_argument("--curve", choices=("g1", "g2"), default="g1")
     ap.add_argument("--lg", default="10:25", help="classes lo:hi (hi exclusive)")
     ap.add_argument("--reps", type=int, default=3)
+    ap.add_argument("--change", default=None, help="classes that may change, e.g. 21,25 (default: all)")
     ap.add_argument("--out", default=None)
     a = ap.parse_args(argv)
     lo, hi = (int(x) for x in a.lg.split(":"))
     g2 = a.curve == "g2"
-    doc = autotune(g2, range(lo, hi), reps=a.reps, log=lambda s: print(s, flush=True))
+    change = None if a.change is None else {int(x) for x in a.change.split(",") if x}
+    doc = autotune(g2, range(lo, hi), reps=a.reps, log=lambda s: print(s, flush=True), change=change)
     path = a.out or tuning_path(g2)
     os.makedirs(os.path.dirname(os.path.abspath(path)), exist_ok=True)
     with open(path, "w") as fh:

@@ -210,3 +210,17 @@ def test_null_arguments_are_errors_not_crashes():
     assert L.csk_msm_set_tuning(None, 0, None, 0) == _capi.CSK_ERR_ARG
     assert L.csk_ctx_create(0, None) == _capi.CSK_ERR_ARG
     assert L.csk_event_query(None, None) == _capi.CSK_ERR_ARG
+
+
+def test_tuning_tables_agree_with_their_sweeps():
+    import json
+    from cusnarks_amd import tune
+    # every class was timed by one build: its time is its width's, and no width of
+    # the sweep is much faster
+    for g2 in (False, True):
+        with open(tune.tuning_path(g2)) as fh:
+            classes = json.load(fh)["classes"]
+        for lg, e in classes.items():
+            sweep = {int(c): ms for c, ms in e["sweep_c_ms"].items()}
+            own = sweep[e["window_bits"]]
+            assert abs(e["ms"] / own - 1) < 0.1 and own < 1.1 * min(sweep.values()), (g2, lg)
