@@ -775,9 +775,9 @@ __device__ __forceinline__ void store29(uint32_t *d, const XYZZ2_29 &a) {
 __device__ __forceinline__ XYZZ29 inf29() { return {Fq29{}, f29_const(Q29::one), Fq29{}, Fq29{}}; }
 
 // It is bound by power: 94% of the cycles issue a vector instruction, and the
-// clock falls to 1.95 GHz (2.25 in a loop of multiply-adds alone) under the 1485
+// clock falls to 1.97 GHz (2.29 in a loop of multiply-adds alone) under the 1485
 // multiply-adds per entry of its 2160 instructions (2^24 points, 2.35 * 10^8
-// entries: 16.2 ms, 1.45 * 10^10 entries/s).  A 9% shorter loop gained 1.5%; only
+// entries: 16.1 ms, 1.46 * 10^10 entries/s).  A 9% shorter loop gained 1.5%; only
 // fewer multiply-adds per entry would gain more.
 template <class F>
 __global__ void __launch_bounds__(256) k_accumulate29(const MsmSeg *__restrict__ segs, uint32_t Kj,
@@ -1347,7 +1347,7 @@ void window_sums(const uint32_t *off, uint32_t *buckets, uint32_t nwin, uint32_t
 // waves that hold every value in LDS (coop29.h).  Infinity is tracked in a flag every lane holds.
 // Measured: 120 doublings 174 us on G1, 273 on G2 (whole scalars' 248 doublings
 // with one lane per product: 855 and 1997 us).  One window (table runs: the
-// inversion and the conversions): 33 us, 167 with a binary Euclid on one lane.
+// inversion and the conversions): 33 us, 167 with a bit-by-bit Euclid on one lane.
 template <class F>
 __global__ void __launch_bounds__(kChainThreads) k_final(const MsmSeg *__restrict__ segs,
                                                          const uint32_t *__restrict__ wsum, uint32_t W, uint32_t c) {
