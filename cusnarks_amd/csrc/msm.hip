@@ -420,7 +420,8 @@ int msm_noalloc_setup(int device) {
 // that runs needs no more, so a width is accepted or refused by n and cfg alone.
 static size_t noalloc_bytes(const MsmPlan &pl, uint32_t rseg) {
   const uint32_t seg = rseg && rseg < pl.Lr ? rseg : pl.Lr;
-  return msm_workspace_bytes(pl, false) + Carver::round(pl.max_entries * 4) + Carver::round((uint64_t)pl.J * pl.W * (pl.B / seg) * 144);
+  return msm_workspace_bytes(pl, false) + Carver::round(pl.max_entries * 4) +
+         Carver::round((uint64_t)pl.J * pl.W * (pl.B / seg) * 144);
 }
 
 }  // namespace csk
