@@ -588,22 +588,27 @@ __global__ void __launch_bounds__(THREADS) k_sort_pass2(const uint32_t *__restri
   if (!LONG && seg == gridDim.x - 1 && threadIdx.x == 0) offsets[Ktot] = end;
   if (!LONG && hi == HB - 1)
     for (uint32_t k = key0 + L2 + threadIdx.x; k < (gw + 1) * B; k += THREADS) offsets[k] = end;
-  if (!LONG && s == 0 && threadIdx.x == 0) offsets[key0] = start;
-  if (!LONG && end - start > split) return;
   if (s == 0) {
-    for (uint32_t e0 = start; e0 < end; e0 += 8 * THREADS) {
+    if (LONG) return;
+    if (threadIdx.x == 0) offsets[key0] = start;
+    // an equal share of the window's entries each: the bins may be most uneven (c = 14:
+    // 126 is 9 * 14, so the top window holds only carries, 2^24 of them in one bin)
+    const uint32_t w0 = goff[cb + w * HB * NT], w1 = goff[cb + (w + 1) * HB * NT], share = (w1 - w0 + HB - 1) / HB;
+    const uint32_t last = min(w1, w0 + (hi + 1) * share);
+    for (uint32_t e0 = w0 + hi * share; e0 < last; e0 += 8 * THREADS) {
       uint32_t v[8];
       for (int k = 0; k < 8; k++) {  // unconditional (clamped) loads, as below
         const uint32_t e = e0 + k * THREADS + threadIdx.x;
-        v[k] = tix[e < end ? e : end - 1];
+        v[k] = tix[e < last ? e : last - 1];
       }
       for (int k = 0; k < 8; k++) {
         const uint32_t e = e0 + k * THREADS + threadIdx.x;
-        if (e < end) sorted[e] = v[k];
+        if (e < last) sorted[e] = v[k];
       }
     }
     return;
   }
+  if (!LONG && end - start > split) return;
   for (uint32_t i = threadIdx.x; i < L2; i += THREADS) cntv[i] = 0;
   __syncthreads();
   // eight unconditional (clamped) loads in flight per thread, then their counts

@@ -104,3 +104,19 @@ def test_batch_takes_the_sizes_of_single_calls():
     tune.install(ctx, False, {"classes": {"27": {"window_bits": 18}}})
     one = MsmBatch.workspace_bytes([1 << 27], ctx=ctx)
     assert MsmBatch.workspace_bytes([1 << 27] * 2, ctx=ctx) == 2 * one
+
+
+@pytest.mark.parametrize("g2,n,c", [(False, 50000, 7), (False, 50000, 9), (False, 70001, 14), (False, 300000, 18),
+                                    (False, 30000, 17), (True, 30000, 8), (True, 30000, 14), (True, 5000, 2)])
+def test_top_windows_whose_bins_are_buckets(g2, n, c):
+    # the parts' bits leave the top window 0 to 7 bits: its entries, half of the
+    # points' carries in one bucket for 0, are ordered by the sort's first pass
+    ctx, nw = _capi.default_context(), 32 if g2 else 16
+    pts, out, want = DeviceBuffer(ctx, n * nw * 4), DeviceBuffer(ctx, nw * 4), DeviceBuffer(ctx, nw * 4)
+    k = inputs.field_elements(924, n)
+    k[: n // 3, 2:] = 0
+    sc = DeviceBuffer.from_array(ctx, k)
+    fixed_base(DeviceBuffer.from_array(ctx, inputs.field_elements(925, n, nonzero=True)), n, pts, g2=g2, ctx=ctx)
+    msm_device(sc, pts, n, want, g2=g2, ctx=ctx)
+    msm_device(sc, pts, n, out, g2=g2, ctx=ctx, window_bits=c)
+    assert np.array_equal(out.download((nw,)), want.download((nw,)))
