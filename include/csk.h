@@ -112,7 +112,7 @@ int csk_msm_g2(csk_ctx *ctx, const uint32_t *d_scalars, const uint32_t *d_points
                uint64_t n, uint32_t *d_out, const csk_msm_cfg *cfg, void *stream);
 /* out[i] = the multiexp of member i (as csk_msm_g1 / csk_msm_g2, settings chosen as
  * there), i < count <= 64, enqueued on stream in the context's workspace.  Small members of
- * one window width run as one pipeline. */
+ * one window width run as one pipeline.  Members are checked before any is enqueued. */
 int csk_msm_multi(csk_ctx *ctx, int ec2, uint32_t count, const uint32_t *const *d_scalars,
                   const uint32_t *const *d_points, const uint64_t *n, uint32_t *const *d_out, void *stream);
 int csk_msm_g1_host(csk_ctx *ctx, const uint32_t *scalars, const uint32_t *points,
